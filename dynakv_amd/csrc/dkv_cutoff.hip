@@ -14,15 +14,18 @@
 // mask: its length is the number of positions m whose prefix sum c_m reaches thr, and
 // out = x on the first len dims (min(len, low_rank)), x * 0 after them.
 //
-// Two kernels on the caller's stream:
-//   cutoff_logits_kernel  16 rows x 64 logits per workgroup (4 waves, 16x16x32 MFMA over D),
-//                         bias added in fp32, rounded to the compute dtype (addmm's output),
-//                         written to the caller's workspace;
-//   cutoff_rows_kernel    one wave per (row, group, K|V): softmax in fp32 of the rounded
-//                         logits (probabilities rounded to the compute dtype, as torch.softmax
-//                         returns them), prefix sums accumulated in fp32 and rounded to the
-//                         compute dtype, the count against the threshold rounded to the
-//                         compute dtype, the masked copy and the int32 length.
+// Kernels, by the shape of the call:
+//   cutoff_small_kernel   D <= 128, a decode step's rows: one launch of 8 waves per 16 rows;
+//   cutoff_fused_kernel   D <= 128, a prompt's rows: one launch, a wave takes 16 rows through
+//                         logits, softmax, count and masked copy with a row in four lanes;
+//   cutoff_logits_ks_kernel (few rows) or cutoff_logits_tile_kernel, then cutoff_rows_kernel
+//                         D >= 256 (the joint head): the logits into the caller's workspace,
+//                         then one wave per (row, group, K|V).
+// Every path rounds as the reference does: bias added in fp32 and the sum rounded to the compute
+// dtype (addmm's output), softmax in fp32 of the rounded logits with the probabilities rounded
+// to the compute dtype (as torch.softmax returns them), prefix sums accumulated in fp32 and
+// rounded to the compute dtype, counted against the threshold rounded to the compute dtype. The
+// rounded logits are left in the caller's workspace.
 // W is taken transposed, Wt[g][n][k] = W_g[k][n] (the input dimension contiguous), so both MFMA
 // operands are 16-byte row loads; the Python layer prepares that copy once per weight.
 #include "dkv_internal.h"
@@ -45,7 +48,9 @@ struct CutoffParams {
   CutoffMat mat[2];
   long long x_ld, out_ld, len_ld;
   int M, G, D, low_rank;
-  float threshold;     // already rounded to the compute dtype
+  float count_min;     // smallest fp32 value whose rounding to the compute dtype is >= the
+                       // threshold (itself rounded to the compute dtype)
+  int vec;             // 16-byte stores of out and logits are aligned
 };
 
 template <int DT>
@@ -74,7 +79,7 @@ __device__ __forceinline__ uint16_t f32_elt(float v) {
     return (uint16_t)dkv_f32_to_f16_bits(v);
 }
 
-// grid: (D / 64, ceil(M / 16), 2 * G); wave w computes logits n0 + 16w .. +16 of 16 rows.
+// One wave: logits n0 .. n0 + 15 of rows row0 .. row0 + 15.
 // MFMA operands: A = x rows (lane: row i = lane % 16, inputs 8*(lane/16) .. +8 of the k-step),
 // B = Wt rows (lane: output n = lane % 16, the same inputs); the result lane holds rows
 // 4*(lane/16) + u of output column lane % 16.
@@ -109,19 +114,11 @@ __device__ __forceinline__ void logits_tile(const CutoffParams& p, int mat, int 
       cm.logits[((long long)m * p.G + g) * D + n0 + i] = f32_elt<DT>(acc[u] + bias);
   }
 }
-template <int DT>
-__global__ __launch_bounds__(256) void cutoff_logits_kernel(CutoffParams p) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  logits_tile<DT>(p, blockIdx.z & 1, blockIdx.z >> 1, blockIdx.y * CT_ROWS,
-                  blockIdx.x * CT_COLS + wave * 16, lane);
-}
-
 // Split-K logits for wide heads (D = 128 * STEPS, the joint 1024-d head: STEPS = 8): grid
 // (D / 16, ceil(M / 16), 2 * G), one workgroup per 16 logits of 16 rows; wave w takes the
 // quarter w of the input dimension, issues every operand load of its STEPS k-steps before the
 // first product, and the four partial sums are added in wave order through LDS (one memory
-// round trip per workgroup instead of one per k-step, four times the workgroups of
-// cutoff_logits_kernel).
+// round trip per workgroup instead of one per k-step).
 template <int DT, int STEPS>
 __global__ __launch_bounds__(256) void cutoff_logits_ks_kernel(CutoffParams p) {
   __shared__ dkv_f32x4 sP[4][64];
@@ -159,6 +156,168 @@ __global__ __launch_bounds__(256) void cutoff_logits_ks_kernel(CutoffParams p) {
   }
 }
 
+// 16 bytes per lane from a buffer resource straight to LDS, lane l's at lds_base + 16 * l.
+__device__ __forceinline__ void ct_lds_load16(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds_base,
+                                              uint32_t byte_off) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+               ::"s"(lds_base), "v"(byte_off), "s"(rsrc)
+               : "memory", "m0");
+}
+__device__ __forceinline__ uint32_t ct_lds_addr(const void* p) {
+  return (uint32_t)(uintptr_t)(__attribute__((address_space(3))) const void*)p;
+}
+
+constexpr int CG_TN = 128;  // logits per tiled workgroup
+constexpr int CG_KS = 64;   // inputs per staged step
+
+// Logits of wide heads for many rows (a prompt), D = 128 * STEPS: workgroup = TM rows x 128
+// logits, four waves of TM/2 x 64, the inputs staged in LDS 64 at a time (three buffers,
+// direct-to-LDS loads, 16-byte chunk c of a row at position c ^ (row % 8)). A = W rows, staged in
+// the order that gives lane (row n, g) the 16 consecutive logits 16g .. of its wave's 64 (LDS row
+// 16 * blk + i is logit 16 * (i / 4) + 4 * blk + i % 4), B = x rows. The products of each quarter
+// of the inputs are summed by themselves and the quarters added in order, as
+// cutoff_logits_ks_kernel adds its waves' partial sums: the same logits bit for bit.
+// Bound: LDS operand reads (32 x 64 products per wave) and the barrier per step. D = 1024, 3001
+// rows: about 20 us for K and V, 0.6 PFLOP/s (110 us in 16 x 16 tiles).
+template <int DT, int STEPS, int TM>
+__global__ __launch_bounds__(256, 2) void cutoff_logits_tile_kernel(CutoffParams p) {
+  constexpr int D = 128 * STEPS, NC = D / CG_TN, NK = D / CG_KS, RB = TM / 32;
+  constexpr int NBUF = TM == 32 ? 4 : 2;       // steps in LDS
+  constexpr int LOADS = CG_TN / 32 + TM / 32;  // loads per wave and step
+  __shared__ __attribute__((aligned(16))) uint8_t sW[NBUF][CG_TN * CG_KS * 2];
+  __shared__ __attribute__((aligned(16))) uint8_t sX[NBUF][TM * CG_KS * 2];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, g = lane >> 4;
+  // ids go to the 8 XCDs round-robin: XCD = (K | V) x (every fourth row tile), a row tile's
+  // column tiles consecutive on it, so an L2 takes in one matrix and a quarter of the rows
+  const int rt_n = (p.M + TM - 1) / TM, nrg = (rt_n + 3) / 4;
+  const int xcd = blockIdx.x & 7, rank = blockIdx.x >> 3;
+  const int mat = xcd & 1;
+  const int ct = rank % NC, rt = rank / NC % nrg * 4 + (xcd >> 1), grp = rank / NC / nrg;
+  if (rt >= rt_n) return;
+  const int col0 = ct * CG_TN, row0 = rt * TM;
+  const CutoffMat& cm = p.mat[mat];
+  const int rows = min(TM, p.M - row0);
+
+  const __amdgpu_buffer_rsrc_t rx =
+      dkv_make_rsrc(cm.x + (long long)row0 * p.x_ld + (long long)grp * D,
+                    (uint32_t)(((long long)(rows - 1) * p.x_ld + D) * 2));
+  const __amdgpu_buffer_rsrc_t rw =
+      dkv_make_rsrc(cm.wt + ((long long)grp * D + col0) * D, (uint32_t)(CG_TN * D * 2));
+  // loads of step k (past the last step: the last one again, into a buffer nobody reads):
+  // instruction c of wave w fills LDS rows 8 * (4c + w) .. + 7, lane l row l / 8's chunk
+  // position l % 8
+  auto issue = [&](int k) {
+    const int buf = k % NBUF, k0 = min(k, NK - 1) * CG_KS;
+#pragma unroll
+    for (int c = 0; c < CG_TN / 32; ++c) {
+      const int r8 = 8 * (4 * c + wave), r = r8 + (lane >> 3);
+      const int chunk = (lane & 7) ^ (r & 7);
+      const int i = r & 15, blk = (r >> 4) & 3;
+      const int col = (r & 64) + 16 * (i >> 2) + 4 * blk + (i & 3);
+      ct_lds_load16(rw, ct_lds_addr(&sW[buf][r8 * CG_KS * 2]),
+                    (uint32_t)((col * D + k0 + 8 * chunk) * 2));
+    }
+#pragma unroll
+    for (int c = 0; c < TM / 32; ++c) {
+      const int r8 = 8 * (4 * c + wave), r = r8 + (lane >> 3);
+      const int chunk = (lane & 7) ^ (r & 7);
+      // rows past M read the last row
+      ct_lds_load16(rx, ct_lds_addr(&sX[buf][r8 * CG_KS * 2]),
+                    (uint32_t)(((long long)min(r, rows - 1) * p.x_ld + k0 + 8 * chunk) * 2));
+    }
+  };
+  const int wr = (wave >> 1) * (TM / 2), wc = (wave & 1) * 64;
+  dkv_f32x4 acc[RB][4], tot[RB][4];
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+    for (int blk = 0; blk < 4; ++blk) {
+      acc[rb][blk] = dkv_f32x4{0.f, 0.f, 0.f, 0.f};
+      tot[rb][blk] = dkv_f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+#pragma unroll
+  for (int k = 0; k < NBUF - 1; ++k) issue(k);
+#pragma unroll 1
+  for (int q = 0; q < 4; ++q) {
+#pragma unroll 1
+    for (int kk = 0; kk < NK / 4; ++kk) {
+      const int k = q * (NK / 4) + kk;
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NBUF - 2) * LOADS) : "memory");  // step k's loads are done
+      __syncthreads();  // step k is in LDS for every wave; the buffer of step k - 1 is free
+      issue(k + NBUF - 1);
+      const uint8_t *wt = sW[k % NBUF], *xt = sX[k % NBUF];
+#pragma unroll
+      for (int s = 0; s < CG_KS / 32; ++s) {
+        const int pos = 16 * ((4 * s + g) ^ (n & 7));
+        dkv_u32x4 a[4], b[RB];
+#pragma unroll
+        for (int blk = 0; blk < 4; ++blk)
+          a[blk] = *(const dkv_u32x4*)(wt + (wc + 16 * blk + n) * (CG_KS * 2) + pos);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+          b[rb] = *(const dkv_u32x4*)(xt + (wr + 16 * rb + n) * (CG_KS * 2) + pos);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+          for (int blk = 0; blk < 4; ++blk)
+            acc[rb][blk] = mfma_16x16x32<DT>(a[blk], b[rb], acc[rb][blk]);
+      }
+    }
+#pragma unroll
+    for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+      for (int blk = 0; blk < 4; ++blk) {
+        tot[rb][blk] += acc[rb][blk];
+        acc[rb][blk] = dkv_f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  const int n0 = col0 + wc + 16 * g;  // this lane's 16 logits
+  float bias[16];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) bias[e] = elt_f32<DT>(cm.b[(long long)grp * D + n0 + e]);
+#pragma unroll
+  for (int rb = 0; rb < RB; ++rb) {
+    const int m = row0 + wr + 16 * rb + n;
+    if (m >= p.M) continue;
+    uint32_t w[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const int blk = e >> 1, u = 2 * (e & 1);
+      w[e] = (uint32_t)f32_elt<DT>(tot[rb][blk][u] + bias[2 * e]) |
+             ((uint32_t)f32_elt<DT>(tot[rb][blk][u + 1] + bias[2 * e + 1]) << 16);
+    }
+    uint16_t* lo = cm.logits + ((long long)m * p.G + grp) * D + n0;
+    if (p.vec) {
+      *(dkv_u32x4*)lo = dkv_u32x4{w[0], w[1], w[2], w[3]};
+      *(dkv_u32x4*)(lo + 8) = dkv_u32x4{w[4], w[5], w[6], w[7]};
+    } else {
+#pragma unroll
+      for (int e = 0; e < 16; ++e) lo[e] = (uint16_t)(w[e / 2] >> (16 * (e & 1)));
+    }
+  }
+}
+
+// e^d of d <= 0: exp2 of the product's leading part times its remainder (log2(e) as a hi + lo
+// pair), so the relative error stays that of v_exp_f32. d = -inf gives 0, NaN stays NaN.
+__device__ __forceinline__ float cf_exp(float d) {
+  constexpr float L_HI = 1.44269502162933349609375f, L_LO = 1.92596299112661746887e-8f;
+  constexpr float LN2 = 0.693147180559945286f;
+  d = d < -200.f ? -200.f : d;  // 2^-288 is 0 in fp32; a NaN fails the compare and stays
+  const float y = d * L_HI;
+  const float r = __builtin_fmaf(d, L_LO, __builtin_fmaf(d, L_HI, -y));
+  const float e = __builtin_amdgcn_exp2f(y);
+  return __builtin_fmaf(e, r * LN2, e);
+}
+
+// a / s from r = 1 / s: the product and one correction step (within an ulp of the division).
+__device__ __forceinline__ float cf_div(float a, float s, float r) {
+  const float q = a * r;
+  return __builtin_fmaf(__builtin_fmaf(-q, s, a), r, q);
+}
+
 // The retained count of one (row m, group g) of a matrix, computed by one wave from the
 // row's rounded logits (global workspace or LDS). Lane l owns the E = D / 64 consecutive
 // positions l*E .. l*E + E - 1 of the row.
@@ -189,22 +348,23 @@ __device__ __forceinline__ int cutoff_row_len(const CutoffParams& p, const uint1
   float s = 0.f;
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    x[e] = expf(x[e] - mx);
+    x[e] = cf_exp(x[e] - mx);
     s += x[e];
   }
   s = dkv_wave_sum_fast(s);
   // probabilities in the compute dtype, then their prefix sums accumulated in fp32
+  const float rcp = 1.0f / s;
   float run = 0.f;
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    run += dkv_round_to<DT>(x[e] / s);
+    run += dkv_round_to<DT>(cf_div(x[e], s, rcp));
     x[e] = run;  // inclusive prefix within the lane
   }
   const float inc = dkv_wave_scan_fast(run);  // inclusive scan of the lane totals
   const float excl = inc - run;
   int cnt = 0;
 #pragma unroll
-  for (int e = 0; e < E; ++e) cnt += dkv_round_to<DT>(excl + x[e]) >= p.threshold ? 1 : 0;
+  for (int e = 0; e < E; ++e) cnt += excl + x[e] >= p.count_min ? 1 : 0;
   cnt = dkv_wave_sum_fast_i(cnt);
   return min(cnt, max(p.low_rank, 0));
 }
@@ -255,7 +415,7 @@ __global__ __launch_bounds__(256) void cutoff_rows_kernel(CutoffParams p) {
   row_task<DT, E>(p, (int)(task / n_rows), task % n_rows, lane);
 }
 
-// Few rows (M <= 16, D <= 128: a decode step) in one launch of 8 waves per (group, K|V): the
+// Few rows of D <= 128 (a decode step) in one launch of 8 waves per (16 rows, group, K|V): the
 // logits of the rows go to LDS (wave w: output columns 16w .. 16w+15; every operand load issued
 // before the first product, the masked copies' inputs loaded ahead as well), then wave w takes
 // rows w and w + 8: count, masked copy, length. One memory round trip before the stores.
@@ -263,7 +423,7 @@ constexpr int CS_WAVES = 8;
 
 template <int DT>
 __device__ __forceinline__ void small_logits(const CutoffParams& p, int mat, int g, int wave,
-                                             int lane, uint16_t (*sLog)[128], int row0 = 0) {
+                                             int lane, uint16_t (*sLog)[128], int row0) {
   const int n0 = 16 * wave;
   if (n0 >= p.D) return;
   const int i = lane & 15, kg = lane >> 4;
@@ -300,26 +460,26 @@ template <int DT, int E>
 __global__ __launch_bounds__(64 * CS_WAVES) void cutoff_small_kernel(CutoffParams p) {
   __shared__ uint16_t sLog[CT_ROWS][128];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int mat = blockIdx.x & 1, g = blockIdx.x >> 1;
+  const int mat = blockIdx.x & 1, g = blockIdx.x >> 1, row0 = blockIdx.y * CT_ROWS;
   const CutoffMat& cm = p.mat[mat];
   const int D = p.D;
   uint16_t xr[2][E];
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
-    const int m = min(wave + CS_WAVES * r, p.M - 1);
+    const int m = min(row0 + wave + CS_WAVES * r, p.M - 1);
     const uint16_t* xs = cm.x + (long long)m * p.x_ld + (long long)g * D + lane * E;
 #pragma unroll
     for (int e = 0; e < E; ++e) xr[r][e] = xs[e];
   }
-  small_logits<DT>(p, mat, g, wave, lane, sLog);
+  small_logits<DT>(p, mat, g, wave, lane, sLog, row0);
   __syncthreads();
   constexpr uint16_t EXP = DT == DKV_BF16 ? 0x7f80 : 0x7c00;
   constexpr uint16_t QNAN = DT == DKV_BF16 ? 0x7fc0 : 0x7e00;
 #pragma unroll
   for (int r = 0; r < 2; ++r) {
-    const int m = wave + CS_WAVES * r;
+    const int m = row0 + wave + CS_WAVES * r;
     if (m >= p.M) break;
-    const int len = cutoff_row_len<DT, E>(p, &sLog[m][0], lane);
+    const int len = cutoff_row_len<DT, E>(p, &sLog[m - row0][0], lane);
     uint16_t* xo = cm.out + (long long)m * p.out_ld + (long long)g * D + lane * E;
     // x * 1 or x * 0 written bitwise, as row_task writes them
 #pragma unroll
@@ -329,6 +489,165 @@ __global__ __launch_bounds__(64 * CS_WAVES) void cutoff_small_kernel(CutoffParam
       xo[e] = lane * E + e < len ? xb : zb;
     }
     if (lane == 0) cm.lens[(long long)m * p.len_ld + g] = len;
+  }
+}
+
+// max / sum over the four lanes n, n + 16, n + 32, n + 48
+__device__ __forceinline__ float cf_max4(float v) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+}
+__device__ __forceinline__ float cf_sum4(float v) {
+  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
+constexpr int CF_WAVES = 4;
+
+// The whole cutoff head of a prompt with D = 16 * NB <= 128 in one launch. Workgroup (x, group
+// and matrix): W_g staged once in LDS in operand order, then each wave takes 16-row tiles
+// grid-stride, the next tile's rows loading while one is worked on.
+// MFMA operands: A = W rows (the logits), B = x rows, with the W rows permuted so that lane
+// (row n = lane % 16, g = lane / 16) receives the D / 4 consecutive logits D / 4 * g .. of its
+// row: A row i of block blk is logit D / 4 * (i / 4) + 4 * blk + i % 4. A row's maximum, sum
+// and prefix sums then need two exchanges between four lanes instead of six steps across the
+// wave for each, for 16 rows at once, and the masked copy is the B operand itself.
+// Bound: VALU (softmax and counts, ~25 instructions per logit) and HBM about alike. 8192 rows x
+// 8 groups x 128, bf16: 31.7 us for 102 MB (3.2 TB/s; two kernels, one a wave per row, 108.3).
+template <int DT, int NB>
+__global__ __launch_bounds__(64 * CF_WAVES, 3) void cutoff_fused_kernel(CutoffParams p) {
+  constexpr int D = 16 * NB, KS = D / 32, PL = D / 4;  // PL: logits per lane
+  __shared__ __attribute__((aligned(16))) dkv_u32x4 sW[NB * KS][64];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, g = lane >> 4;
+  const int mat = blockIdx.y & 1, grp = blockIdx.y >> 1;
+  const CutoffMat& cm = p.mat[mat];
+  const int tiles = (p.M + 15) / 16, step = gridDim.x * CF_WAVES;
+  int tile = blockIdx.x * CF_WAVES + wave;
+
+  dkv_u32x4 xn[KS];
+  auto load_x = [&](int t) {
+    // rows past M (and tiles past the last) read the last row
+    const uint16_t* xr = cm.x + (long long)min(16 * t + n, p.M - 1) * p.x_ld + grp * D + 8 * g;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) xn[s] = *(const dkv_u32x4*)(xr + 32 * s);
+  };
+  load_x(tile);
+  for (int f = wave; f < NB * KS; f += CF_WAVES) {
+    const int blk = f / KS, s = f % KS;
+    sW[f][lane] = *(const dkv_u32x4*)(
+        cm.wt + ((long long)grp * D + PL * (n >> 2) + 4 * blk + (n & 3)) * D + 32 * s + 8 * g);
+  }
+  uint32_t bias[PL / 2];  // packed pairs of this lane's logits
+#pragma unroll
+  for (int e = 0; e < PL / 2; ++e) {
+    const uint16_t* b = cm.b + grp * D + PL * g + 2 * e;
+    bias[e] = (uint32_t)b[0] | ((uint32_t)b[1] << 16);
+  }
+  __syncthreads();
+
+  for (; tile < tiles; tile += step) {
+    // keeps the W operands in LDS: hoisted out of the loop they would take 128 registers
+    asm volatile("" ::: "memory");
+    dkv_u32x4 x[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) x[s] = xn[s];
+    load_x(tile + step);
+
+    dkv_f32x4 acc[NB];
+#pragma unroll
+    for (int blk = 0; blk < NB; ++blk) {
+      acc[blk] = dkv_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int s = 0; s < KS; ++s)
+        acc[blk] = mfma_16x16x32<DT>(sW[blk * KS + s][lane], x[s], acc[blk]);
+    }
+    // the rounded logits, packed (element e of the lane: logit PL * g + e)
+    uint32_t lg[PL / 2];
+#pragma unroll
+    for (int e = 0; e < PL / 2; ++e) {
+      const float v0 = acc[e / 2][2 * (e & 1)] + elt_f32<DT>((uint16_t)bias[e]);
+      const float v1 = acc[e / 2][2 * (e & 1) + 1] + elt_f32<DT>((uint16_t)(bias[e] >> 16));
+      lg[e] = (uint32_t)f32_elt<DT>(v0) | ((uint32_t)f32_elt<DT>(v1) << 16);
+    }
+    const int m = 16 * tile + n;
+    const bool live = m < p.M;
+    if (live) {
+      uint16_t* lo = cm.logits + ((long long)m * p.G + grp) * D + PL * g;
+      if (p.vec) {
+#pragma unroll
+        for (int v = 0; v < PL / 8; ++v)
+          *(dkv_u32x4*)(lo + 8 * v) =
+              dkv_u32x4{lg[4 * v], lg[4 * v + 1], lg[4 * v + 2], lg[4 * v + 3]};
+      } else {
+#pragma unroll
+        for (int e = 0; e < PL; ++e) lo[e] = (uint16_t)(lg[e / 2] >> (16 * (e & 1)));
+      }
+    }
+    auto logit = [&](int e) { return elt_f32<DT>((uint16_t)(lg[e / 2] >> (16 * (e & 1)))); };
+    float mx = logit(0);
+#pragma unroll
+    for (int e = 1; e < PL; ++e) mx = fmaxf(mx, logit(e));
+    mx = cf_max4(mx);
+    float pr[PL];
+    float part[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int e = 0; e < PL; ++e) {
+      pr[e] = cf_exp(logit(e) - mx);
+      part[e & 3] += pr[e];
+    }
+    const float sum = cf_sum4((part[0] + part[1]) + (part[2] + part[3]));
+    // probabilities in the compute dtype, their prefix sums in fp32
+    const float rcp = 1.0f / sum;
+    float run = 0.f;
+#pragma unroll
+    for (int e = 0; e < PL; ++e) {
+      run += dkv_round_to<DT>(cf_div(pr[e], sum, rcp));
+      pr[e] = run;
+    }
+    // the totals of the row's lanes before this one
+    const float t16 = __shfl_xor(run, 16, 64);
+    const float t32 = __shfl_xor(run + t16, 32, 64);
+    const float excl = ((g & 1) ? t16 : 0.f) + ((g & 2) ? t32 : 0.f);
+    // a prefix sum counts when its rounding reaches the threshold, i.e. when it reaches the
+    // smallest fp32 value that rounds to it
+    int cnt = 0;
+#pragma unroll
+    for (int e = 0; e < PL; ++e) cnt += excl + pr[e] >= p.count_min ? 1 : 0;
+    cnt += __shfl_xor(cnt, 16, 64);
+    cnt += __shfl_xor(cnt, 32, 64);
+    const int len = min(cnt, max(p.low_rank, 0));
+
+    if (!live) continue;
+    // x * 1 or x * 0 written bitwise, as row_task writes them
+    constexpr uint32_t EXP = DT == DKV_BF16 ? 0x7f80u : 0x7c00u;
+    constexpr uint32_t QNAN = DT == DKV_BF16 ? 0x7fc0u : 0x7e00u;
+    uint16_t* xo = cm.out + (long long)m * p.out_ld + grp * D + 8 * g;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const uint32_t w[4] = {x[s].x, x[s].y, x[s].z, x[s].w};
+      const int keep = len - 32 * s - 8 * g;  // elements of this piece that stay
+      uint32_t o[4];
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const uint32_t a = w[d] & 0xffffu, b = w[d] >> 16;
+        const uint32_t za = (a & EXP) == EXP ? QNAN : (a & 0x8000u);
+        const uint32_t zb = (b & EXP) == EXP ? QNAN : (b & 0x8000u);
+        o[d] = (2 * d < keep ? a : za) | ((2 * d + 1 < keep ? b : zb) << 16);
+      }
+      if (p.vec) {
+        *(dkv_u32x4*)(xo + 32 * s) = dkv_u32x4{o[0], o[1], o[2], o[3]};
+      } else {
+#pragma unroll
+        for (int e = 0; e < 8; ++e) xo[32 * s + e] = (uint16_t)(o[e / 2] >> (16 * (e & 1)));
+      }
+    }
+    if (g == 0) cm.lens[(long long)m * p.len_ld + grp] = len;
   }
 }
 
@@ -379,7 +698,7 @@ __device__ __forceinline__ void append_row(const TailParams& t, int mat, long lo
 
 // One launch for the whole tail of a decode step's cutoff head: workgroup 2g + mat computes the
 // logits of group g of matrix mat (K or V) for 16 rows at a time (wave w: columns 16w + 64c, as
-// cutoff_logits_kernel computes them), then its waves take those rows' counts and appends;
+// logits_tile computes them), then its waves take those rows' counts and appends;
 // the workgroups past 2G rotate the query rows (RoPE at position pos), one per wave.
 template <int DT, int E>
 __global__ __launch_bounds__(256) void cutoff_layer_kernel(TailParams t) {
@@ -463,10 +782,47 @@ __global__ __launch_bounds__(64 * CS_WAVES) void cutoff_layer_small_kernel(TailP
     dkv_rope_pair<DT>(t.q + (qr / t.Hq) * t.q_sb + (qr % t.Hq) * 128, lane, t.pos, t.log_theta);
 }
 
-// the logits of every (row, group, K|V) into the workspace: split-K for D of 256 and more
+template <int DT, int STEPS, int TM>
+void launch_logits_tile(const CutoffParams& p, hipStream_t st) {
+  const int nc = 128 * STEPS / CG_TN, rt = (p.M + TM - 1) / TM;
+  const unsigned grid = (unsigned)(8LL * nc * ((rt + 3) / 4) * p.G);
+  hipLaunchKernelGGL((cutoff_logits_tile_kernel<DT, STEPS, TM>), dim3(grid), dim3(256), 0, st, p);
+}
+
+// The logits of every (row, group, K|V) into the workspace, D of 256, 512 or 1024. Graph-replayed
+// us of the whole call (bf16 / fp16, one group, D = 1024), split-K / 32-row / 64-row tiles: 64
+// rows 9.5 / 11.0 / 12.3, 100 rows 13.0 / 11.2 / 12.4, 512 rows 35.8 / 12.6 / 13.7, 800 rows 52.9
+// / 16.1 / 15.4, 3001 rows 122.6 / 42.4 / 32.7; D = 512: 150 rows 8.2 / 8.6 / 9.3, 512 rows
+// 13.1 / 9.0 / 9.7, 1500 rows 30.0 / 12.5 / 12.0; D = 256: 301 rows 6.4 / 7.3, 800 rows 9.3 /
+// 8.0. So the split-K kernel while its workgroups stay within three per CU (its 16 x 16 tiles
+// read 64 KB of operands for 0.5 MFLOP, but all at once), then 32-row tiles while they leave CUs
+// idle or about fill them, then 64-row ones. The tile kernels address x by 32-bit offsets
+// from a tile's first row, so a larger row stride stays on split-K.
 void launch_logits(const CutoffParams& p, int dtype, hipStream_t st) {
   const int D = p.D, M = p.M, G = p.G;
   const unsigned gy = (unsigned)((M + CT_ROWS - 1) / CT_ROWS), gz = (unsigned)(2 * G);
+  if ((long long)(D / 16) * gy * gz > 3 * 256 && p.x_ld < (1LL << 23)) {
+#define DKV_LT(STEPS_, TM_)                             \
+  do {                                                  \
+    if (dtype == DKV_BF16)                              \
+      launch_logits_tile<DKV_BF16, STEPS_, TM_>(p, st); \
+    else                                                \
+      launch_logits_tile<DKV_F16, STEPS_, TM_>(p, st);  \
+  } while (0)
+    const bool small = (long long)(D / CG_TN) * ((M + 31) / 32) * gz <= 320;
+    if (D == 1024) {
+      if (small) DKV_LT(8, 32);
+      else DKV_LT(8, 64);
+    } else if (D == 512) {
+      if (small) DKV_LT(4, 32);
+      else DKV_LT(4, 64);
+    } else {
+      if (small) DKV_LT(2, 32);
+      else DKV_LT(2, 64);
+    }
+#undef DKV_LT
+    return;
+  }
 #define DKV_LKS(STEPS_)                                                                        \
   do {                                                                                         \
     if (dtype == DKV_BF16)                                                                     \
@@ -480,12 +836,8 @@ void launch_logits(const CutoffParams& p, int dtype, hipStream_t st) {
     DKV_LKS(8);
   else if (D == 512)
     DKV_LKS(4);
-  else if (D == 256)
-    DKV_LKS(2);
-  else if (dtype == DKV_BF16)
-    hipLaunchKernelGGL(cutoff_logits_kernel<DKV_BF16>, dim3(D / CT_COLS, gy, gz), dim3(256), 0, st, p);
   else
-    hipLaunchKernelGGL(cutoff_logits_kernel<DKV_F16>, dim3(D / CT_COLS, gy, gz), dim3(256), 0, st, p);
+    DKV_LKS(2);
 #undef DKV_LKS
 }
 
@@ -494,6 +846,31 @@ void launch_rows(const CutoffParams& p, hipStream_t st) {
   const long long tasks = 2LL * p.M * p.G;
   hipLaunchKernelGGL((cutoff_rows_kernel<DT, E>), dim3((unsigned)((tasks + 3) / 4)), dim3(256), 0,
                      st, p);
+}
+
+template <int DT, int NB>
+void launch_fused(const CutoffParams& p, hipStream_t st) {
+  // about three resident workgroups per CU (registers); every wave the same number of tiles
+  const int tiles = (p.M + 15) / 16;
+  const int most = max(1, 3 * 256 / (2 * p.G));
+  const int per_wave = (tiles + most * CF_WAVES - 1) / (most * CF_WAVES);
+  const int gx = (tiles + per_wave * CF_WAVES - 1) / (per_wave * CF_WAVES);
+  hipLaunchKernelGGL((cutoff_fused_kernel<DT, NB>), dim3(gx, 2 * p.G), dim3(64 * CF_WAVES), 0, st,
+                     p);
+}
+
+// The smallest fp32 value whose rounding to the compute dtype is >= thr (a value of that
+// dtype): the midpoint between thr and its predecessor, or the next fp32 value when the tie
+// goes to the predecessor.
+float count_min_of(int dtype, float thr) {
+  if (!(thr > 0.f) || !(thr <= 2.f)) return thr <= 0.f ? -INFINITY : thr;  // prefix sums are in [0, ~1]
+  const uint16_t bits = dtype == DKV_BF16 ? __builtin_bit_cast(uint16_t, (__bf16)thr)
+                                          : __builtin_bit_cast(uint16_t, (_Float16)thr);
+  const uint16_t prev_bits = (uint16_t)(bits - 1);
+  const float prev = dtype == DKV_BF16 ? (float)__builtin_bit_cast(__bf16, prev_bits)
+                                       : (float)__builtin_bit_cast(_Float16, prev_bits);
+  const float mid = prev + 0.5f * (thr - prev);  // exact: one more bit than the dtype holds
+  return (bits & 1) == 0 ? mid : nextafterf(mid, INFINITY);
 }
 
 }  // namespace
@@ -543,21 +920,49 @@ extern "C" int dkv_cutoff_kv(void* stream, int dtype, const void* xk, const void
   p.D = D;
   p.low_rank = low_rank < 0 ? D : min(low_rank, D);
   // the reference compares against 0.1 in the compute dtype
-  p.threshold = dtype == DKV_BF16 ? (float)(__bf16)threshold : (float)(_Float16)threshold;
+  p.count_min = count_min_of(
+      dtype, dtype == DKV_BF16 ? (float)(__bf16)threshold : (float)(_Float16)threshold);
+  p.vec = (((uintptr_t)out_k | (uintptr_t)out_v | (uintptr_t)workspace) % 16 == 0 &&
+           out_ld % 8 == 0)
+              ? 1
+              : 0;
   const int E = D / 64;
   if (E != 1 && E != 2 && E != 4 && E != 8 && E != 16) return DKV_E_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
-  if (M <= CT_ROWS && D <= 128) {
+  // D <= 128: the 8-wave kernel (a 16-row tile per workgroup) while the tiles about fill the
+  // 256 CUs once, the wave-per-tile kernel past that. Graph-replayed us per call, 8-wave / wave
+  // per tile: G = 8, D = 128: 33 rows 5.2 / 6.7, 301 rows 7.0 / 7.2, 1024 rows 13.4 / 8.5, 8192
+  // rows 72.3 / 31.7 (two kernels, a wave per row, before: 5.9, 8.7, 19.6, 108.3); G = 4: 301
+  // rows 5.3 / 7.1, 1024 rows 8.4 / 7.7.
+  const long long row_tiles = (M + CT_ROWS - 1) / CT_ROWS;
+  if (D <= 128 && (row_tiles == 1 || 2 * G * row_tiles <= 320)) {
+    const dim3 sgrid((unsigned)(2 * G), (unsigned)row_tiles);
     if (dtype == DKV_BF16) {
       if (E == 1)
-        hipLaunchKernelGGL((cutoff_small_kernel<DKV_BF16, 1>), dim3(2 * G), dim3(64 * CS_WAVES), 0, st, p);
+        hipLaunchKernelGGL((cutoff_small_kernel<DKV_BF16, 1>), sgrid, dim3(64 * CS_WAVES), 0, st, p);
       else
-        hipLaunchKernelGGL((cutoff_small_kernel<DKV_BF16, 2>), dim3(2 * G), dim3(64 * CS_WAVES), 0, st, p);
+        hipLaunchKernelGGL((cutoff_small_kernel<DKV_BF16, 2>), sgrid, dim3(64 * CS_WAVES), 0, st, p);
     } else {
       if (E == 1)
-        hipLaunchKernelGGL((cutoff_small_kernel<DKV_F16, 1>), dim3(2 * G), dim3(64 * CS_WAVES), 0, st, p);
+        hipLaunchKernelGGL((cutoff_small_kernel<DKV_F16, 1>), sgrid, dim3(64 * CS_WAVES), 0, st, p);
       else
-        hipLaunchKernelGGL((cutoff_small_kernel<DKV_F16, 2>), dim3(2 * G), dim3(64 * CS_WAVES), 0, st, p);
+        hipLaunchKernelGGL((cutoff_small_kernel<DKV_F16, 2>), sgrid, dim3(64 * CS_WAVES), 0, st, p);
+    }
+    DKV_HIP_CHECK_LAUNCH();
+    return DKV_OK;
+  }
+  if (D <= 128) {
+    if (2 * G > 65535) return DKV_E_UNSUPPORTED;
+    if (dtype == DKV_BF16) {
+      if (E == 1)
+        launch_fused<DKV_BF16, 4>(p, st);
+      else
+        launch_fused<DKV_BF16, 8>(p, st);
+    } else {
+      if (E == 1)
+        launch_fused<DKV_F16, 4>(p, st);
+      else
+        launch_fused<DKV_F16, 8>(p, st);
     }
     DKV_HIP_CHECK_LAUNCH();
     return DKV_OK;
@@ -572,8 +977,6 @@ extern "C" int dkv_cutoff_kv(void* stream, int dtype, const void* xk, const void
       launch_rows<DKV_F16, e>(p, st);                           \
     break;
   switch (E) {
-    DKV_ROWS_CASE(1)
-    DKV_ROWS_CASE(2)
     DKV_ROWS_CASE(4)
     DKV_ROWS_CASE(8)
     DKV_ROWS_CASE(16)
@@ -629,7 +1032,9 @@ int dkv_layer_cutoff_append_rope(void* stream, const DkvDecodeLayer* L, const vo
   p.G = G;
   p.D = D;
   p.low_rank = L->low_rank < 0 ? D : min(L->low_rank, D);
-  p.threshold = dtype == DKV_BF16 ? (float)(__bf16)L->threshold : (float)(_Float16)L->threshold;
+  p.count_min = count_min_of(
+      dtype, dtype == DKV_BF16 ? (float)(__bf16)L->threshold : (float)(_Float16)L->threshold);
+  p.vec = 0;
   t.flat[0] = L->flat_k;
   t.flat[1] = L->flat_v;
   t.flat_ld[0] = L->flat_k_ld;
