@@ -10,8 +10,9 @@
 // Here: dkv_rope_dense rotates dense K in place (rotate-half RoPE, fp32 angles
 // float(pos) * inv_freq as the decode kernels form them, result rounded to the cache dtype);
 // dkv_prefill_attention is a causal GQA flash-attention forward on MFMA:
-//   one workgroup = 128 queries of one query head (4 waves x 2 blocks of 16 queries, so every
-//   K and V operand read from LDS serves two products), the work items handed out longest
+//   one workgroup = 64 or 128 queries of one query head (4 waves x 2 blocks of 16 queries for a
+//   grid that fills the chip several times, so every K and V operand read from LDS serves two
+//   products; smaller grids 8 or 4 waves of one block), the work items handed out longest
 //   first and evenly over the 8 XCDs, a KV head's query heads on one XCD (the grid's own
 //   order gave XCD k only the query blocks k, k+8, ...: 0.40 ms against 0.25 at B=4,
 //   S=2048); key tiles of 64
@@ -20,16 +21,14 @@
 //   S^T = K Q^T on 16x16x32 MFMA (each lane then holds one query's scores for 16 keys), online
 //   softmax in fp32 with lane maxima by permlane swaps (the running maximum raised only when a
 //   tile's exceeds it by more than 2^8, so most tiles skip the rescale), P kept as a bf16/fp16
-//   hi + lo pair and
-//   P.V on 16x16x32 MFMA with both parts in the k dimension (V read transposed from LDS).
+//   hi + lo pair and P.V on 16x16x32 MFMA over 32 keys at a time, one product with the hi parts
+//   and one with the lo parts against the same V operand (read transposed from LDS ahead of the
+//   softmax).
 #include "dkv_common.h"
 
 namespace {
 
 constexpr int FA_DH = 128;
-constexpr int FA_QB = 2;      // 16-query blocks per wave
-constexpr int FA_QW = 16 * FA_QB;  // queries per wave
-constexpr int FA_BQ = 4 * FA_QW;   // queries per workgroup (4 waves)
 constexpr float FA_RESCALE = 8.f;  // log2 units a tile's maximum may exceed the running one
 constexpr int FA_BK = 64;     // keys per tile
 constexpr int FA_TILE_BYTES = FA_BK * FA_DH * 2;  // 16 KB
@@ -60,9 +59,9 @@ __device__ __forceinline__ dkv_f32x4 mfma32(const dkv_u32x4& a, const dkv_u32x4&
 }
 
 __device__ __forceinline__ void fa_lds_load16(__amdgpu_buffer_rsrc_t rsrc, uint32_t lds_base,
-                                              uint32_t byte_off) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
-               ::"s"(lds_base), "v"(byte_off), "s"(rsrc)
+                                              uint32_t byte_off, uint32_t tile_off) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds"
+               ::"s"(lds_base), "v"(byte_off), "s"(rsrc), "s"(tile_off)
                : "memory", "m0");
 }
 
@@ -73,6 +72,12 @@ __device__ __forceinline__ uint32_t fa_lds_addr(const void* p) {
 __device__ __forceinline__ float fa_max(float a, float b) {
   float r;
   asm("v_max_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+  return r;
+}
+
+__device__ __forceinline__ float fa_max3(float a, float b, float c) {
+  float r;
+  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
   return r;
 }
 
@@ -108,12 +113,21 @@ __device__ __forceinline__ void split_hi_lo(const float (&p)[4], dkv_u32x2& hi, 
   }
 }
 
-// grid: (ceil(Sq / 128), Hq, B); 256 threads (the workgroup's item is remapped from its
-// linear id, see below). ODT: output dtype (DT or fp32).
-template <int DT, int ODT>
-__global__ __launch_bounds__(256, 2) void fa_prefill_kernel(PrefillParams p) {
-  __shared__ __attribute__((aligned(16))) uint8_t sK[2][FA_TILE_BYTES];
-  __shared__ __attribute__((aligned(16))) uint8_t sV[2][FA_TILE_BYTES];
+// grid: (ceil(Sq / (16 QB NW)), Hq, B); NW waves of QB blocks of 16 queries (the workgroup's item
+// is remapped from its linear id, see below). ODT: output dtype (DT or fp32).
+// Bound: issue slots. Per wave and tile (QB = 2) 96 products of 16 cycles against ~235 vector
+// instructions, which measure 6.6 cycles each beside a full product stream (10.5 for exp2): the
+// vector work of one wave has to fit beside the products of the others. B = 4, S = 2048, 32/8
+// heads: 187 us, 1.1 PFLOP/s of products (203 us with each P.V operand pair built by two moves, a
+// serial maximum chain and per-lane load offsets for every tile).
+template <int DT, int ODT, int FA_QB, int FA_NW>
+__global__ __launch_bounds__(64 * FA_NW, FA_NW == 8 ? 4 : 2) void fa_prefill_kernel(PrefillParams p) {
+  constexpr int FA_QW = 16 * FA_QB;     // queries per wave
+  constexpr int FA_BQ = FA_NW * FA_QW;  // queries per workgroup
+  constexpr int FA_LW = FA_BK / 4 / FA_NW;  // K (or V) loads per wave and tile
+  // 1 KB aligned: the operand reads form their addresses by exclusive-or
+  __shared__ __attribute__((aligned(1024))) uint8_t sK[2][FA_TILE_BYTES];
+  __shared__ __attribute__((aligned(1024))) uint8_t sV[2][FA_TILE_BYTES];
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n = lane & 15, g = lane >> 4;
@@ -175,20 +189,31 @@ __global__ __launch_bounds__(256, 2) void fa_prefill_kernel(PrefillParams p) {
   const __amdgpu_buffer_rsrc_t rv = dkv_make_rsrc(p.v, p.v_bytes);
   const long long kbase = (long long)b * p.k_sb + (long long)kvh * p.k_sh;
   const long long vbase = (long long)b * p.v_sb + (long long)kvh * p.v_sh;
-  // tile loads: wave w, instruction c stores keys 16w + 4c + l/16, LDS chunk position l%16,
-  // which holds the key's 16-byte dims chunk (l%16) ^ (key % 16)
-  auto issue = [&](int t) {
-    const int buf = t & 1;
+  // tile loads: wave w, instruction c stores keys 64 / NW * w + 4c + l/16, LDS chunk position
+  // l%16, which holds the key's 16-byte dims chunk (l%16) ^ (key % 16). A tile inside the key range
+  // moves the lanes' offsets by a scalar; in the last one each lane's key is checked.
+  // (Key 4c + l/16's chunk is key l/16's with 4c added to the exclusive-or.)
+  const int kk0 = FA_BK / FA_NW * wave + (lane >> 4);
+  const uint32_t chunk0 = 16u * ((lane & 15) ^ (kk0 & 15));
+  const uint32_t ko = (uint32_t)((kbase + (long long)kk0 * p.k_ss) * 2);
+  const uint32_t vo = (uint32_t)((vbase + (long long)kk0 * p.v_ss) * 2);
+  auto issue = [&](const __amdgpu_buffer_rsrc_t& rs, uint32_t row, long long ss, uint8_t* buf,
+                   int t) {
+    const uint32_t step = (uint32_t)ss * 2;  // bytes per key
+    const uint32_t dst = fa_lds_addr(buf) + FA_BK / FA_NW * wave * 256;
+    const uint32_t toff = (uint32_t)t * FA_BK * step;
+    if ((t + 1) * FA_BK <= k_end) {
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const int kk = 16 * wave + 4 * c + (lane >> 4);
-      const int key = t * FA_BK + kk;
-      const int chunk = (lane & 15) ^ (kk & 15);
-      const bool ok = key < k_end;
-      const uint32_t ko = ok ? (uint32_t)((kbase + (long long)key * p.k_ss + 8 * chunk) * 2) : 0x7ffffff0u;
-      const uint32_t vo = ok ? (uint32_t)((vbase + (long long)key * p.v_ss + 8 * chunk) * 2) : 0x7ffffff0u;
-      fa_lds_load16(rk, fa_lds_addr(&sK[buf][(16 * wave + 4 * c) * 256]), ko);
-      fa_lds_load16(rv, fa_lds_addr(&sV[buf][(16 * wave + 4 * c) * 256]), vo);
+      for (int c = 0; c < FA_LW; ++c)
+        fa_lds_load16(rs, dst + 4 * c * 256, row + (chunk0 ^ (64u * c)), toff + 4 * c * step);
+    } else {
+#pragma unroll
+      for (int c = 0; c < FA_LW; ++c) {
+        const int key = t * FA_BK + kk0 + 4 * c;
+        fa_lds_load16(rs, dst + 4 * c * 256,
+                      key < k_end ? row + (chunk0 ^ (64u * c)) + toff + 4 * c * step : 0x7ffffff0u,
+                      0u);
+      }
     }
   };
 
@@ -206,36 +231,45 @@ __global__ __launch_bounds__(256, 2) void fa_prefill_kernel(PrefillParams p) {
     l_run[qb] = 0.f;
   }
 
-  if (t0 < n_tiles) issue(t0);
+  // S^T = K Q^T of key block kb: A = K rows (lane: key 16kb + n, dims 32s + 8g .. +8), B = Q^T of
+  // block qb; lane (query n, g) then holds keys 16kb + 4g + u, unscaled (see the maxima below)
+  const uint32_t krd = n * 256 + 16 * (g ^ n);  // + 4096 * kb, dims chunk 4s + g: ^ 64 * s
+  typedef __attribute__((address_space(3))) dkv_u32x4 lds_u32x4;
+  auto qk = [&](uint32_t kt, int kb, dkv_f32x4(&z)[FA_QB][4]) {
+#pragma unroll
+    for (int qb = 0; qb < FA_QB; ++qb) z[qb][kb] = dkv_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const dkv_u32x4 a = *(const lds_u32x4*)(((kt + krd) ^ (64 * s)) + 4096 * kb);
+#pragma unroll
+      for (int qb = 0; qb < FA_QB; ++qb) z[qb][kb] = mfma32<DT>(a, qop[qb][s], z[qb][kb]);
+    }
+  };
+
+  // transposed V reads: lane L = 4i + q of each 16-lane group reads key 16kb + 4g + i, dims
+  // 16db + 4q .. +3 (8 bytes; ^ 32 * db, + 4096 * kb); lane i then holds dim 16db + i of keys
+  // 4g .. 4g+3
+  const uint32_t vrd = (4 * g + (n >> 2)) * 256 + 16 * (((n & 3) >> 1) ^ (4 * g + (n >> 2))) + 8 * (n & 1);
+  typedef __attribute__((address_space(3))) dkv_i16x4 lds_i16x4;
+
+  if (t0 < n_tiles) {
+    issue(rk, ko, p.k_ss, sK[t0 & 1], t0);
+    issue(rv, vo, p.v_ss, sV[t0 & 1], t0);
+  }
   for (int t = t0; t < n_tiles; ++t) {
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();  // tile t is in LDS for every wave; tile t-1's buffer is free
-    if (t + 1 < n_tiles) issue(t + 1);
+    if (t + 1 < n_tiles) {
+      issue(rk, ko, p.k_ss, sK[(t + 1) & 1], t + 1);
+      issue(rv, vo, p.v_ss, sV[(t + 1) & 1], t + 1);
+    }
     const int key0 = t * FA_BK;
     if (key0 >= wave_k_end) continue;  // every key of the tile is past the wave's queries
-    const uint8_t* kt = sK[t & 1];
-    const uint8_t* vt = sV[t & 1];
-
-    // S^T = K Q^T: A = K rows (lane: key 16kb + n, dims 32s + 8g .. +8), B = Q^T of block qb;
-    // lane (query n, g) then holds keys 16kb + 4g + u
-    float z[FA_QB][4][4];
+    const uint32_t kt = fa_lds_addr(sK[t & 1]);
+    const uint32_t vt = fa_lds_addr(sV[t & 1]) + vrd;
+    dkv_f32x4 z[FA_QB][4];
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      dkv_f32x4 sacc[FA_QB];
-#pragma unroll
-      for (int qb = 0; qb < FA_QB; ++qb) sacc[qb] = dkv_f32x4{0.f, 0.f, 0.f, 0.f};
-      const uint8_t* row = kt + (16 * kb + n) * 256;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const dkv_u32x4 a = *(const dkv_u32x4*)(row + 16 * ((4 * s + g) ^ n));
-#pragma unroll
-        for (int qb = 0; qb < FA_QB; ++qb) sacc[qb] = mfma32<DT>(a, qop[qb][s], sacc[qb]);
-      }
-#pragma unroll
-      for (int qb = 0; qb < FA_QB; ++qb)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) z[qb][kb][u] = sacc[qb][u];  // unscaled (see below)
-    }
+    for (int kb = 0; kb < 4; ++kb) qk(kt, kb, z);
     if (key0 + FA_BK > k_end || key0 < ks || (p.causal && key0 + FA_BK - 1 > p.q_offset + wq0)) {
 #pragma unroll
       for (int qb = 0; qb < FA_QB; ++qb) {
@@ -249,18 +283,31 @@ __global__ __launch_bounds__(256, 2) void fa_prefill_kernel(PrefillParams p) {
           }
       }
     }
+    // V operands of key blocks 0 and 1: read ahead of the softmax
+    dkv_u32x2 vx[8][2];
+    auto vread = [&](int j, int db) {
+      const uint32_t src = (vt ^ (32 * db)) + 8192 * j;
+#pragma unroll
+      for (int kk = 0; kk < 2; ++kk)
+        vx[db][kk] = __builtin_bit_cast(
+            dkv_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4*)(src + 4096 * kk)));
+    };
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int db = 0; db < 8; ++db) vread(0, db);
+    __builtin_amdgcn_sched_barrier(0);
     float tmax[FA_QB];
 #pragma unroll
     for (int qb = 0; qb < FA_QB; ++qb) {
-      float m = z[qb][0][0];
+      float m[4];
 #pragma unroll
       for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-        for (int u = 0; u < 4; ++u) m = fa_max(m, z[qb][kb][u]);
+        m[kb] = fa_max3(fa_max3(z[qb][kb][0], z[qb][kb][1], z[qb][kb][2]), z[qb][kb][3],
+                        z[qb][kb][3]);
       // the scale is applied to the tile's maximum and inside the exponent's fma (one VALU
       // per score less than scaling every score: 2-3% of the launch); it is positive (the
       // entry point checks), so the maximum commutes with it
-      tmax[qb] = fa_max4(m) * p.scale_log2;
+      tmax[qb] = fa_max4(fa_max3(fa_max3(m[0], m[1], m[2]), m[3], m[3])) * p.scale_log2;
     }
     if (__ballot(tmax[0] > m_run[0] + FA_RESCALE || tmax[FA_QB - 1] > m_run[FA_QB - 1] + FA_RESCALE)) {
 #pragma unroll
@@ -278,40 +325,38 @@ __global__ __launch_bounds__(256, 2) void fa_prefill_kernel(PrefillParams p) {
       }
     }
 
-    // P.V: for each key block kb, one 16x16x32 product per 16 dims and query block with
-    // k = 8g + e pairing part e/4 of key 16kb + 4g + e%4 (B: this lane's P hi then lo) with that
-    // key's V values (A: the four keys' values of dim 16db + n, twice)
+    // P of key blocks 2j and 2j + 1, hi and lo parts: the B operands of P.V pair key block 2j's
+    // keys 4g .. 4g+3 in k = 8g .. 8g+3 with key block 2j + 1's in k = 8g+4 .. 8g+7
+    dkv_u32x4 bh[2][FA_QB], bl[2][FA_QB];
+    auto probs = [&](int j, int kk, int qb) {
+      float pu[4];
 #pragma unroll
-    for (int kb = 0; kb < 4; ++kb) {
-      dkv_u32x4 bop[FA_QB];
-#pragma unroll
-      for (int qb = 0; qb < FA_QB; ++qb) {
-        float pu[4];
-#pragma unroll
-        for (int u = 0; u < 4; ++u) {
-          pu[u] = __builtin_amdgcn_exp2f(__builtin_fmaf(z[qb][kb][u], p.scale_log2, -m_run[qb]));
-          l_run[qb] += pu[u];
-        }
-        dkv_u32x2 ph, pl;
-        split_hi_lo<DT>(pu, ph, pl);
-        bop[qb] = dkv_u32x4{ph.x, ph.y, pl.x, pl.y};
+      for (int u = 0; u < 4; ++u) {
+        pu[u] = __builtin_amdgcn_exp2f(
+            __builtin_fmaf(z[qb][2 * j + kk][u], p.scale_log2, -m_run[qb]));
+        l_run[qb] += pu[u];
       }
-      // transposed read: lane L = 4j + q of each 16-lane group reads key 16kb + 4g + j,
-      // dims 16db + 4q .. +3 (8 bytes); lane i then holds dim 16db + i of keys 4g .. 4g+3
-      const int key = 16 * kb + 4 * g + (n >> 2);
-      const uint8_t* vrow = vt + key * 256;
+      dkv_u32x2 ph, pl;
+      split_hi_lo<DT>(pu, ph, pl);
+      bh[j][qb][2 * kk] = ph.x;
+      bh[j][qb][2 * kk + 1] = ph.y;
+      bl[j][qb][2 * kk] = pl.x;
+      bl[j][qb][2 * kk + 1] = pl.y;
+    };
+#pragma unroll
+    for (int i = 0; i < 2 * FA_QB; ++i) probs(0, i & 1, i >> 1);
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
 #pragma unroll
       for (int db = 0; db < 8; ++db) {
-        const int dchunk = 2 * db + ((n & 3) >> 1);
-        const uint8_t* src = vrow + 16 * (dchunk ^ (key & 15)) + 8 * (n & 1);
-        const dkv_u32x2 xv = __builtin_bit_cast(
-            dkv_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                           (__attribute__((address_space(3))) dkv_i16x4*)(
-                               (__attribute__((address_space(3))) uint8_t*)src)));
-        const dkv_u32x4 aop = __builtin_bit_cast(
-            dkv_u32x4, dkv_u64x2{__builtin_bit_cast(uint64_t, xv), __builtin_bit_cast(uint64_t, xv)});
+        __builtin_amdgcn_sched_barrier(0);
+        const dkv_u32x4 aop = {vx[db][0].x, vx[db][0].y, vx[db][1].x, vx[db][1].y};
+        if (j == 0) vread(1, db);
 #pragma unroll
-        for (int qb = 0; qb < FA_QB; ++qb) acc[qb][db] = mfma32<DT>(aop, bop[qb], acc[qb][db]);
+        for (int qb = 0; qb < FA_QB; ++qb) acc[qb][db] = mfma32<DT>(aop, bh[j][qb], acc[qb][db]);
+#pragma unroll
+        for (int qb = 0; qb < FA_QB; ++qb) acc[qb][db] = mfma32<DT>(aop, bl[j][qb], acc[qb][db]);
+        if (j == 0 && db % (4 / FA_QB) == 4 / FA_QB - 1) probs(1, db / (4 / FA_QB) % 2, db / (8 / FA_QB));
       }
     }
   }
@@ -334,6 +379,32 @@ __global__ __launch_bounds__(256, 2) void fa_prefill_kernel(PrefillParams p) {
           dkv_store_f32<ODT>(p.out, ob + 16 * db + 4 * g + u, acc[qb][db][u] * inv);
     }
   }
+}
+
+template <int DT, int ODT, int QB, int NW>
+void launch_prefill_shape(const PrefillParams& p, hipStream_t st) {
+  constexpr int BQ = 16 * QB * NW;
+  hipLaunchKernelGGL((fa_prefill_kernel<DT, ODT, QB, NW>),
+                     dim3((unsigned)((p.Sq + BQ - 1) / BQ), (unsigned)p.Hq, (unsigned)p.B),
+                     dim3(64 * NW), 0, st, p);
+}
+// The shape by the number of 128-query workgroups: more than two rounds of the 512 that fit the
+// chip take two query blocks per wave (each K and V operand read from LDS serves two products);
+// up to that, one block per wave and 8 waves (four waves per SIMD instead of two, while the LDS
+// reads have room); one workgroup per CU or fewer take 64 queries, for twice the workgroups.
+// Graph-replayed us, 2 blocks x 4 waves / 1 x 8 / 1 x 4 (32 query heads, 8 KV heads): 128
+// workgroups (B = 1, S = 512) 19.4 / 17.2 / 14.2; 256 (B = 1, S = 1024) 33.4 / 29.6 / 26.7; 384
+// (B = 3, S = 512) 23.5 / 21.4 / 21.8; 576 (B = 2, S = 1111) 44.0 / 42.0 / 46.9; 1024 (B = 4, S =
+// 1024) 60.2 / 58.6 / 70.0; 1536 (B = 3, S = 2048) 142 / 146 / 171; 2048 (B = 4) 184 / 193 / 222.
+template <int DT, int ODT>
+void launch_prefill(const PrefillParams& p, hipStream_t st) {
+  const long long wg = (long long)((p.Sq + 127) / 128) * p.Hq * p.B;
+  if (wg > 1024)
+    launch_prefill_shape<DT, ODT, 2, 4>(p, st);
+  else if (wg > 256)
+    launch_prefill_shape<DT, ODT, 1, 8>(p, st);
+  else
+    launch_prefill_shape<DT, ODT, 1, 4>(p, st);
 }
 
 // In-place rotate-half RoPE on dense rows x[r][s][d] (d < 128): position pos0 + s, angle
@@ -466,18 +537,17 @@ extern "C" int dkv_prefill_attention(void* stream, int dtype, const void* q, lon
   p.k_bytes = (uint32_t)(k_elems * 2);
   p.v_bytes = (uint32_t)(v_elems * 2);
   p.kstart = kstart;
-  const dim3 grid((unsigned)((Sq + FA_BQ - 1) / FA_BQ), (unsigned)Hq, (unsigned)B);
   hipStream_t st = (hipStream_t)stream;
   if (dtype == DKV_BF16) {
     if (out_dtype == DKV_F32)
-      hipLaunchKernelGGL((fa_prefill_kernel<DKV_BF16, DKV_F32>), grid, dim3(256), 0, st, p);
+      launch_prefill<DKV_BF16, DKV_F32>(p, st);
     else
-      hipLaunchKernelGGL((fa_prefill_kernel<DKV_BF16, DKV_BF16>), grid, dim3(256), 0, st, p);
+      launch_prefill<DKV_BF16, DKV_BF16>(p, st);
   } else {
     if (out_dtype == DKV_F32)
-      hipLaunchKernelGGL((fa_prefill_kernel<DKV_F16, DKV_F32>), grid, dim3(256), 0, st, p);
+      launch_prefill<DKV_F16, DKV_F32>(p, st);
     else
-      hipLaunchKernelGGL((fa_prefill_kernel<DKV_F16, DKV_F16>), grid, dim3(256), 0, st, p);
+      launch_prefill<DKV_F16, DKV_F16>(p, st);
   }
   DKV_HIP_CHECK_LAUNCH();
   return DKV_OK;
