@@ -9,11 +9,16 @@
 // is R(16T) R(n) composed in fp32 from the rows of the RoPE table (dkv_rope_table: cos and sin
 // of the fp32 angles n * inv_freq and 16T * inv_freq), not a sine and cosine per element.
 //
-// Workgroup = (64 tokens, cache row, K | V), four waves of 16 tokens. The row's basis ([rank]
-// [dim], ranks past R zero) is staged in LDS and read transposed (ds_read_b64_tr_b16) as the A
-// operand (dims x ranks); each lane loads its token's 8 coefficients of a 32-rank chunk as the B
-// operand; the result out^T[dim][token] leaves every lane four consecutive dims of one token
-// for each 16-dim block, and the rotate-half pairs (d, d + 64) in the same lane.
+// Workgroup = (RW * 16 * tiles tokens, cache row, K | V), four waves of 16 tokens at a time. The
+// row's basis ([rank][dim], ranks past R zero) is staged in LDS, read transposed
+// (ds_read_b64_tr_b16) once and kept in registers as the A operand (dims x ranks) of every tile;
+// each lane loads its token's 8 coefficients of a 32-rank chunk as the B operand, a tile ahead. The
+// dims are dealt to the A rows so that lane (token n, g) ends up with dims 16g .. 16g + 15 and
+// 64 + 16g .. of its token: the rotate-half pairs (d, d + 64) in one lane, stored 16 bytes at a
+// time. A lane's positions all have one offset in their 16-position tile, so R(n) stays in
+// registers too.
+// Bound: HBM. B = 4, 8 groups, S = 2048, rank 128 (67 MB): 21 us, 3.2 TB/s; with one 64-token tile
+// per workgroup, the basis staged for each and 8-byte stores 32 us.
 #include "dkv_common.h"
 #include "dkv_mfma_ops.h"
 
@@ -24,11 +29,12 @@ constexpr int RW = 4;  // waves per workgroup (16 tokens each)
 constexpr int RT_FIXED = 17;  // RoPE table rows before the tile rows R(16T)
 
 template <int DT>
-__global__ __launch_bounds__(RW * 64) void recon_kv_kernel(
+__global__ __launch_bounds__(RW * 64, 2) void recon_kv_kernel(
     const uint16_t* __restrict__ ck, const uint16_t* __restrict__ cv, long long c_sr,
     long long c_st, const uint16_t* __restrict__ kb, const uint16_t* __restrict__ vb,
     long long b_sg, long long b_sr, uint16_t* __restrict__ ko, uint16_t* __restrict__ vo,
-    long long o_sr, long long o_st, int G, int S, int R, int pos0, const float* __restrict__ rope) {
+    long long o_sr, long long o_st, int G, int S, int R, int pos0, const float* __restrict__ rope,
+    int tiles) {
   __shared__ __attribute__((aligned(16))) uint16_t sB[DH * DH];  // [rank][dim]
   const bool is_k = blockIdx.z == 0;
   const int row = blockIdx.y, grp = row % G;
@@ -38,14 +44,26 @@ __global__ __launch_bounds__(RW * 64) void recon_kv_kernel(
   const uint16_t* bg = (is_k ? kb : vb) + (long long)grp * b_sg;
   uint16_t* o = is_k ? ko : vo;
 
-  // this lane's token and its coefficient pieces (ranks 32 cc + 8g .. +8; R is a multiple of 8)
-  const int t = (blockIdx.x * RW + wave) * 16 + n;
-  const uint16_t* cr = c + (long long)row * c_sr + (long long)min(t, S - 1) * c_st;
-  dkv_u32x4 xc[4];
+  // a lane's token of tile i and its coefficient pieces (ranks 32 cc + 8g .. +8; R is a multiple
+  // of 8); tokens past S read as zeros
+  const int tok0 = (blockIdx.x * tiles * RW + wave) * 16 + n;
+  const uint16_t* cr = c + (long long)row * c_sr;
+  dkv_u32x4 xn[4];
+  auto load_x = [&](int t) {
+    const uint16_t* cp = cr + (long long)min(t, S - 1) * c_st;
 #pragma unroll
-  for (int cc = 0; cc < 4; ++cc) {
-    const int r0 = 32 * cc + 8 * g;
-    xc[cc] = (t < S && r0 < R) ? *(const dkv_u32x4*)(cr + r0) : dkv_u32x4{0u, 0u, 0u, 0u};
+    for (int cc = 0; cc < 4; ++cc) {
+      const int r0 = 32 * cc + 8 * g;
+      xn[cc] = (t < S && r0 < R) ? *(const dkv_u32x4*)(cp + r0) : dkv_u32x4{0u, 0u, 0u, 0u};
+    }
+  };
+  load_x(tok0);
+  // R(n) of the lane's positions, frequencies 16g .. 16g + 15 as (cos, sin) pairs
+  dkv_f32x4 rn[8];
+  if (is_k) {
+    const float* rp = rope + ((pos0 + n) & 15) * 128 + 32 * g;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) rn[e] = *(const dkv_f32x4*)(rp + 4 * e);
   }
   // the basis, 16-byte pieces (rank r, dims d8 .. d8 + 7), ranks past R as zeros
   for (int pc = tid; pc < DH * DH / 8; pc += RW * 64) {
@@ -54,64 +72,78 @@ __global__ __launch_bounds__(RW * 64) void recon_kv_kernel(
         r < R ? *(const dkv_u32x4*)(bg + (long long)r * b_sr + d8) : dkv_u32x4{0u, 0u, 0u, 0u};
   }
   __syncthreads();
-
-  dkv_f32x4 acc[8];
-#pragma unroll
-  for (int blk = 0; blk < 8; ++blk) acc[blk] = dkv_f32x4{0.f, 0.f, 0.f, 0.f};
+  // A operands: block blk = 4h + b, row i holds dim 64h + 16 (i / 4) + 4b + i % 4; lane (n, g)
+  // receives ranks 32 cc + 8g .. +3 and +4 .. +7 of its row's dim
   typedef __attribute__((address_space(3))) dkv_i16x4 lds_i16x4;
+  dkv_u32x4 a[4][8];
 #pragma unroll
-  for (int cc = 0; cc < 4; ++cc) {
-    if (32 * cc >= R) break;  // uniform: chunks wholly past the rank are zero
+  for (int cc = 0; cc < 4; ++cc)
 #pragma unroll
     for (int blk = 0; blk < 8; ++blk) {
-      // lane (n, g) receives ranks 32 cc + 8g .. +3 and +4 .. +7 of dim 16 blk + n
-      const uint16_t* src = sB + (32 * cc + 8 * g + (n >> 2)) * DH + 16 * blk + 4 * (n & 3);
+      const uint16_t* src = sB + (32 * cc + 8 * g + (n >> 2)) * DH + 64 * (blk >> 2) +
+                            16 * (n & 3) + 4 * (blk & 3);
       const dkv_u32x2 b0 = __builtin_bit_cast(
           dkv_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                          (lds_i16x4*)(__attribute__((address_space(3))) uint16_t*)src));
       const dkv_u32x2 b1 = __builtin_bit_cast(
           dkv_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
                          (lds_i16x4*)(__attribute__((address_space(3))) uint16_t*)(src + 4 * DH)));
-      acc[blk] = dkv_mfma32<DT>(dkv_u32x4{b0.x, b0.y, b1.x, b1.y}, xc[cc], acc[blk]);
+      a[cc][blk] = dkv_u32x4{b0.x, b0.y, b1.x, b1.y};
     }
-  }
-  if (t >= S) return;
-  // lane (n, g): dims 16 blk + 4g + u of token t in acc[blk][u]
-  if (is_k) {
-    const int pos = pos0 + t;
-    // (cos, sin) of frequencies 16 blk + 4g .. +3: 32 contiguous bytes of a table row
-    const float* rn = rope + (pos & 15) * 128 + 8 * g;
-    const float* rt = rope + (RT_FIXED + (pos >> 4)) * 128 + 8 * g;
+
+  for (int i = 0; i < tiles; ++i) {
+    const int t = tok0 + i * RW * 16;
+    if (t - n >= S) break;  // the wave's tokens are all past the end (uniform)
+    dkv_f32x4 acc[8];
 #pragma unroll
-    for (int blk = 0; blk < 4; ++blk) {
-      const dkv_f32x4 n0 = *(const dkv_f32x4*)(rn + 32 * blk), n1 = *(const dkv_f32x4*)(rn + 32 * blk + 4);
-      const dkv_f32x4 t0 = *(const dkv_f32x4*)(rt + 32 * blk), t1 = *(const dkv_f32x4*)(rt + 32 * blk + 4);
-      const float nc[4] = {n0.x, n0.z, n1.x, n1.z}, ns[4] = {n0.y, n0.w, n1.y, n1.w};
-      const float tc[4] = {t0.x, t0.z, t1.x, t1.z}, ts[4] = {t0.y, t0.w, t1.y, t1.w};
+    for (int blk = 0; blk < 8; ++blk) acc[blk] = dkv_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        const float cs = tc[u] * nc[u] - ts[u] * ns[u], sn = ts[u] * nc[u] + tc[u] * ns[u];
-        // the projection rounded to the dtype first, then rotated: the reference's two steps
-        // (the up-projection's product in the dtype, then apply_rotary_pos_emb_)
-        const float a = dkv_round_to<DT>(acc[blk][u]), bb = dkv_round_to<DT>(acc[blk + 4][u]);
-        acc[blk][u] = a * cs - bb * sn;
-        acc[blk + 4][u] = bb * cs + a * sn;
+    for (int cc = 0; cc < 4; ++cc)
+#pragma unroll
+      for (int blk = 0; blk < 8; ++blk) acc[blk] = dkv_mfma32<DT>(a[cc][blk], xn[cc], acc[blk]);
+    if (i + 1 < tiles) load_x(t + RW * 16);
+    if (t >= S) continue;
+    // lane (n, g): dims 64h + 16g + 4b + u of token t in acc[4h + b][u]
+    if (is_k) {
+      const float* rt = rope + (RT_FIXED + ((pos0 + t) >> 4)) * 128 + 32 * g;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {  // frequencies 16g + 2e, + 1
+        const dkv_f32x4 tt = *(const dkv_f32x4*)(rt + 4 * e);
+#pragma unroll
+        for (int f = 0; f < 2; ++f) {
+          const int b = e >> 1, u = 2 * (e & 1) + f;
+          const float tc = tt[2 * f], ts = tt[2 * f + 1], nc = rn[e][2 * f], ns = rn[e][2 * f + 1];
+          const float cs = tc * nc - ts * ns, sn = ts * nc + tc * ns;
+          // the projection rounded to the dtype first, then rotated: the reference's two steps
+          // (the up-projection's product in the dtype, then apply_rotary_pos_emb_)
+          const float x = dkv_round_to<DT>(acc[b][u]), y = dkv_round_to<DT>(acc[4 + b][u]);
+          acc[b][u] = x * cs - y * sn;
+          acc[4 + b][u] = y * cs + x * sn;
+        }
       }
     }
-  }
-  uint16_t* orow = o + (long long)row * o_sr + (long long)t * o_st;
+    uint16_t* orow = o + (long long)row * o_sr + (long long)t * o_st + 16 * g;
 #pragma unroll
-  for (int blk = 0; blk < 8; ++blk) {
-    uint32_t w[2];
+    for (int h = 0; h < 2; ++h) {
+      uint32_t w[8];
 #pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const float lo = acc[blk][2 * e], hi = acc[blk][2 * e + 1];
-      if constexpr (DT == DKV_BF16)
-        w[e] = dkv_f32_to_bf16_bits(lo) | (dkv_f32_to_bf16_bits(hi) << 16);
-      else
-        w[e] = dkv_f32_to_f16_bits(lo) | (dkv_f32_to_f16_bits(hi) << 16);
+      for (int e = 0; e < 8; ++e) {
+        const float lo = acc[4 * h + (e >> 1)][2 * (e & 1)];
+        const float hi = acc[4 * h + (e >> 1)][2 * (e & 1) + 1];
+        if constexpr (DT == DKV_BF16)
+          w[e] = dkv_f32_to_bf16_bits(lo) | (dkv_f32_to_bf16_bits(hi) << 16);
+        else
+          w[e] = dkv_f32_to_f16_bits(lo) | (dkv_f32_to_f16_bits(hi) << 16);
+      }
+      uint16_t* od = orow + 64 * h;
+      if (((uintptr_t)od & 15) == 0) {
+        *(dkv_u32x4*)od = dkv_u32x4{w[0], w[1], w[2], w[3]};
+        *(dkv_u32x4*)(od + 8) = dkv_u32x4{w[4], w[5], w[6], w[7]};
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) *(dkv_u32x2*)(od + 4 * e) = dkv_u32x2{w[2 * e], w[2 * e + 1]};
+      }
     }
-    *(dkv_u32x2*)(orow + 16 * blk + 4 * g) = dkv_u32x2{w[0], w[1]};
   }
 }
 
@@ -136,18 +168,23 @@ extern "C" int dkv_recon_kv(void* stream, int dtype, const void* ck, const void*
       (o_sr & 3) || (o_st & 3))
     return DKV_E_UNSUPPORTED;
   if (S > 65535 * 64 || rows > 65535) return DKV_E_UNSUPPORTED;
-  const dim3 grid((unsigned)((S + 63) / 64), (unsigned)rows, 2);
+  // 64-token tiles per workgroup: the grid within the 512 workgroups that run at once (two per
+  // CU). us at 1 / 2 / 4 tiles: 512 tiles in all (B = 1, S = 2048, G = 8) 10.1 / 9.9 / 12.3; 1024
+  // (B = 2) 20.1 / 14.1 / 15.9; 2048 (B = 4) 36.6 / 27.6 / 21.0.
+  const long long t64 = (S + 63) / 64, per = (t64 * rows * 2 + 511) / 512;
+  const int tiles = (int)(per < t64 ? per : t64);
+  const dim3 grid((unsigned)((t64 + tiles - 1) / tiles), (unsigned)rows, 2);
   hipStream_t st = (hipStream_t)stream;
   if (dtype == DKV_BF16)
     hipLaunchKernelGGL(recon_kv_kernel<DKV_BF16>, grid, dim3(RW * 64), 0, st,
                        (const uint16_t*)ck, (const uint16_t*)cv, c_sr, c_st,
                        (const uint16_t*)k_basis, (const uint16_t*)v_basis, b_sg, b_sr,
-                       (uint16_t*)k_out, (uint16_t*)v_out, o_sr, o_st, G, S, R, pos0, rope);
+                       (uint16_t*)k_out, (uint16_t*)v_out, o_sr, o_st, G, S, R, pos0, rope, tiles);
   else
     hipLaunchKernelGGL(recon_kv_kernel<DKV_F16>, grid, dim3(RW * 64), 0, st,
                        (const uint16_t*)ck, (const uint16_t*)cv, c_sr, c_st,
                        (const uint16_t*)k_basis, (const uint16_t*)v_basis, b_sg, b_sr,
-                       (uint16_t*)k_out, (uint16_t*)v_out, o_sr, o_st, G, S, R, pos0, rope);
+                       (uint16_t*)k_out, (uint16_t*)v_out, o_sr, o_st, G, S, R, pos0, rope, tiles);
   DKV_HIP_CHECK_LAUNCH();
   return DKV_OK;
 }
