@@ -59,12 +59,18 @@ _SIGNATURES = {
     "dkv_dense_choose_split": (_i, [_i, _i, _i]),
     "dkv_recon_kv": (_i, [_vp, _i, _vp, _vp, _ll, _ll, _vp, _vp, _ll, _ll, _vp, _vp, _ll, _ll,
                           _i, _i, _i, _i, _i, _vp, _i]),
+    "dkv_recon_kv_bt": (_i, [_vp, _i, _vp, _vp, _ll, _ll, _vp, _vp, _ll, _ll, _vp, _vp, _ll, _ll,
+                          _i, _i, _i, _i, _i, _vp, _i]),
     "dkv_dense_append": (_i, [_vp, _i, _vp, _ll, _vp, _vp, _ll, _i, _i, _i, _i, _i, _f]),
     "dkv_decode_dense": (_i, [_vp, _i, _vp, _ll, _ll, _vp, _vp, _ll, _i, _vp, _ll, _vp, _ll, _ll,
                               _i, _i, _i, _i, _i, _i]),
     "dkv_rope_table_floats": (_ll, [_i]),
     "dkv_rope_table": (_i, [_vp, _vp, _i, _i, _f]),
     "dkv_decode_splitk": (_i, [_vp, _i, _i, _vp, _ll, _ll, _vp, _ll, _ll, _vp, _ll, _ll,
+                               _vp, _ll, _vp, _ll, _vp, _vp, _ll, _ll, _vp, _vp, _ll, _ll,
+                               _vp, _i, _vp, _ll, _vp, _ll, _ll, _i,
+                               _i, _i, _i, _i, _i, _i, _i, _i]),
+    "dkv_decode_splitk_bt": (_i, [_vp, _i, _i, _vp, _ll, _ll, _vp, _ll, _ll, _vp, _ll, _ll,
                                _vp, _ll, _vp, _ll, _vp, _vp, _ll, _ll, _vp, _vp, _ll, _ll,
                                _vp, _i, _vp, _ll, _vp, _ll, _ll, _i,
                                _i, _i, _i, _i, _i, _i, _i, _i]),

@@ -32,7 +32,7 @@ template <int DT>
 __global__ __launch_bounds__(RW * 64, 2) void recon_kv_kernel(
     const uint16_t* __restrict__ ck, const uint16_t* __restrict__ cv, long long c_sr,
     long long c_st, const uint16_t* __restrict__ kb, const uint16_t* __restrict__ vb,
-    long long b_sg, long long b_sr, uint16_t* __restrict__ ko, uint16_t* __restrict__ vo,
+    long long b_sg, long long b_sr, int bt, uint16_t* __restrict__ ko, uint16_t* __restrict__ vo,
     long long o_sr, long long o_st, int G, int S, int R, int pos0, const float* __restrict__ rope,
     int tiles) {
   __shared__ __attribute__((aligned(16))) uint16_t sB[DH * DH];  // [rank][dim]
@@ -65,31 +65,43 @@ __global__ __launch_bounds__(RW * 64, 2) void recon_kv_kernel(
 #pragma unroll
     for (int e = 0; e < 8; ++e) rn[e] = *(const dkv_f32x4*)(rp + 4 * e);
   }
-  // the basis, 16-byte pieces (rank r, dims d8 .. d8 + 7), ranks past R as zeros
-  for (int pc = tid; pc < DH * DH / 8; pc += RW * 64) {
-    const int r = pc >> 4, d8 = (pc & 15) * 8;
-    *(dkv_u32x4*)(sB + r * DH + d8) =
-        r < R ? *(const dkv_u32x4*)(bg + (long long)r * b_sr + d8) : dkv_u32x4{0u, 0u, 0u, 0u};
-  }
-  __syncthreads();
   // A operands: block blk = 4h + b, row i holds dim 64h + 16 (i / 4) + 4b + i % 4; lane (n, g)
   // receives ranks 32 cc + 8g .. +3 and +4 .. +7 of its row's dim
   typedef __attribute__((address_space(3))) dkv_i16x4 lds_i16x4;
   dkv_u32x4 a[4][8];
+  if (bt) {
+    // a transposed basis ([dim][rank]) holds them as they are taken
 #pragma unroll
-  for (int cc = 0; cc < 4; ++cc)
+    for (int cc = 0; cc < 4; ++cc)
 #pragma unroll
-    for (int blk = 0; blk < 8; ++blk) {
-      const uint16_t* src = sB + (32 * cc + 8 * g + (n >> 2)) * DH + 64 * (blk >> 2) +
-                            16 * (n & 3) + 4 * (blk & 3);
-      const dkv_u32x2 b0 = __builtin_bit_cast(
-          dkv_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                         (lds_i16x4*)(__attribute__((address_space(3))) uint16_t*)src));
-      const dkv_u32x2 b1 = __builtin_bit_cast(
-          dkv_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                         (lds_i16x4*)(__attribute__((address_space(3))) uint16_t*)(src + 4 * DH)));
-      a[cc][blk] = dkv_u32x4{b0.x, b0.y, b1.x, b1.y};
+      for (int blk = 0; blk < 8; ++blk) {
+        const int r0 = 32 * cc + 8 * g, d = 64 * (blk >> 2) + 16 * (n >> 2) + 4 * (blk & 3) + (n & 3);
+        a[cc][blk] = r0 < R ? *(const dkv_u32x4*)(bg + (long long)d * b_sr + r0)
+                            : dkv_u32x4{0u, 0u, 0u, 0u};
+      }
+  } else {
+    // the basis, 16-byte pieces (rank r, dims d8 .. d8 + 7), ranks past R as zeros
+    for (int pc = tid; pc < DH * DH / 8; pc += RW * 64) {
+      const int r = pc >> 4, d8 = (pc & 15) * 8;
+      *(dkv_u32x4*)(sB + r * DH + d8) =
+          r < R ? *(const dkv_u32x4*)(bg + (long long)r * b_sr + d8) : dkv_u32x4{0u, 0u, 0u, 0u};
     }
+    __syncthreads();
+#pragma unroll
+    for (int cc = 0; cc < 4; ++cc)
+#pragma unroll
+      for (int blk = 0; blk < 8; ++blk) {
+        const uint16_t* src = sB + (32 * cc + 8 * g + (n >> 2)) * DH + 64 * (blk >> 2) +
+                              16 * (n & 3) + 4 * (blk & 3);
+        const dkv_u32x2 b0 = __builtin_bit_cast(
+            dkv_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                           (lds_i16x4*)(__attribute__((address_space(3))) uint16_t*)src));
+        const dkv_u32x2 b1 = __builtin_bit_cast(
+            dkv_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                           (lds_i16x4*)(__attribute__((address_space(3))) uint16_t*)(src + 4 * DH)));
+        a[cc][blk] = dkv_u32x4{b0.x, b0.y, b1.x, b1.y};
+      }
+  }
 
   for (int i = 0; i < tiles; ++i) {
     const int t = tok0 + i * RW * 16;
@@ -149,7 +161,7 @@ __global__ __launch_bounds__(RW * 64, 2) void recon_kv_kernel(
 
 }  // namespace
 
-extern "C" int dkv_recon_kv(void* stream, int dtype, const void* ck, const void* cv,
+static int recon_kv(int bt, void* stream, int dtype, const void* ck, const void* cv,
                             long long c_sr, long long c_st, const void* k_basis,
                             const void* v_basis, long long b_sg, long long b_sr, void* k_out,
                             void* v_out, long long o_sr, long long o_st, int rows, int G, int S,
@@ -178,13 +190,31 @@ extern "C" int dkv_recon_kv(void* stream, int dtype, const void* ck, const void*
   if (dtype == DKV_BF16)
     hipLaunchKernelGGL(recon_kv_kernel<DKV_BF16>, grid, dim3(RW * 64), 0, st,
                        (const uint16_t*)ck, (const uint16_t*)cv, c_sr, c_st,
-                       (const uint16_t*)k_basis, (const uint16_t*)v_basis, b_sg, b_sr,
+                       (const uint16_t*)k_basis, (const uint16_t*)v_basis, b_sg, b_sr, bt,
                        (uint16_t*)k_out, (uint16_t*)v_out, o_sr, o_st, G, S, R, pos0, rope, tiles);
   else
     hipLaunchKernelGGL(recon_kv_kernel<DKV_F16>, grid, dim3(RW * 64), 0, st,
                        (const uint16_t*)ck, (const uint16_t*)cv, c_sr, c_st,
-                       (const uint16_t*)k_basis, (const uint16_t*)v_basis, b_sg, b_sr,
+                       (const uint16_t*)k_basis, (const uint16_t*)v_basis, b_sg, b_sr, bt,
                        (uint16_t*)k_out, (uint16_t*)v_out, o_sr, o_st, G, S, R, pos0, rope, tiles);
   DKV_HIP_CHECK_LAUNCH();
   return DKV_OK;
+}
+
+extern "C" int dkv_recon_kv(void* stream, int dtype, const void* ck, const void* cv,
+                            long long c_sr, long long c_st, const void* k_basis,
+                            const void* v_basis, long long b_sg, long long b_sr, void* k_out,
+                            void* v_out, long long o_sr, long long o_st, int rows, int G, int S,
+                            int R, int pos0, const float* rope, int rope_tiles) {
+  return recon_kv(0, stream, dtype, ck, cv, c_sr, c_st, k_basis, v_basis, b_sg, b_sr, k_out, v_out,
+                  o_sr, o_st, rows, G, S, R, pos0, rope, rope_tiles);
+}
+
+extern "C" int dkv_recon_kv_bt(void* stream, int dtype, const void* ck, const void* cv,
+                               long long c_sr, long long c_st, const void* k_basis,
+                               const void* v_basis, long long b_sg, long long b_sd, void* k_out,
+                               void* v_out, long long o_sr, long long o_st, int rows, int G, int S,
+                               int R, int pos0, const float* rope, int rope_tiles) {
+  return recon_kv(1, stream, dtype, ck, cv, c_sr, c_st, k_basis, v_basis, b_sg, b_sd, k_out, v_out,
+                  o_sr, o_st, rows, G, S, R, pos0, rope, rope_tiles);
 }

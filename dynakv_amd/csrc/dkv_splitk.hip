@@ -68,10 +68,13 @@ constexpr int DPP_ROW_SHL8 = 0x108;      // DPP row_shl:8: lane i of a 16-lane r
 struct SplitParams {
   const uint16_t* q;
   long long q_sb, q_sh;
+  // bases: element (unit u, rank r, dim d) at u * unit + r * sr + d (bt = 0, sr the rank
+  // stride), or at u * unit + d * sr + r (bt = 1: a transposed basis, sr the dim stride)
   const uint16_t* k_basis;
   long long k_unit, k_sr;
   const uint16_t* v_basis;
   long long v_unit, v_sr;
+  int bt;
   const uint16_t* k_flat;
   const uint16_t* v_flat;
   int k_ld, v_ld;
@@ -389,10 +392,19 @@ __device__ __forceinline__ void merge_records_w(const SplitParams& p, const floa
 }
 
 // This thread's share of the unit's V basis (16-byte piece ch: rank ch / 16, dims
-// 8 * (ch % 16)); unconditional loads (pieces of ranks past R read rank R-1's and are zeroed
-// when staged), so that none waits for another.
+// 8 * (ch % 16); of a transposed basis dim ch / 16, ranks 8 * (ch % 16)); unconditional loads
+// (pieces of ranks past R read real ones and are zeroed when staged), so that none waits for
+// another.
 __device__ __forceinline__ void load_vbasis(const SplitParams& p, int kvh, dkv_u32x4 (&vbr)[VB_CHUNKS]) {
   const uint16_t* vb = p.v_basis + (long long)kvh * p.v_unit;
+  if (p.bt) {
+#pragma unroll
+    for (int k = 0; k < VB_CHUNKS; ++k) {
+      const int ch = (int)threadIdx.x + k * NTHREADS;
+      vbr[k] = *(const dkv_u32x4*)(vb + (long long)(ch >> 4) * p.v_sr + min(8 * (ch & 15), p.R - 8));
+    }
+    return;
+  }
 #pragma unroll
   for (int k = 0; k < VB_CHUNKS; ++k) {
     const int ch = min((int)threadIdx.x + k * NTHREADS, p.R * (DH / 8) - 1);
@@ -441,12 +453,17 @@ __device__ __forceinline__ void project_store(const SplitParams& p, int unit, ui
   const int b = unit / p.Hkv, kvh = unit % p.Hkv;
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int n = lane & 15, g = lane >> 4;
-  uint16_t* sVB = reinterpret_cast<uint16_t*>(scratch);          // [128][DH], rank-major
+  // [128][DH], rank-major; a transposed basis [dim][128], 16-byte chunk c of dim d at position
+  // c ^ (d % 16)
+  uint16_t* sVB = reinterpret_cast<uint16_t*>(scratch);
   const float* sA = reinterpret_cast<const float*>(scratch + DH * DH * 2);
 #pragma unroll
-  for (int k = 0; k < VB_CHUNKS; ++k)
-    *(dkv_u32x4*)(sVB + (tid + k * NTHREADS) * 8) =
-        tid + k * NTHREADS < p.R * (DH / 8) ? vbr[k] : dkv_u32x4{0u, 0u, 0u, 0u};
+  for (int k = 0; k < VB_CHUNKS; ++k) {
+    const int ch = tid + k * NTHREADS;
+    const int at = p.bt ? (ch & ~15) | ((ch & 15) ^ ((ch >> 4) & 15)) : ch;
+    const bool live = p.bt ? 8 * (ch & 15) < p.R : ch < p.R * (DH / 8);
+    *(dkv_u32x4*)(sVB + at * 8) = live ? vbr[k] : dkv_u32x4{0u, 0u, 0u, 0u};
+  }
   __syncthreads();
   // out[hs][d] = sum_r a[hs][r] VB[r][d] on 16x16x32 MFMA: wave w takes dims 16w..16w+15.
   // A: the merged coefficients of head slot n, ranks 32c + 8g..+7, as hi + lo parts in the
@@ -475,15 +492,20 @@ __device__ __forceinline__ void project_store(const SplitParams& p, int unit, ui
         split_f16x2(xs[2 * e], xs[2 * e + 1], p.minus_one, hi[e], lo[e]);
       }
     }
-    const uint16_t* src = sVB + (k0 + (n >> 2)) * DH + d0 + 4 * (n & 3);
-    typedef __attribute__((address_space(3))) dkv_i16x4 lds_i16x4;
-    const dkv_u32x2 b0 = __builtin_bit_cast(
-        dkv_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                       (lds_i16x4*)(__attribute__((address_space(3))) uint16_t*)src));
-    const dkv_u32x2 b1 = __builtin_bit_cast(
-        dkv_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
-                       (lds_i16x4*)(__attribute__((address_space(3))) uint16_t*)(src + 4 * DH)));
-    const dkv_u32x4 bop = dkv_u32x4{b0.x, b0.y, b1.x, b1.y};
+    dkv_u32x4 bop;
+    if (p.bt) {  // ranks k0 .. k0 + 7 of dim d0 + n
+      bop = *(const dkv_u32x4*)(sVB + (d0 + n) * DH + 8 * ((4 * c + g) ^ n));
+    } else {
+      const uint16_t* src = sVB + (k0 + (n >> 2)) * DH + d0 + 4 * (n & 3);
+      typedef __attribute__((address_space(3))) dkv_i16x4 lds_i16x4;
+      const dkv_u32x2 b0 = __builtin_bit_cast(
+          dkv_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                         (lds_i16x4*)(__attribute__((address_space(3))) uint16_t*)src));
+      const dkv_u32x2 b1 = __builtin_bit_cast(
+          dkv_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                         (lds_i16x4*)(__attribute__((address_space(3))) uint16_t*)(src + 4 * DH)));
+      bop = dkv_u32x4{b0.x, b0.y, b1.x, b1.y};
+    }
     o = mfma_k<DT>(dkv_u32x4{lo[0], lo[1], lo[2], lo[3]}, bop, o);
     o = mfma_k<DT>(dkv_u32x4{hi[0], hi[1], hi[2], hi[3]}, bop, o);
   }
@@ -616,6 +638,18 @@ __global__ __launch_bounds__(NTHREADS, 1) void splitk_kernel(SplitParams p) {
     // the others to the staging copy.
     const uint16_t* kb = p.k_basis + (long long)kvh * p.k_unit;
     const int j = tid & 127, dq = tid >> 7;  // 4 groups of 8-dim slices
+    static_assert(NREG_PP == 4, "a transposed basis is staged whole");
+    if (p.bt) {
+      // already [dim][rank]: 16-byte pieces (dim ch / 16, ranks 8 * (ch % 16); R is a multiple
+      // of 8)
+#pragma unroll
+      for (int it = 0; it < 4; ++it) {
+        const int ch = tid + it * NTHREADS, d = ch >> 4, r8 = 8 * (ch & 15);
+        dkv_u32x4 v = *(const dkv_u32x4*)(kb + (long long)d * p.k_sr + min(r8, R - 8));
+        if (r8 >= R) v = dkv_u32x4{0u, 0u, 0u, 0u};
+        *(dkv_u32x4*)(sBK + d * BK_LD + r8) = v;
+      }
+    } else
 #pragma unroll
     for (int it = 0; it < 4; ++it) {
       const int d8 = (dq + 4 * it) * 8;
@@ -1262,7 +1296,8 @@ __global__ __launch_bounds__(256) void merge_kernel(SplitParams p) {
     const uint16_t* vb = p.v_basis + (long long)kvh * p.v_unit;
     float o = 0.f;
 #pragma unroll 8
-    for (int j = half; j < R; j += 2) o = fmaf(sA[j], elt_to_f32<DT>(vb[(long long)j * p.v_sr + d]), o);
+    for (int j = half; j < R; j += 2)
+      o = fmaf(sA[j], elt_to_f32<DT>(vb[p.bt ? (long long)d * p.v_sr + j : (long long)j * p.v_sr + d]), o);
     __syncthreads();
     sO[half][d] = o;
     __syncthreads();
@@ -1518,7 +1553,7 @@ extern "C" int dkv_profile_end(double* split_ms, double* merge_ms, int* calls) {
 
 // Argument checks shared by both entry points; 0 when the call is valid, or a status.
 // On success *n_floats receives the workspace size the call needs (0 when nothing is launched).
-static int splitk_check(int route, int dtype, const void* q, const void* k_basis,
+static int splitk_check(int route, int dtype, int bt, const void* q, const void* k_basis,
                         long long k_unit_stride, long long k_basis_sr, const void* v_basis,
                         long long v_unit_stride, long long v_basis_sr, const void* k_flat,
                         long long k_ld, const void* v_flat, long long v_ld, const int* lens_k,
@@ -1544,6 +1579,7 @@ static int splitk_check(int route, int dtype, const void* q, const void* k_basis
   // 16-byte aligned V basis rows for the vector loads of the fused merge
   if (((uintptr_t)v_basis & 15) || (v_basis_sr & 7) || (v_unit_stride & 7))
     return DKV_E_UNSUPPORTED;
+  if (bt && R % 8 != 0) return DKV_E_UNSUPPORTED;  // 16-byte pieces along the rank
   if (k_ld <= 0 || v_ld <= 0) return DKV_E_ARG;
   // buffer offsets are 32-bit byte offsets from the start of a row
   const long long rows = (long long)B * G;
@@ -1564,7 +1600,7 @@ static int splitk_check(int route, int dtype, const void* q, const void* k_basis
 
 // Launch the split kernel (and the merge kernel when one is needed) of a call that passed
 // splitk_check, with `workspace` holding at least the floats splitk_check asked for.
-static int splitk_launch(void* stream, int route, int dtype, const void* q, long long q_sb,
+static int splitk_launch(void* stream, int route, int dtype, int bt, const void* q, long long q_sb,
                          long long q_sh, const void* k_basis, long long k_unit_stride,
                          long long k_basis_sr, const void* v_basis, long long v_unit_stride,
                          long long v_basis_sr, const void* k_flat, long long k_ld,
@@ -1587,6 +1623,7 @@ static int splitk_launch(void* stream, int route, int dtype, const void* q, long
   p.v_basis = (const uint16_t*)v_basis;
   p.v_unit = v_unit_stride;
   p.v_sr = v_basis_sr;
+  p.bt = bt;
   p.k_flat = (const uint16_t*)k_flat;
   p.v_flat = (const uint16_t*)v_flat;
   p.k_ld = (int)k_ld;
@@ -1639,7 +1676,7 @@ static int splitk_launch(void* stream, int route, int dtype, const void* q, long
   return DKV_OK;
 }
 
-extern "C" int dkv_decode_splitk(void* stream, int route, int dtype, const void* q, long long q_sb,
+static int decode_splitk(int bt, void* stream, int route, int dtype, const void* q, long long q_sb,
                                  long long q_sh, const void* k_basis, long long k_unit_stride,
                                  long long k_basis_sr, const void* v_basis,
                                  long long v_unit_stride, long long v_basis_sr,
@@ -1652,17 +1689,55 @@ extern "C" int dkv_decode_splitk(void* stream, int route, int dtype, const void*
                                  long long out_sh, int out_dtype, int B, int Hq, int Hkv, int G,
                                  int S, int R, int Dh, int split_len) {
   long long need = 0;
-  const int rc = splitk_check(route, dtype, q, k_basis, k_unit_stride, k_basis_sr, v_basis,
+  const int rc = splitk_check(route, dtype, bt, q, k_basis, k_unit_stride, k_basis_sr, v_basis,
                               v_unit_stride, v_basis_sr, k_flat, k_ld, v_flat, v_ld, lens_k,
                               offs_k, tk_ss, lens_v, offs_v, tv_ss, rope, rope_tiles, out,
                               out_dtype, B, Hq, Hkv, G, S, R, Dh, &split_len, &need);
   if (rc != DKV_OK || need == 0) return rc;
   if (!workspace) return DKV_E_ARG;
   if (workspace_floats < need) return DKV_E_WORKSPACE;
-  return splitk_launch(stream, route, dtype, q, q_sb, q_sh, k_basis, k_unit_stride, k_basis_sr,
+  return splitk_launch(stream, route, dtype, bt, q, q_sb, q_sh, k_basis, k_unit_stride, k_basis_sr,
                        v_basis, v_unit_stride, v_basis_sr, k_flat, k_ld, v_flat, v_ld, lens_k,
                        offs_k, tk_sb, tk_ss, lens_v, offs_v, tv_sb, tv_ss, rope, workspace, out,
                        out_sb, out_sh, out_dtype, B, Hq, Hkv, G, S, R, Dh, split_len);
+}
+
+extern "C" int dkv_decode_splitk(void* stream, int route, int dtype, const void* q, long long q_sb,
+                                 long long q_sh, const void* k_basis, long long k_unit_stride,
+                                 long long k_basis_sr, const void* v_basis,
+                                 long long v_unit_stride, long long v_basis_sr,
+                                 const void* k_flat, long long k_ld, const void* v_flat,
+                                 long long v_ld, const int* lens_k, const int* offs_k,
+                                 long long tk_sb, long long tk_ss, const int* lens_v,
+                                 const int* offs_v, long long tv_sb, long long tv_ss,
+                                 const float* rope, int rope_tiles, float* workspace,
+                                 long long workspace_floats, void* out, long long out_sb,
+                                 long long out_sh, int out_dtype, int B, int Hq, int Hkv, int G,
+                                 int S, int R, int Dh, int split_len) {
+  return decode_splitk(0, stream, route, dtype, q, q_sb, q_sh, k_basis, k_unit_stride,
+                       k_basis_sr, v_basis, v_unit_stride, v_basis_sr, k_flat, k_ld, v_flat,
+                       v_ld, lens_k, offs_k, tk_sb, tk_ss, lens_v, offs_v, tv_sb, tv_ss, rope,
+                       rope_tiles, workspace, workspace_floats, out, out_sb, out_sh, out_dtype,
+                       B, Hq, Hkv, G, S, R, Dh, split_len);
+}
+
+extern "C" int dkv_decode_splitk_bt(void* stream, int route, int dtype, const void* q, long long q_sb,
+                                 long long q_sh, const void* k_basis, long long k_unit_stride,
+                                 long long k_basis_sd, const void* v_basis,
+                                 long long v_unit_stride, long long v_basis_sd,
+                                 const void* k_flat, long long k_ld, const void* v_flat,
+                                 long long v_ld, const int* lens_k, const int* offs_k,
+                                 long long tk_sb, long long tk_ss, const int* lens_v,
+                                 const int* offs_v, long long tv_sb, long long tv_ss,
+                                 const float* rope, int rope_tiles, float* workspace,
+                                 long long workspace_floats, void* out, long long out_sb,
+                                 long long out_sh, int out_dtype, int B, int Hq, int Hkv, int G,
+                                 int S, int R, int Dh, int split_len) {
+  return decode_splitk(1, stream, route, dtype, q, q_sb, q_sh, k_basis, k_unit_stride,
+                       k_basis_sd, v_basis, v_unit_stride, v_basis_sd, k_flat, k_ld, v_flat,
+                       v_ld, lens_k, offs_k, tk_sb, tk_ss, lens_v, offs_v, tv_sb, tv_ss, rope,
+                       rope_tiles, workspace, workspace_floats, out, out_sb, out_sh, out_dtype,
+                       B, Hq, Hkv, G, S, R, Dh, split_len);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -1722,7 +1797,7 @@ extern "C" int dkv_decode_splitk_noalloc(
     const float* rope, int rope_tiles, void* out, long long out_sb, long long out_sh,
     int out_dtype, int B, int Hq, int Hkv, int G, int S, int R, int Dh, int split_len) {
   long long need = 0;
-  int rc = splitk_check(route, dtype, q, k_basis, k_unit_stride, k_basis_sr, v_basis,
+  int rc = splitk_check(route, dtype, 0, q, k_basis, k_unit_stride, k_basis_sr, v_basis,
                         v_unit_stride, v_basis_sr, k_flat, k_ld, v_flat, v_ld, lens_k, offs_k,
                         tk_ss, lens_v, offs_v, tv_ss, rope, rope_tiles, out, out_dtype, B, Hq,
                         Hkv, G, S, R, Dh, &split_len, &need);
@@ -1731,7 +1806,7 @@ extern "C" int dkv_decode_splitk_noalloc(
   float* ws = nullptr;
   rc = noalloc_scratch((hipStream_t)stream, &ws);
   if (rc != DKV_OK) return rc;
-  return splitk_launch(stream, route, dtype, q, q_sb, q_sh, k_basis, k_unit_stride, k_basis_sr,
+  return splitk_launch(stream, route, dtype, 0, q, q_sb, q_sh, k_basis, k_unit_stride, k_basis_sr,
                        v_basis, v_unit_stride, v_basis_sr, k_flat, k_ld, v_flat, v_ld, lens_k,
                        offs_k, tk_sb, tk_ss, lens_v, offs_v, tv_sb, tv_ss, rope, ws, out, out_sb,
                        out_sh, out_dtype, B, Hq, Hkv, G, S, R, Dh, split_len);

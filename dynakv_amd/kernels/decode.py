@@ -72,6 +72,7 @@ class UnitLayout:
     v_unit: int
     k_basis: torch.Tensor
     v_basis: torch.Tensor
+    transposed: bool = False  # the bases are contiguous along the rank, not the dim
 
 
 # Largest row stride (elements) of a flat buffer the split kernel addresses: each workgroup's
@@ -90,6 +91,13 @@ def flat_ok(t: torch.Tensor) -> bool:
 def _basis_ok(t: torch.Tensor) -> bool:
     return (t.dim() == 3 and t.stride(2) == 1 and t.stride(1) % 8 == 0
             and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0)
+
+
+def _basis_t_ok(t: torch.Tensor) -> bool:
+    """A basis held transposed (unit rank stride, e.g. ``U.transpose(1, 2)``): the kernels read it
+    in place. A rank-major copy of both bases costs two launches, about 10 us on MI355X."""
+    return (t.dim() == 3 and t.stride(1) == 1 and t.stride(2) % 8 == 0 and t.stride(0) % 8 == 0
+            and t.shape[1] % 8 == 0 and t.data_ptr() % 16 == 0)
 
 
 def splitk_layout(q3: torch.Tensor, k_up: torch.Tensor, v_up: torch.Tensor,
@@ -120,11 +128,14 @@ def splitk_layout(q3: torch.Tensor, k_up: torch.Tensor, v_up: torch.Tensor,
     if hq // n_kv > SPLITK_MAX_HPG:
         return None
     kb, vb = k_up, v_up
-    if not _basis_ok(kb):
+    k_ok, v_ok = _basis_ok(kb), _basis_ok(vb)
+    if not (k_ok and v_ok) and _basis_t_ok(kb) and _basis_t_ok(vb):
+        return UnitLayout(n_kv, kb.stride(0), vb.stride(0), kb, vb, True)
+    if not k_ok:
         kb = kb.contiguous()
         if n_kv == 1 and hb == hq:
             kb = kb[:1]
-    if not _basis_ok(vb):
+    if not v_ok:
         vb = vb.contiguous()
         if n_kv == 1 and hb == hq:
             vb = vb[:1]
@@ -165,11 +176,13 @@ def splitk_attention(q3: torch.Tensor, k_flat: torch.Tensor, v_flat: torch.Tenso
     nfl = lib.dkv_splitk_workspace_floats(B, hq, layout.n_kv, S, R, split_len)
     ws = workspace(q3.device, st, int(nfl))
     rope, rope_tiles = rope_table(q3.device, st, theta, S)
-    rc = lib.dkv_decode_splitk(
+    # stride of the bases' non-unit axis: the rank, or the dim of transposed bases
+    fn, ax = (lib.dkv_decode_splitk_bt, 2) if layout.transposed else (lib.dkv_decode_splitk, 1)
+    rc = fn(
         st, route, _lib.dtype_code(q3.dtype),
         q3.data_ptr(), q3.stride(0), q3.stride(1),
-        layout.k_basis.data_ptr(), layout.k_unit, layout.k_basis.stride(1),
-        layout.v_basis.data_ptr(), layout.v_unit, layout.v_basis.stride(1),
+        layout.k_basis.data_ptr(), layout.k_unit, layout.k_basis.stride(ax),
+        layout.v_basis.data_ptr(), layout.v_unit, layout.v_basis.stride(ax),
         k_flat.data_ptr(), k_flat.stride(0), v_flat.data_ptr(), v_flat.stride(0),
         lens_k.data_ptr(), offs_k.data_ptr(), lens_k.stride(0), lens_k.stride(1),
         lens_v.data_ptr(), offs_v.data_ptr(), lens_v.stride(0), lens_v.stride(1),

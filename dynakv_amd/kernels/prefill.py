@@ -19,7 +19,7 @@ import math
 import torch
 
 from .. import _lib
-from .decode import rope_table
+from .decode import _basis_t_ok, rope_table
 
 
 def _extent(t: torch.Tensor) -> int:
@@ -139,7 +139,10 @@ def recon_kv(ck: torch.Tensor, cv: torch.Tensor, k_basis: torch.Tensor, v_basis:
             or not (cv.dtype == k_basis.dtype == v_basis.dtype == dt)
             or v_basis.shape != k_basis.shape or rows != batch * G):
         return None
-    kb, vb = k_basis.contiguous(), v_basis.contiguous()
+    bt = (not (k_basis.is_contiguous() and v_basis.is_contiguous())
+          and _basis_t_ok(k_basis) and _basis_t_ok(v_basis)
+          and k_basis.stride() == v_basis.stride())
+    kb, vb = (k_basis, v_basis) if bt else (k_basis.contiguous(), v_basis.contiguous())
     if (ck.stride(0) % 8 or ck.stride(1) % 8 or ck.data_ptr() % 16 or cv.data_ptr() % 16
             or kb.data_ptr() % 16 or vb.data_ptr() % 16):
         return None
@@ -148,11 +151,11 @@ def recon_kv(ck: torch.Tensor, cv: torch.Tensor, k_basis: torch.Tensor, v_basis:
     lib = _lib.load()
     st = _lib.stream_of(ck)
     rope, tiles = rope_table(ck.device, st, theta, int(pos0) + S)
-    _lib.check(lib.dkv_recon_kv(st, _lib.dtype_code(dt), ck.data_ptr(),
-                                cv.data_ptr(), ck.stride(0), ck.stride(1), kb.data_ptr(),
-                                vb.data_ptr(), kb.stride(0), kb.stride(1), k.data_ptr(),
-                                v.data_ptr(), S * Dh, Dh, rows, G, S, R, int(pos0),
-                                rope.data_ptr(), tiles), "dkv_recon_kv")
+    fn, ax = (lib.dkv_recon_kv_bt, 2) if bt else (lib.dkv_recon_kv, 1)
+    _lib.check(fn(st, _lib.dtype_code(dt), ck.data_ptr(), cv.data_ptr(), ck.stride(0),
+                  ck.stride(1), kb.data_ptr(), vb.data_ptr(), kb.stride(0), kb.stride(ax),
+                  k.data_ptr(), v.data_ptr(), S * Dh, Dh, rows, G, S, R, int(pos0),
+                  rope.data_ptr(), tiles), "dkv_recon_kv")
     return k, v
 
 

@@ -290,6 +290,23 @@ int dkv_decode_splitk(void* stream, int route, int dtype,
                       int B, int Hq, int Hkv, int G, int S, int R, int Dh, int split_len);
 
 /*
+ * dkv_decode_splitk for transposed bases (U rather than U^T in memory): element (rank r, dim d) of
+ * KV head k's basis at  base + k * unit_stride + d * basis_sd + r,  for both K and V. R a multiple
+ * of 8; the same results bit for bit as from a rank-major copy of the bases.
+ */
+int dkv_decode_splitk_bt(void* stream, int route, int dtype,
+                         const void* q, long long q_sb, long long q_sh,
+                         const void* k_basis, long long k_unit_stride, long long k_basis_sd,
+                         const void* v_basis, long long v_unit_stride, long long v_basis_sd,
+                         const void* k_flat, long long k_ld, const void* v_flat, long long v_ld,
+                         const int* lens_k, const int* offs_k, long long tk_sb, long long tk_ss,
+                         const int* lens_v, const int* offs_v, long long tv_sb, long long tv_ss,
+                         const float* rope, int rope_tiles,
+                         float* workspace, long long workspace_floats,
+                         void* out, long long out_sb, long long out_sh, int out_dtype,
+                         int B, int Hq, int Hkv, int G, int S, int R, int Dh, int split_len);
+
+/*
  * Dense GQA decode attention over an uncompressed cache: the baseline of the end-to-end
  * comparison (the reference's uncompressed model, scripts/benchmark_throughput.py:17-77, reads
  * every cached token's rotated key and value at full width; it has no kernel of its own for it).
@@ -444,6 +461,15 @@ int dkv_recon_kv(void* stream, int dtype, const void* ck, const void* cv, long l
                  long long c_st, const void* k_basis, const void* v_basis, long long b_sg,
                  long long b_sr, void* k_out, void* v_out, long long o_sr, long long o_st,
                  int rows, int G, int S, int R, int pos0, const float* rope, int rope_tiles);
+
+/*
+ * dkv_recon_kv for transposed bases: element (rank r, dim d) of group g's basis at
+ * base + g * b_sg + d * b_sd + r, for both K and V; the same results bit for bit.
+ */
+int dkv_recon_kv_bt(void* stream, int dtype, const void* ck, const void* cv, long long c_sr,
+                    long long c_st, const void* k_basis, const void* v_basis, long long b_sg,
+                    long long b_sd, void* k_out, void* v_out, long long o_sr, long long o_st,
+                    int rows, int G, int S, int R, int pos0, const float* rope, int rope_tiles);
 int dkv_rope_apply(void* stream, int dtype, void* x, long long x_sb, long long x_sh,
                    long long x_ss, const void* cos, const void* sin, long long cs_sb,
                    long long cs_ss, int B, int H, int S);
