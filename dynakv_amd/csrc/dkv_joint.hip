@@ -13,14 +13,15 @@
 //   tokens ordered by their count of 32-rank chunks (a counting sort) into a workspace.
 // joint_scores_sorted_kernel -- workgroup = (512 sorted tokens of a window, basis head h, batch
 //   row b), or with the heads in pairs (256 tokens, heads 2h and 2h+1, b) so that each
-//   coefficient load serves both heads' products; the longest ranges are dispatched first. The
+//   coefficient load serves both heads' products, or for few tokens 128 of one head; the
+//   longest ranges are dispatched first. The
 //   workgroup's tokens form blocks of 16; wave w takes blocks w and NBLK-1-w (one short, one
 //   long). K^T = B_h^T . X^T accumulates on 16x16x32 MFMA over the rank chunks of
 //   32, each block only up to its own longest token's chunk. Each basis chunk ([128 dims][32
 //   ranks], 8 KB contiguous in HBM) is loaded once per workgroup into LDS (four buffers per
 //   head, one barrier per two chunks) and every A operand read from it serves the wave's active
 //   blocks; the coefficients go straight into B operand registers (lane = one token x 8 ranks,
-//   elements past the token's count zeroed), two chunks ahead, each serving every head of the
+//   elements past the token's count zeroed), two or four chunks ahead, each serving every head of the
 //   workgroup. Then per block: the lane's token rotated by R(p) = R(16T) R(n) (p = 16T + n, its
 //   position; composed from LDS tables) in fp32, K' split into bf16 hi + lo, scores on MFMA
 //   against the unrotated query (hi and lo parts in separate operand columns, formed once per
@@ -152,18 +153,17 @@ __global__ __launch_bounds__(JSORT_THREADS) void joint_sort_kernel(JSortParams p
   __syncthreads();  // sW cleared
 #pragma unroll
   for (int it = 0; it < IT; ++it) {
-    const int k = bk[it];
-    uint64_t pending = __ballot(k >= 0);
-    rk[it] = 0;
-    while (pending) {  // one step per distinct bucket of the wave
-      const int kk = __shfl(k, __ffsll((unsigned long long)pending) - 1, 64);
-      const uint64_t same = __ballot(k == kk);
-      if (k == kk)
-        rk[it] = __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32),
-                                           __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
-      if (lane == 0) sW[kk][it * NW + wave] = __popcll(same);
-      pending &= ~same;
+    // the lanes of the wave in this lane's bucket, by one ballot per bit of the bucket number
+    // (a step per distinct bucket took up to 33 dependent exchanges)
+    uint64_t same = __ballot(bk[it] >= 0);
+#pragma unroll
+    for (int bit = 0; bit < 6; ++bit) {
+      const uint64_t on = __ballot((bk[it] >> bit) & 1);
+      same &= ((bk[it] >> bit) & 1) ? on : ~on;
     }
+    rk[it] = __builtin_amdgcn_mbcnt_hi((uint32_t)(same >> 32),
+                                       __builtin_amdgcn_mbcnt_lo((uint32_t)same, 0u));
+    if (bk[it] >= 0 && rk[it] == 0) sW[bk[it]][it * NW + wave] = __popcll(same);
   }
   __syncthreads();
   // bucket k (wave k % NW, lane j = (pass, wave)): the exclusive scan of its counts over j and
@@ -171,24 +171,14 @@ __global__ __launch_bounds__(JSORT_THREADS) void joint_sort_kernel(JSortParams p
   static_assert(IT * NW <= 64, "one lane per (pass, wave)");
   for (int k = wave; k < NK; k += NW) {
     const int c = lane < IT * NW ? sW[k][lane] : 0;
-    int incl = c;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int v = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += v;
-    }
+    const int incl = (int)dkv_wave_scan_fast((float)c);  // counts up to 2048: exact in fp32
     if (lane < IT * NW) sW[k][lane] = incl - c;
     if (lane == 63) sTot[k] = incl;
   }
   __syncthreads();
   if (wave == 0) {
     const int tot = lane < NK ? sTot[lane] : 0;
-    int incl = tot;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const int v = __shfl_up(incl, d, 64);
-      if (lane >= d) incl += v;
-    }
+    const int incl = (int)dkv_wave_scan_fast((float)tot);
     if (lane < NK) sTot[lane] = npad + incl - tot;  // the bucket's first slot
   }
   for (int i = tid; i < npad; i += JSORT_THREADS) {
@@ -222,9 +212,9 @@ __global__ __launch_bounds__(JSORT_THREADS) void joint_sort_kernel(JSortParams p
 // composed per lane from the R(n) table and the window's R(16T) rows in LDS; the query operand
 // is then the same for every token and formed once per head. Scores are stored at the tokens'
 // positions.
-template <int DT, int MODE, int ODT, int NHB>
+// NHB basis heads and CB 16-token blocks per wave; a wave's coefficients are loaded PF chunks ahead.
+template <int DT, int MODE, int ODT, int NHB, int CB, int PF>
 __global__ __launch_bounds__(JTHREADS, 1) void joint_scores_sorted_kernel(JScoresParams p) {
-  constexpr int CB = JCB / NHB;            // 16-token blocks per wave
   constexpr int TOK = JWAVES * CB * 16;    // tokens per workgroup
   static_assert(JSWIN % TOK == 0 && 512 % TOK == 0, "windows hold whole workgroups");
   __shared__ __attribute__((aligned(16))) dkv_u32x4 sB[4][NHB][JDH * JCH / 8];
@@ -367,7 +357,7 @@ __global__ __launch_bounds__(JTHREADS, 1) void joint_scores_sorted_kernel(JScore
   // The rank loop: chunk c's basis sits in sB[c & 3], written at step c-2 (or before the loop),
   // and a barrier follows every odd step, so buffer (c+2) & 3 (last read at step c-2) may take
   // chunk c+2's basis, loaded two steps ago, and the registers it came from the basis of c+4.
-  // The coefficients of chunk c+2 are loaded, after chunk c's products are issued, into the
+  // The coefficients of chunk c+PF are loaded, after chunk c's products are issued, into the
   // registers chunk c used. Each block's products and coefficient loads stop at its own chunk
   // count (wave-uniform branches); loads past the last chunk clamp the basis index.
   auto rank_loop = [&](auto safe_tag) {
@@ -384,12 +374,15 @@ __global__ __launch_bounds__(JTHREADS, 1) void joint_scores_sorted_kernel(JScore
         }
       }
     };
-    dkv_u32x4 xa[CB], xb[CB];
+    static_assert(PF == 2 || PF == 4, "chunk c's coefficients in xs[c % PF], two chunks a barrier");
+    dkv_u32x4 xs[PF][CB];
     dkv_u32x4 ba[NHB], bb[NHB];
 #pragma unroll
     for (int hh = 0; hh < NHB; ++hh) ba[hh] = bb[hh] = dkv_u32x4{0u, 0u, 0u, 0u};
 #pragma unroll
-    for (int cb = 0; cb < CB; ++cb) xa[cb] = xb[cb] = dkv_u32x4{0u, 0u, 0u, 0u};
+    for (int k = 0; k < PF; ++k)
+#pragma unroll
+      for (int cb = 0; cb < CB; ++cb) xs[k][cb] = dkv_u32x4{0u, 0u, 0u, 0u};
     auto load_b = [&](int c, int hh) {
       return *(const dkv_u32x4*)(bsrc + hh * p.bt_sh + p.bt_sc * min(c, nch - 1));
     };
@@ -401,8 +394,8 @@ __global__ __launch_bounds__(JTHREADS, 1) void joint_scores_sorted_kernel(JScore
         ba[hh] = load_b(2, hh);
         bb[hh] = load_b(3, hh);
       }
-      load_x(0, xa);
-      load_x(1, xb);
+#pragma unroll
+      for (int k = 0; k < PF; ++k) load_x(k, xs[k]);
     }
     __syncthreads();
     auto step = [&](int c, dkv_u32x4(&x)[CB], dkv_u32x4(&bn)[NHB], bool sync) {
@@ -431,16 +424,21 @@ __global__ __launch_bounds__(JTHREADS, 1) void joint_scores_sorted_kernel(JScore
               for (int blk = 0; blk < 8; ++blk)
                 acc[hh][blk][cb] = dkv_mfma32<DT>(a[hh][blk], x[cb], acc[hh][blk][cb]);
           }
-        load_x(c + 2, x);
+        load_x(c + PF, x);
       }
       if (sync) __syncthreads();
     };
     int c = 0;
-    for (; c + 1 < nch; c += 2) {
-      step(c, xa, ba, false);
-      step(c + 1, xb, bb, true);
+    for (; c + PF - 1 < nch; c += PF) {
+#pragma unroll
+      for (int k = 0; k < PF; k += 2) {
+        step(c + k, xs[k], ba, false);
+        step(c + k + 1, xs[k + 1], bb, true);
+      }
     }
-    if (c < nch) step(c, xa, ba, false);
+#pragma unroll
+    for (int k = 0; k < PF - 1; ++k)
+      if (c + k < nch) step(c + k, xs[k], (k & 1) ? bb : ba, k & 1);
   };
   if (b == p.B - 1)
     rank_loop(std::integral_constant<bool, true>{});
@@ -1042,9 +1040,19 @@ extern "C" int dkv_joint_scores(void* stream, int mode, int dtype, int out_dtype
   p.win = joint_window(S);
   p.nwin = (S + p.win - 1) / p.win;
   // two basis heads per workgroup when the heads pair up (each coefficient load then serves
-  // both heads' products)
-  const int nhb = n_basis % 2 == 0 ? 2 : 1;
-  const int tok = JTOK / nhb;
+  // both heads' products); up to 128 such workgroups, half the CUs or fewer, 128 tokens of one
+  // head per workgroup instead, the coefficients four chunks ahead (a wave has the registers for
+  // it with one block): four times the workgroups for the same chain of chunks. Graph-replayed us
+  // of the whole call (32 query, 8 KV heads), large / small shape: 1 x 100 tokens (4 workgroups)
+  // 43.6 / 38.2, 2 x 411 (16) 61.7 / 48.5, 1 x 4096 (64) 90.4 / 69.8, 2 x 4096 (128) 87.0 / 75.8;
+  // 3 x 8000 with 4 KV heads (192) 62.6 / 67.9, 4 x 4096 (256) 90.6 / 105.
+  int nhb = n_basis % 2 == 0 ? 2 : 1;
+  int tok = JTOK / nhb;
+  const bool few = (long long)p.nwin * (p.win / tok) * (n_basis / nhb) * B <= 128;
+  if (few) {
+    nhb = 1;
+    tok = JWAVES * 16;
+  }
   p.n_basis = n_basis;
   const long long n_wg = (long long)p.nwin * (p.win / tok) * (n_basis / nhb) * B;
   if (n_wg > 0x7fffffffLL) return DKV_E_UNSUPPORTED;
@@ -1069,11 +1077,14 @@ extern "C" int dkv_joint_scores(void* stream, int mode, int dtype, int out_dtype
   const dim3 grid((unsigned)n_wg);
 #define DKV_JS_LAUNCH(DT_, MODE_, ODT_)                                                        \
   do {                                                                                         \
-    if (nhb == 2)                                                                              \
-      hipLaunchKernelGGL((joint_scores_sorted_kernel<DT_, MODE_, ODT_, 2>), grid,              \
+    if (few)                                                                                   \
+      hipLaunchKernelGGL((joint_scores_sorted_kernel<DT_, MODE_, ODT_, 1, 1, 4>), grid,        \
+                         dim3(JTHREADS), 0, st, p);                                            \
+    else if (nhb == 2)                                                                         \
+      hipLaunchKernelGGL((joint_scores_sorted_kernel<DT_, MODE_, ODT_, 2, JCB / 2, 2>), grid,  \
                          dim3(JTHREADS), 0, st, p);                                            \
     else                                                                                       \
-      hipLaunchKernelGGL((joint_scores_sorted_kernel<DT_, MODE_, ODT_, 1>), grid,              \
+      hipLaunchKernelGGL((joint_scores_sorted_kernel<DT_, MODE_, ODT_, 1, JCB, 2>), grid,      \
                          dim3(JTHREADS), 0, st, p);                                            \
   } while (0)
   if (mode == 1) {
