@@ -8,6 +8,7 @@ CPU or eager-PyTorch path.
 from __future__ import annotations
 
 import ctypes as C
+import importlib.util
 import threading
 from pathlib import Path
 
@@ -122,6 +123,7 @@ class DecodeLayerArgs(C.Structure):
 
 _lock = threading.Lock()
 _lib = None
+_calls = None
 
 
 class DynaKVError(RuntimeError):
@@ -150,6 +152,27 @@ def load() -> C.CDLL:
     return _lib
 
 
+def calls():
+    """The per-call entry points as the ``_dkv_call`` module's functions: the same C functions as
+    ``load()``'s, without ctypes' argument conversion (~5 us of a 40-argument call). Raises if the
+    module has not been built."""
+    global _calls
+    if _calls is not None:
+        return _calls
+    load()  # the library (and torch's HIP runtime) first: the module binds to it
+    with _lock:
+        if _calls is None:
+            path = LIB_PATH.with_name("_dkv_call.so")
+            if not path.exists():
+                raise RuntimeError(f"dynakv_amd call module not found at {path}; "
+                                   "build it with `python -m dynakv_amd.build`")
+            spec = importlib.util.spec_from_file_location("_dkv_call", path)
+            mod = importlib.util.module_from_spec(spec)
+            spec.loader.exec_module(mod)
+            _calls = mod
+    return _calls
+
+
 def exported_symbols() -> list[str]:
     return list(_SIGNATURES)
 
@@ -176,22 +199,23 @@ def flat_covers_rows(t: torch.Tensor) -> bool:
     """The C ABI's contract for packed flat buffers (rows, ld): rows * ld elements addressable
     from the base pointer inside the tensor's storage (each kernel's buffer resource for row r
     covers the elements from row r to the buffer's end, ``dkv_flat_range_elems``)."""
-    if t.dim() != 2 or t.stride(0) < 0:
+    if t.dim() != 2:
         return False
+    ld = t.stride(0)
     avail = t.untyped_storage().nbytes() // t.element_size() - t.storage_offset()
-    return t.shape[0] * t.stride(0) <= avail
+    return ld >= 0 and t.shape[0] * ld <= avail
 
 
 def view_extent(t: torch.Tensor) -> int:
     """Elements addressable from ``t.data_ptr()`` by its shape and strides (one past its last
-    element), from the library's own definition (``dkv_view_extent_elems``)."""
-    nd = t.dim()
-    shape = (C.c_longlong * max(nd, 1))(*t.shape)
-    stride = (C.c_longlong * max(nd, 1))(*t.stride())
-    n = int(load().dkv_view_extent_elems(nd, shape, stride))
-    if n < 0:
-        raise ValueError("dkv_view_extent_elems rejected the view")
-    return n
+    element): the library's ``dkv_view_extent_elems``, evaluated here (two ctypes arrays per call
+    cost more than the launch they guard)."""
+    last = 1
+    for n, st in zip(t.shape, t.stride()):
+        if n <= 0:
+            return 0
+        last += (n - 1) * st
+    return last
 
 
 def flat_operand(t: torch.Tensor) -> torch.Tensor:
@@ -217,11 +241,18 @@ def retire(t: torch.Tensor | None) -> None:
         _RETIRED_BUFFERS.append(t)
 
 
+# torch.cuda.current_stream(d).cuda_stream without building a Stream object (2 us of a call whose
+# launch takes 3): torch's own raw accessor where this torch has it
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_of(t: torch.Tensor) -> int:
     """Raw hipStream_t of torch's current stream on t's device."""
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise RuntimeError(
             f"dynakv_amd kernels need device tensors (got {t.device}); there is no CPU path")
+    if _raw_stream is not None:
+        return _raw_stream(t.get_device())
     return torch.cuda.current_stream(t.device).cuda_stream
 
 

@@ -1,7 +1,8 @@
 """Build the C-ABI shared library ``dynakv_amd/lib/libdynakv_amd.so`` for gfx950.
 
-Plain ``hipcc`` per source file (in parallel), then one link step. The library is built
-in-tree so it travels with the repository snapshot to the GPU host.
+Plain ``hipcc`` per source file (in parallel), then one link step, then the CPython binding of its
+per-call entry points (``dkv_call.cpp``, ``dynakv_amd/lib/_dkv_call.so``) linked against it. Both
+are built in-tree so they travel with the repository snapshot to the GPU host.
 
 Usage: ``python -m dynakv_amd.build`` (or ``dynakv_amd.build.build()``).
 """
@@ -13,12 +14,14 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_DIR = PKG_DIR / "lib"
 LIB_PATH = LIB_DIR / "libdynakv_amd.so"
+CALL_PATH = LIB_DIR / "_dkv_call.so"
 OBJ_DIR = PKG_DIR / "_build"
 SOURCES = ("dkv_append.hip", "dkv_generic.hip", "dkv_splitk.hip", "dkv_cutoff.hip",
            "dkv_prefill.hip", "dkv_layer.hip", "dkv_model.hip", "dkv_joint.hip", "dkv_dense.hip",
@@ -59,6 +62,18 @@ def _compile(src: Path, obj: Path) -> None:
         raise RuntimeError(f"hipcc failed for {src.name}:\n{' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
 
 
+def _build_binding() -> None:
+    """The CPython module over the library's entry points, found beside it at run time."""
+    tmp = CALL_PATH.with_suffix(".so.tmp")
+    cmd = [_hipcc(), "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wno-cast-function-type",
+           "-I", sysconfig.get_paths()["include"], str(CSRC / "dkv_call.cpp"), "-o", str(tmp),
+           f"-L{LIB_DIR}", "-l:libdynakv_amd.so", "-Wl,-rpath,$ORIGIN"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"binding failed:\n{' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
+    os.replace(tmp, CALL_PATH)
+
+
 def build(verbose: bool = True) -> Path:
     """Compile every HIP source and link the shared library. Always rebuilds."""
     OBJ_DIR.mkdir(exist_ok=True)
@@ -74,6 +89,7 @@ def build(verbose: bool = True) -> Path:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
+    _build_binding()
     if verbose:
         print(f"[dynakv_amd] built {LIB_PATH}", file=sys.stderr)
     return LIB_PATH

@@ -182,7 +182,7 @@ class CustomDynamicCache(_CacheBase):
         sv = vs if vs.stride(-1) == 1 else vs.contiguous()
         nk, nv = kl.to(torch.int32), vl.to(torch.int32)
         B, new_s = kl.shape
-        rc = _lib.load().dkv_append_prefill_kv(
+        rc = _lib.calls().dkv_append_prefill_kv(
             _lib.stream_of(fk), _lib.dtype_code(fk.dtype), seq, B, new_s, max_dim,
             sk.data_ptr(), sk.stride(0), sk.stride(1), nk.data_ptr(), nk.stride(0), nk.stride(1),
             fk.data_ptr(), fk.stride(0), lk.data_ptr(), okk.data_ptr(), lk.stride(0),
@@ -206,7 +206,7 @@ class CustomDynamicCache(_CacheBase):
         st = _lib.stream_of(flat)
         states = new_states if new_states.stride(-1) == 1 else new_states.contiguous()
         nl = new_len.to(torch.int32)
-        rc = _lib.load().dkv_append_prefill(
+        rc = _lib.calls().dkv_append_prefill(
             st, _lib.dtype_code(flat.dtype), states.data_ptr(), states.stride(0), states.stride(1),
             nl.data_ptr(), nl.stride(0), nl.stride(1), flat.data_ptr(), flat.stride(0),
             lens.data_ptr(), offs.data_ptr(), lens.stride(0), lens.stride(1),
@@ -234,7 +234,7 @@ class CustomDynamicCache(_CacheBase):
         if is_decode:
             flat, lens, offs, ptr, seq, _ = cache
             states, nl = self._decode_view(new_states, new_len)
-            rc = _lib.load().dkv_append_decode(
+            rc = _lib.calls().dkv_append_decode(
                 _lib.stream_of(flat), _lib.dtype_code(flat.dtype), states.data_ptr(),
                 states.stride(0), nl.data_ptr(), nl.stride(0), flat.data_ptr(), flat.stride(0),
                 lens.data_ptr(), offs.data_ptr(), lens.stride(0), lens.stride(1), ptr.data_ptr(),
@@ -354,7 +354,7 @@ class CustomDynamicCache(_CacheBase):
                 vs, vl = self._decode_view(value_states, value_len)
                 fk, lk, ok, pk, seq, _ = ck
                 fv, lv, ov, pv, _, _ = cv
-                rc = _lib.load().dkv_append_decode_kv(
+                rc = _lib.calls().dkv_append_decode_kv(
                     _lib.stream_of(fk), _lib.dtype_code(fk.dtype), key_len.shape[0], md, seq,
                     ks.data_ptr(), ks.stride(0), kl.data_ptr(), kl.stride(0),
                     fk.data_ptr(), fk.stride(0), lk.data_ptr(), ok.data_ptr(),
@@ -378,7 +378,7 @@ class CustomDynamicCache(_CacheBase):
     def _launch_decode_single(self, cache, new_states, new_len, max_dim):
         flat, lens, offs, ptr, seq, _ = cache
         states, nl = self._decode_view(new_states, new_len)
-        rc = _lib.load().dkv_append_decode(
+        rc = _lib.calls().dkv_append_decode(
             _lib.stream_of(flat), _lib.dtype_code(flat.dtype), states.data_ptr(), states.stride(0),
             nl.data_ptr(), nl.stride(0), flat.data_ptr(), flat.stride(0), lens.data_ptr(),
             offs.data_ptr(), lens.stride(0), lens.stride(1), ptr.data_ptr(), seq,
@@ -391,7 +391,7 @@ class CustomDynamicCache(_CacheBase):
         out = flat.new_empty(rows, seq, max_dim)
         if rows == 0 or seq == 0:
             return out.zero_()
-        rc = _lib.load().dkv_decompress(
+        rc = _lib.calls().dkv_decompress(
             _lib.stream_of(flat), _lib.dtype_code(flat.dtype), flat.data_ptr(), flat.stride(0),
             lens.data_ptr(), offs.data_ptr(), lens.stride(0), lens.stride(1), out.data_ptr(),
             rows, seq, max_dim)

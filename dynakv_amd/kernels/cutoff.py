@@ -114,38 +114,37 @@ def cutoff_kv(key_states: torch.Tensor, value_states: torch.Tensor, wt_k: torch.
             or wt_k.dtype != dt or wt_v.dtype != dt):
         raise ValueError("cutoff head runs in float16 or bfloat16 (inputs and weights alike)")
     G, D = wt_k.shape[0], wt_k.shape[1]
-    hidden = key_states.shape[-1]
+    shape = key_states.shape
+    hidden = shape[-1]
     if hidden != G * D:
         raise ValueError(f"states have {hidden} dims, weights cover {G} x {D}")
-    lead = key_states.shape[:-1]
-    xk = _rows(key_states.reshape(-1, hidden))
-    xv = _rows(value_states.reshape(-1, hidden))
-    if xv.stride(0) != xk.stride(0):
-        xk = xk.clone(memory_format=torch.contiguous_format)
-        xv = xv.clone(memory_format=torch.contiguous_format)
-    M = xk.shape[0]
+    lead = shape[:-1]
     dev = key_states.device
-    out = torch.empty((2, M, hidden), dtype=dt, device=dev)  # one allocation each for the
-    lens = torch.empty((2, M, G), dtype=torch.int32, device=dev)  # outputs and the lengths
-    out_k, out_v, len_k, len_v = out[0], out[1], lens[0], lens[1]
+    if (key_states.is_contiguous() and value_states.is_contiguous() and hidden % 8 == 0
+            and key_states.data_ptr() % 16 == 0 and value_states.data_ptr() % 16 == 0):
+        xk, xv, ld = key_states, value_states, hidden  # whole rows as they lie
+        M = xk.numel() // hidden
+    else:
+        xk = _rows(key_states.reshape(-1, hidden))
+        xv = _rows(value_states.reshape(-1, hidden))
+        if xv.stride(0) != xk.stride(0):
+            xk = xk.clone(memory_format=torch.contiguous_format)
+            xv = xv.clone(memory_format=torch.contiguous_format)
+        M, ld = xk.shape[0], xk.stride(0)
+    out_k = torch.empty(shape, dtype=dt, device=dev)
+    out_v = torch.empty(shape, dtype=dt, device=dev)
+    len_k, len_v = torch.empty((2, *lead) if G == 1 else (2, *lead, G), dtype=torch.int32,
+                               device=dev).unbind(0)  # one allocation for both
     if M > 0:
-        lib = _lib.load()
+        lib = _lib.calls()
         st = _lib.stream_of(key_states)
         nb = int(lib.dkv_cutoff_workspace_bytes(M, G, D))
         ws = _workspace(dev, st, nb)
         lr = -1 if low_rank is None else int(low_rank)
-        rc = lib.dkv_cutoff_kv(st, _lib.dtype_code(dt), xk.data_ptr(), xv.data_ptr(), xk.stride(0),
+        rc = lib.dkv_cutoff_kv(st, _lib.dtype_code(dt), xk.data_ptr(), xv.data_ptr(), ld,
                                wt_k.data_ptr(), wt_v.data_ptr(), b_k.data_ptr(), b_v.data_ptr(),
-                               float(threshold), lr, out_k.data_ptr(), out_v.data_ptr(),
-                               out_k.stride(0), len_k.data_ptr(), len_v.data_ptr(), len_k.stride(0),
-                               ws.data_ptr(), ws.numel(), M, G, D)
+                               float(threshold), lr, out_k.data_ptr(), out_v.data_ptr(), hidden,
+                               len_k.data_ptr(), len_v.data_ptr(), G, ws.data_ptr(), ws.numel(),
+                               M, G, D)
         _lib.check(rc, "dkv_cutoff_kv")
-    out_k = out_k.reshape(*lead, hidden)
-    out_v = out_v.reshape(*lead, hidden)
-    if G == 1:
-        len_k = len_k.reshape(*lead)
-        len_v = len_v.reshape(*lead)
-    else:
-        len_k = len_k.reshape(*lead, G)
-        len_v = len_v.reshape(*lead, G)
     return out_k, len_k, out_v, len_v

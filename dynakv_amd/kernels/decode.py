@@ -30,7 +30,7 @@ _WS_CACHE: dict = {}    # (device, stream) -> zeroed fp32 workspace
 def rope_table(device: torch.device, stream: int, theta: float, seq_len: int):
     """RoPE table with at least ceil(seq_len / 16) tile rows for ``theta`` (cached, grown by
     doubling; a replaced table stays allocated, ``_lib.retire``)."""
-    lib = _lib.load()
+    lib = _lib.calls()
     need = max(1, (seq_len + 15) // 16)
     key = (device.index, stream, float(theta))
     ent = _ROPE_CACHE.get(key)
@@ -109,13 +109,14 @@ def splitk_layout(q3: torch.Tensor, k_up: torch.Tensor, v_up: torch.Tensor,
     ``expand``) is one shared basis; otherwise every query head is its own unit.
     """
     dt = q3.dtype
-    if dt not in (torch.float16, torch.bfloat16) or q3.device.type != "cuda":
+    if dt not in (torch.float16, torch.bfloat16) or not q3.is_cuda:
         return None
     if not (k_flat.dtype == v_flat.dtype == k_up.dtype == v_up.dtype == dt):
         return None
-    if k_up.dim() != 3 or v_up.shape != k_up.shape:
+    shape = k_up.shape
+    if len(shape) != 3 or v_up.shape != shape:
         return None
-    hb, r, dh = k_up.shape
+    hb, r, dh = shape
     B, hq, qdh = q3.shape
     if dh != SPLITK_HEAD_DIM or qdh != dh or r > SPLITK_MAX_RANK or r <= 0 or hq % hb:
         return None
@@ -152,42 +153,48 @@ def splitk_attention(q3: torch.Tensor, k_flat: torch.Tensor, v_flat: torch.Tenso
 
     The output is in ``q3``'s dtype (the reference's contract) unless ``out_dtype=torch.float32``
     asks for the merged result before that rounding."""
-    lib = _lib.load()
+    lib = _lib.calls()
     B, hq, dh = q3.shape
-    if q3.stride(2) != 1:
+    q_sb, q_sh, q_sd = q3.stride()
+    if q_sd != 1:
         q3 = q3.contiguous()
+        q_sb, q_sh, _ = q3.stride()
     S = lens_k.shape[1]
-    R = layout.k_basis.shape[1]
-    for t in (lens_k, offs_k, lens_v, offs_v):
-        if t.dtype != torch.int32:
-            raise ValueError("length/offset tables must be int32")
-    if offs_k.stride() != lens_k.stride() or offs_v.stride() != lens_v.stride():
+    kb, vb = layout.k_basis, layout.v_basis
+    R = kb.shape[1]
+    if not (lens_k.dtype == offs_k.dtype == lens_v.dtype == offs_v.dtype == torch.int32):
+        raise ValueError("length/offset tables must be int32")
+    tk, tv = lens_k.stride(), lens_v.stride()
+    if offs_k.stride() != tk or offs_v.stride() != tv:
         lens_k, offs_k = lens_k.contiguous(), offs_k.contiguous()
         lens_v, offs_v = lens_v.contiguous(), offs_v.contiguous()
-    odt = out_dtype if out_dtype is not None else (out.dtype if out is not None else q3.dtype)
-    if odt not in (q3.dtype, torch.float32):
+        tk, tv = lens_k.stride(), lens_v.stride()
+    qdt = q3.dtype
+    odt = out_dtype if out_dtype is not None else (out.dtype if out is not None else qdt)
+    if odt not in (qdt, torch.float32):
         raise ValueError("out_dtype must be the query dtype or float32")
     if out is None:
         out = torch.empty((B, hq, dh), dtype=odt, device=q3.device)
+        o_sb, o_sh = hq * dh, dh
     elif out.dtype != odt or out.stride(2) != 1:
         raise ValueError("out must have unit last stride and the requested dtype")
+    else:
+        o_sb, o_sh, _ = out.stride()
     k_flat, v_flat = _lib.flat_operand(k_flat), _lib.flat_operand(v_flat)
     st = _lib.stream_of(q3)
-    nfl = lib.dkv_splitk_workspace_floats(B, hq, layout.n_kv, S, R, split_len)
-    ws = workspace(q3.device, st, int(nfl))
-    rope, rope_tiles = rope_table(q3.device, st, theta, S)
+    dev = q3.device
+    ws = workspace(dev, st, lib.dkv_splitk_workspace_floats(B, hq, layout.n_kv, S, R, split_len))
+    rope, rope_tiles = rope_table(dev, st, theta, S)
     # stride of the bases' non-unit axis: the rank, or the dim of transposed bases
     fn, ax = (lib.dkv_decode_splitk_bt, 2) if layout.transposed else (lib.dkv_decode_splitk, 1)
     rc = fn(
-        st, route, _lib.dtype_code(q3.dtype),
-        q3.data_ptr(), q3.stride(0), q3.stride(1),
-        layout.k_basis.data_ptr(), layout.k_unit, layout.k_basis.stride(ax),
-        layout.v_basis.data_ptr(), layout.v_unit, layout.v_basis.stride(ax),
+        st, route, _lib.dtype_code(qdt), q3.data_ptr(), q_sb, q_sh,
+        kb.data_ptr(), layout.k_unit, kb.stride(ax), vb.data_ptr(), layout.v_unit, vb.stride(ax),
         k_flat.data_ptr(), k_flat.stride(0), v_flat.data_ptr(), v_flat.stride(0),
-        lens_k.data_ptr(), offs_k.data_ptr(), lens_k.stride(0), lens_k.stride(1),
-        lens_v.data_ptr(), offs_v.data_ptr(), lens_v.stride(0), lens_v.stride(1),
+        lens_k.data_ptr(), offs_k.data_ptr(), tk[0], tk[1],
+        lens_v.data_ptr(), offs_v.data_ptr(), tv[0], tv[1],
         rope.data_ptr(), rope_tiles, ws.data_ptr(), ws.numel(),
-        out.data_ptr(), out.stride(0), out.stride(1), _lib.dtype_code(out.dtype),
+        out.data_ptr(), o_sb, o_sh, _lib.dtype_code(odt),
         B, hq, layout.n_kv, groups, S, R, dh, split_len)
     _lib.check(rc, "dkv_decode_splitk")
     return out
@@ -230,7 +237,7 @@ def dense_decode_attention(q: torch.Tensor, k_cache: torch.Tensor, v_cache: torc
     ``q``: (B, Hq, 128) or (B, Hq, 1, 128), rotated. ``k_cache`` / ``v_cache``: (B * Hkv, ld)
     with unit last stride; row b * Hkv + g holds token t's rotated key (value) at elements
     t * 128 .. t * 128 + 127; tokens 0 .. S-1 are attended."""
-    lib = _lib.load()
+    lib = _lib.calls()
     q3 = q.squeeze(2) if q.dim() == 4 else q
     if q3.stride(2) != 1 or q3.data_ptr() % 16 or q3.stride(0) % 8 or q3.stride(1) % 8:
         q3 = q3.contiguous()
@@ -268,7 +275,7 @@ def dense_append_(y: torch.Tensor, k_cache: torch.Tensor, v_cache: torch.Tensor,
     ``kv_heads`` value heads of 128); the query heads are rotated in place at ``q_pos``, the key
     heads rotated at ``k_pos`` into ``k_cache`` (B * kv_heads, ld) at token ``k_pos``, the value
     heads copied into ``v_cache``."""
-    lib = _lib.load()
+    lib = _lib.calls()
     if y.dim() != 2 or y.stride(1) != 1:
         raise ValueError("y must be (B, W) with unit last stride")
     if k_cache.stride(1) != 1 or v_cache.stride(1) != 1 or k_cache.stride(0) != v_cache.stride(0):

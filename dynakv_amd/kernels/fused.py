@@ -35,7 +35,7 @@ def fused_attention_dispatch(q, k_flat, k_up, v_flat, v_up, l_k, o_k, l_v, o_v, 
 
 def _fused_vector(q, k_flat, k_up, v_flat, v_up, l_k, o_k, l_v, o_v, theta):
     """Reference-semantics vector kernels: fp32 scores with -inf masking, then the V pass."""
-    lib = _lib.load()
+    lib = _lib.calls()
     batch, num_heads, head_dim = q.shape
     seq_len = l_k.shape[1]
     if q.stride(2) != 1:

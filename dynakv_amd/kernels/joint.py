@@ -69,7 +69,7 @@ def _remember(cache: dict, t: torch.Tensor, key, value) -> None:
 
 
 def _key(t: torch.Tensor, *extra):
-    return (t.data_ptr(), tuple(t.shape), tuple(t.stride()), t._version, *extra)
+    return (t.data_ptr(), t.shape, t.stride(), t._version, *extra)
 
 
 def _repeat_factor(basis: torch.Tensor, n_heads: int) -> int:
@@ -132,7 +132,7 @@ def scores_eligible(q3: torch.Tensor, k_up: torch.Tensor, k_flat: torch.Tensor) 
     Hq, Hb = q3.shape[1], k_up.shape[0]
     if R % 32 or R > 1024 or Hb <= 0 or Hq % Hb or not _flat_ok(k_flat):
         return False
-    return Hq // Hb <= 8 or Hq // _distinct(k_up, Hq).shape[0] <= 8
+    return Hq // Hb <= 8 or Hq // (Hb // _repeat_factor(k_up, Hq)) <= 8
 
 
 def av_eligible(v_up: torch.Tensor, v_flat: torch.Tensor, n_heads: int, S: int) -> bool:
@@ -156,17 +156,17 @@ def joint_scores(q3: torch.Tensor, k_up: torch.Tensor, k_flat: torch.Tensor,
     st = _lib.stream_of(q3)
     rope, tiles = rope_table(q3.device, st, theta, S)
     out = torch.empty((B, Hq, S), dtype=out_dtype, device=q3.device)
-    lib = _lib.load()
-    ws = _sort_workspace(q3.device, st, int(lib.dkv_joint_scores_workspace_ints(B, S)))
+    lib = _lib.calls()
+    ws = _sort_workspace(q3.device, st, lib.dkv_joint_scores_workspace_ints(B, S))
+    bs, qs, ls, os_ = bt.stride(), q3.stride(), lens.stride(), offs.stride()
     rc = lib.dkv_joint_scores(
         st, mode, _lib.dtype_code(q3.dtype), _lib.dtype_code(out_dtype),
-        q3.data_ptr(), q3.stride(0), q3.stride(1),
-        bt.data_ptr(), bt.stride(0), bt.stride(1), bt.shape[0],  # head and chunk strides
+        q3.data_ptr(), qs[0], qs[1],
+        bt.data_ptr(), bs[0], bs[1], bt.shape[0],  # head and chunk strides
         k_flat.data_ptr(), k_flat.stride(0),
-        lens.data_ptr(), lens.stride(0), lens.stride(1),
-        offs.data_ptr(), offs.stride(0), offs.stride(1),
+        lens.data_ptr(), ls[0], ls[1], offs.data_ptr(), os_[0], os_[1],
         rope.data_ptr(), tiles, ws.data_ptr(), ws.numel(),
-        out.data_ptr(), out.stride(0), out.stride(1), out.stride(2),
+        out.data_ptr(), Hq * S, S, 1,
         B, Hq, S, k_up.shape[1], Dh)
     _lib.check(rc, "dkv_joint_scores")
     return out
@@ -177,7 +177,7 @@ def joint_av(scores: torch.Tensor, v_up: torch.Tensor, v_flat: torch.Tensor,
              out_dtype: torch.dtype) -> torch.Tensor:
     """The V pass (B, Hq, Dh) of the route ``mode`` (0: avx, 1: fused) on MFMA."""
     B, Hq, S = scores.shape
-    lib = _lib.load()
+    lib = _lib.calls()
     st = _lib.stream_of(scores)
     R = v_up.shape[1]
     if v_up.stride(2) != 1:
@@ -186,16 +186,16 @@ def joint_av(scores: torch.Tensor, v_up: torch.Tensor, v_flat: torch.Tensor,
     v_flat = _lib.flat_operand(v_flat)
     ws = _workspace(scores.device, st, int(lib.dkv_joint_av_workspace_floats(B, Hq, S, R)))
     out = torch.empty((B, Hq, 128), dtype=out_dtype, device=scores.device)
+    ss, vs, ls, os_ = scores.stride(), v_up.stride(), lens.stride(), offs.stride()
     rc = lib.dkv_joint_av(
         st, mode, _lib.dtype_code(scores.dtype), _lib.dtype_code(v_flat.dtype),
         _lib.dtype_code(out_dtype),
-        scores.data_ptr(), scores.stride(0), scores.stride(1), scores.stride(2),
-        v_up.data_ptr(), v_up.stride(0), v_up.stride(1), v_up.shape[0],
+        scores.data_ptr(), ss[0], ss[1], ss[2],
+        v_up.data_ptr(), vs[0], vs[1], v_up.shape[0],
         v_flat.data_ptr(), v_flat.stride(0),
-        lens.data_ptr(), lens.stride(0), lens.stride(1),
-        offs.data_ptr(), offs.stride(0), offs.stride(1),
+        lens.data_ptr(), ls[0], ls[1], offs.data_ptr(), os_[0], os_[1],
         ws.data_ptr(), ws.numel(),
-        out.data_ptr(), out.stride(0), out.stride(1),
+        out.data_ptr(), Hq * 128, 128,
         B, Hq, S, R, 128)
     _lib.check(rc, "dkv_joint_av")
     return out

@@ -51,7 +51,7 @@ class DecodeLayerPlan:
         if not (_lib.flat_covers_rows(fk) and _lib.flat_covers_rows(fv)):
             raise ValueError("the cache's flat buffers must hold rows * ld elements")
         st = _lib.stream_of(fk)
-        lib = _lib.load()
+        lib = _lib.calls()
         B, G, R, Dh, Hq = self.B, self.G, self.R, self.Dh, self.Hq
         self.cap_seq = min(lk.shape[1], lv.shape[1])
         self.cap_flat = min(fk.shape[1], fv.shape[1])
@@ -88,7 +88,7 @@ class DecodeLayerPlan:
         a.rope, a.rope_tiles = self.rope.data_ptr(), tiles
         a.split_ws, a.split_ws_floats = self.split_ws.data_ptr(), self.split_ws.numel()
         self.args = a
-        self._ptr = ctypes.byref(a)
+        self._ptr = ctypes.addressof(a)  # of self.args, which the plan keeps
         self._slots = (ck, cv)
         # the tensors the argument block points at must stay the cache's own
         self._bufs = (fk, lk, ok, pk, fv, lv, ov, pv)
@@ -124,7 +124,7 @@ class DecodeLayerPlan:
         a.q_sb = q.stride(0) if B > 1 else Hq * Dh
         a.coef_ld = k_coef.stride(0) if B > 1 else self.G * self.R
         out = torch.empty((B, Hq, Dh), dtype=q.dtype, device=q.device)
-        rc = _lib.load().dkv_decode_layer(_lib.stream_of(q), self._ptr, q.data_ptr(),
+        rc = _lib.calls().dkv_decode_layer(_lib.stream_of(q), self._ptr, q.data_ptr(),
                                           k_coef.data_ptr(), v_coef.data_ptr(), out.data_ptr(),
                                           seq, pos)
         _lib.check(rc, "dkv_decode_layer")

@@ -39,7 +39,7 @@ def add_rmsnorm_(x: torch.Tensor, delta: torch.Tensor | None, w: torch.Tensor, e
         raise ValueError("delta must have x's shape")
     if w.shape != (H,) or not w.is_contiguous() or w.dtype != x.dtype:
         raise ValueError("w must be a contiguous (H,) vector of x's dtype")
-    lib = _lib.load()
+    lib = _lib.calls()
     rc = lib.dkv_add_rmsnorm(_lib.stream_of(x), _lib.dtype_code(x.dtype), xr.data_ptr(),
                              xr.stride(0), dr.data_ptr() if dr is not None else None,
                              dr.stride(0) if dr is not None else 0, w.data_ptr(), orr.data_ptr(),
@@ -57,7 +57,7 @@ def silu_mul(gu: torch.Tensor) -> torch.Tensor:
     F = F2 // 2
     out = torch.empty(gu.shape[:-1] + (F,), dtype=gu.dtype, device=gu.device)
     orr = out.view(-1, F)
-    lib = _lib.load()
+    lib = _lib.calls()
     rc = lib.dkv_silu_mul(_lib.stream_of(gu), _lib.dtype_code(gu.dtype), gr.data_ptr(),
                           gr.stride(0), orr.data_ptr(), orr.stride(0), gr.shape[0], F)
     _lib.check(rc, "dkv_silu_mul")
@@ -74,7 +74,7 @@ def silu_mul_pairs(gu: torch.Tensor) -> torch.Tensor:
     F = F2 // 2
     out = torch.empty(gu.shape[:-1] + (F,), dtype=gu.dtype, device=gu.device)
     orr = out.view(-1, F)
-    lib = _lib.load()
+    lib = _lib.calls()
     rc = lib.dkv_silu_mul_pairs(_lib.stream_of(gu), _lib.dtype_code(gu.dtype), gr.data_ptr(),
                                 gr.stride(0), orr.data_ptr(), orr.stride(0), gr.shape[0], F)
     _lib.check(rc, "dkv_silu_mul_pairs")
@@ -98,7 +98,7 @@ def linear(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
         if xr.stride(1) == 1 and xr.data_ptr() % 16 == 0 and xr.stride(0) % 8 == 0 \
                 and w.data_ptr() % 16 == 0 and w.stride(0) % 8 == 0:
             y = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device)
-            rc = _lib.load().dkv_gemv(_lib.stream_of(x), _lib.dtype_code(x.dtype),
+            rc = _lib.calls().dkv_gemv(_lib.stream_of(x), _lib.dtype_code(x.dtype),
                                       xr.data_ptr(), xr.stride(0), w.data_ptr(), w.stride(0),
                                       y.data_ptr(), N, M, N, K)
             _lib.check(rc, "dkv_gemv")
@@ -125,7 +125,7 @@ def rmsnorm_linear(x: torch.Tensor, delta: torch.Tensor | None, w_norm: torch.Te
         N = w.shape[0]
         y = torch.empty(x.shape[:-1] + (N,), dtype=x.dtype, device=x.device)
         r = torch.empty_like(x) if delta is not None else x
-        rc = _lib.load().dkv_gemv_rmsnorm(
+        rc = _lib.calls().dkv_gemv_rmsnorm(
             _lib.stream_of(x), _lib.dtype_code(x.dtype), x.data_ptr(), K,
             delta.data_ptr() if delta is not None else None, K, w_norm.data_ptr(), float(eps),
             r.data_ptr() if delta is not None else None, K, w.data_ptr(), w.stride(0),
@@ -151,7 +151,7 @@ def rmsnorm_glu(x: torch.Tensor, delta: torch.Tensor | None, w_norm: torch.Tenso
     ok_w = (w_gu.dim() == 2 and w_gu.shape[1] == K and N % 2 == 0 and w_gu.stride(1) == 1
             and w_gu.stride(0) % 8 == 0 and w_gu.data_ptr() % 16 == 0 and w_gu.dtype == x.dtype
             and x.dtype in (torch.bfloat16, torch.float16) and K % 8 == 0 and x.is_cuda)
-    lib = _lib.load()
+    lib = _lib.calls()
     if ok_w and M <= 2 and x.is_contiguous() and (delta is None or delta.is_contiguous()) \
             and w_norm.dtype == x.dtype and x.data_ptr() % 16 == 0 \
             and (delta is None or delta.data_ptr() % 16 == 0) and M >= 1:

@@ -41,7 +41,7 @@ def rope_dense_(x: torch.Tensor, *, theta: float, pos0: int = 0) -> torch.Tensor
     x2 = x.reshape(rows, S, 128)
     if x2.data_ptr() != x.data_ptr():
         raise ValueError("rope_dense_ needs a tensor whose leading dims flatten without a copy")
-    lib = _lib.load()
+    lib = _lib.calls()
     _lib.check(lib.dkv_rope_dense(_lib.stream_of(x), _lib.dtype_code(x.dtype), x2.data_ptr(),
                                   x2.stride(0), x2.stride(1), rows, S, int(pos0),
                                   math.log(theta)), "dkv_rope_dense")
@@ -64,7 +64,7 @@ def rope_apply_(x: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor) -> torch.
     if cos.stride() != sin.stride() or cos.stride(-1) != 1:
         cos, sin = cos.contiguous(), sin.contiguous()
     cs_sb = 0 if cos.shape[0] == 1 else cos.stride(0)
-    lib = _lib.load()
+    lib = _lib.calls()
     _lib.check(lib.dkv_rope_apply(_lib.stream_of(x), _lib.dtype_code(x.dtype), x.data_ptr(),
                                   x.stride(0), x.stride(1), x.stride(2), cos.data_ptr(),
                                   sin.data_ptr(), cs_sb, cos.stride(1), B, H, S),
@@ -102,13 +102,13 @@ def prefill_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, *, caus
         if kstart.shape != (B,) or kstart.device != q.device:
             raise ValueError("kstart must be (B,) on q's device")
         kstart = kstart.to(torch.int32).contiguous()
-    lib = _lib.load()
+    lib = _lib.calls()
+    qs, ks, vs, os_ = q.stride(), k.stride(), v.stride(), out.stride()
     rc = lib.dkv_prefill_attention(
         _lib.stream_of(q), _lib.dtype_code(q.dtype),
-        q.data_ptr(), q.stride(0), q.stride(1), q.stride(2),
-        k.data_ptr(), k.stride(0), k.stride(1), k.stride(2), _extent(k),
-        v.data_ptr(), v.stride(0), v.stride(1), v.stride(2), _extent(v),
-        out.data_ptr(), _lib.dtype_code(out.dtype), out.stride(0), out.stride(1), out.stride(2),
+        q.data_ptr(), qs[0], qs[1], qs[2], k.data_ptr(), ks[0], ks[1], ks[2], _extent(k),
+        v.data_ptr(), vs[0], vs[1], vs[2], _extent(v),
+        out.data_ptr(), _lib.dtype_code(odt), os_[0], os_[1], os_[2],
         B, Hq, Hkv, Sq, Sk, Dh, 1 if causal else 0, scale,
         None if kstart is None else kstart.data_ptr())
     _lib.check(rc, "dkv_prefill_attention")
@@ -143,19 +143,20 @@ def recon_kv(ck: torch.Tensor, cv: torch.Tensor, k_basis: torch.Tensor, v_basis:
           and _basis_t_ok(k_basis) and _basis_t_ok(v_basis)
           and k_basis.stride() == v_basis.stride())
     kb, vb = (k_basis, v_basis) if bt else (k_basis.contiguous(), v_basis.contiguous())
-    if (ck.stride(0) % 8 or ck.stride(1) % 8 or ck.data_ptr() % 16 or cv.data_ptr() % 16
+    c_sr, c_st, _ = ck.stride()
+    if (c_sr % 8 or c_st % 8 or ck.data_ptr() % 16 or cv.data_ptr() % 16
             or kb.data_ptr() % 16 or vb.data_ptr() % 16):
         return None
     k = torch.empty((batch, G, S, Dh), dtype=dt, device=ck.device)
     v = torch.empty_like(k)
-    lib = _lib.load()
+    lib = _lib.calls()
     st = _lib.stream_of(ck)
     rope, tiles = rope_table(ck.device, st, theta, int(pos0) + S)
     fn, ax = (lib.dkv_recon_kv_bt, 2) if bt else (lib.dkv_recon_kv, 1)
-    _lib.check(fn(st, _lib.dtype_code(dt), ck.data_ptr(), cv.data_ptr(), ck.stride(0),
-                  ck.stride(1), kb.data_ptr(), vb.data_ptr(), kb.stride(0), kb.stride(ax),
-                  k.data_ptr(), v.data_ptr(), S * Dh, Dh, rows, G, S, R, int(pos0),
-                  rope.data_ptr(), tiles), "dkv_recon_kv")
+    _lib.check(fn(st, _lib.dtype_code(dt), ck.data_ptr(), cv.data_ptr(), c_sr, c_st,
+                  kb.data_ptr(), vb.data_ptr(), kb.stride(0), kb.stride(ax), k.data_ptr(),
+                  v.data_ptr(), S * Dh, Dh, rows, G, S, R, int(pos0), rope.data_ptr(), tiles),
+               "dkv_recon_kv")
     return k, v
 
 

@@ -34,7 +34,7 @@ def abx_sparse(a: torch.Tensor, b: torch.Tensor, x_flat: torch.Tensor, l_vec: to
     if seq_len > 0 and _joint.scores_eligible(a, b, x_flat):
         return _joint.joint_scores(a, b, x_flat, l_vec, offsets, theta=theta, mode=0,
                                    out_dtype=a.dtype)
-    lib = _lib.load()
+    lib = _lib.calls()
     if a.stride(2) != 1:
         a = a.contiguous()
     if b.stride(2) != 1:
@@ -64,7 +64,7 @@ def avx(a: torch.Tensor, x_flat: torch.Tensor, v_up: torch.Tensor, l_vec: torch.
         raise ValueError("offsets are required for the variable-length value cache")
     if _joint.av_eligible(v_up, x_flat, num_heads, seq_len):
         return _joint.joint_av(a, v_up, x_flat, l_vec, offsets, mode=0, out_dtype=a.dtype)
-    lib = _lib.load()
+    lib = _lib.calls()
     if v_up.stride(2) != 1:
         v_up = v_up.contiguous()
     out = torch.empty((batch, num_heads, head_dim), dtype=a.dtype, device=a.device)
