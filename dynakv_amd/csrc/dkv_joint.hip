@@ -26,6 +26,8 @@
 //   position; composed from LDS tables) in fp32, K' split into bf16 hi + lo, scores on MFMA
 //   against the unrotated query (hi and lo parts in separate operand columns, formed once per
 //   head), the route's masking and rounding, stored at the token's position.
+// joint_scores_few_kernel -- the scores of a short call without the pre-pass: workgroup = (32
+//   tokens, basis head, batch row), the rank chunks split over its waves, no barrier between them.
 // joint_av_kernel -- workgroup = (token split, 16 or 32 query heads, batch row b); wave w takes
 //   ranks [128w, 128w + 128). Per 16-token tile: each set of 16 heads' scores through an online
 //   softmax in the log2 domain (every wave computes the same values), P as bf16 hi + lo (fp16
@@ -508,6 +510,168 @@ __global__ __launch_bounds__(JTHREADS, 1) void joint_scores_sorted_kernel(JScore
             dkv_store_f32<ODT>(p.out, ob + (long long)t * p.out_ss, z);
           }
         }
+      }
+    }
+  }
+}
+
+// joint_scores_few_kernel: the scores of a call with few tokens, in the tokens' own order (no
+// pre-pass). Workgroup = (32 tokens, basis head h, batch row b); the 8 waves split the rank chunks
+// up to the longest token's between them, each forming its part of K^T for both 16-token blocks with
+// the basis read straight into A operands (a chunk's block of 16 dims is 1 KB in a row) one chunk
+// ahead; the parts meet in LDS, where wave (block tb, pp) adds the dims of frequencies 16pp .. 16pp +
+// 15, rotates and splits them and multiplies them by the query; the four frequency ranges' scores are
+// added last. The other shapes walk a serial chain of up to 32 chunks with two barriers per four;
+// here it is R / 256 chunks without any. R(p) = R(16T) R(n) as there.
+// Bound: latency, then the basis from L2 (256 KB per 32 tokens and head at R = 1024), which is why
+// larger calls keep the staged shapes.
+constexpr int JF_TOK = 32;
+
+template <int DT, int MODE, int ODT>
+__global__ __launch_bounds__(JTHREADS, 1) void joint_scores_few_kernel(JScoresParams p) {
+  __shared__ __attribute__((aligned(16))) dkv_f32x4 sAcc[JWAVES][16][64];
+  __shared__ __attribute__((aligned(16))) dkv_f32x4 sSc[JWAVES][64];
+  __shared__ __attribute__((aligned(16))) uint32_t sQ[16 * 64];  // as the sorted kernel's
+  __shared__ int sLen[JF_TOK];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int n = lane & 15, g = lane >> 4;
+  const int s0 = blockIdx.x * JF_TOK, h = blockIdx.y, b = blockIdx.z;
+
+  int tlen[2], toff[2];
+#pragma unroll
+  for (int cb = 0; cb < 2; ++cb) {
+    const int t = s0 + 16 * cb + n, tc = min(t, p.S - 1);
+    const int l = p.lens[(long long)b * p.lens_sb + (long long)tc * p.lens_ss];
+    toff[cb] = p.offs[(long long)b * p.offs_sb + (long long)tc * p.offs_ss];
+    tlen[cb] = t < p.S ? min(max(l, 0), p.R) : 0;
+  }
+  // this wave's share of the epilogue: token block tb, frequencies 16pp + 4g .. + 3
+  const int tb = wave >> 2, pp = wave & 3;
+  const int T = min((s0 >> 4) + tb, p.rope_tiles - 1);
+  const float* rd = p.rope + n * 128 + 2 * (16 * pp + 4 * g);
+  const float* rt = p.rope + (long long)(JROPE_FIXED + T) * 128 + 2 * (16 * pp + 4 * g);
+  const dkv_f32x4 d0 = *(const dkv_f32x4*)rd, d1 = *(const dkv_f32x4*)(rd + 4);
+  const dkv_f32x4 t0 = *(const dkv_f32x4*)rt, t1 = *(const dkv_f32x4*)(rt + 4);
+  if (wave == JWAVES - 1) {  // the wave with the fewest chunks forms the query operand
+    uint32_t qh[8];
+    const long long qo = (long long)b * p.q_sb + (long long)h * p.hpg * p.q_sh + lane;
+#pragma unroll
+    for (int hh = 0; hh < 8; ++hh) {
+      const long long o = qo + (hh < p.hpg ? hh : 0) * p.q_sh;
+      qh[hh] = (uint32_t)p.q[o] | ((uint32_t)p.q[o + 64] << 16);
+    }
+#pragma unroll
+    for (int hh = 0; hh < 8; ++hh)
+      if (hh < p.hpg) {
+        uint32_t hi, lo;
+        dkv_split_bf16x2(dkv_elt_to_f32<DT>(qh[hh] & 0xffffu) * p.scale,
+                         dkv_elt_to_f32<DT>(qh[hh] >> 16) * p.scale, hi, lo);
+        sQ[hh * 64 + 4 * ((lane >> 2) ^ hh) + (lane & 3)] = hi;
+        sQ[(8 + hh) * 64 + 4 * ((lane >> 2) ^ (8 + hh)) + (lane & 3)] = lo;
+      }
+  }
+  if (wave == 0 && g == 0) {
+    sLen[n] = tlen[0];
+    sLen[16 + n] = tlen[1];
+  }
+  const int maxlen = (int)dkv_wave_max_fast((float)max(tlen[0], tlen[1]));  // every wave's alike
+  const int nch = __builtin_amdgcn_readfirstlane((maxlen + JCH - 1) / JCH);
+  const int per = max(1, (nch + JWAVES - 1) / JWAVES);
+  const int c_begin = wave * per, c_end = min(nch, c_begin + per);
+
+  const uint32_t end = (uint32_t)dkv_flat_tail_elems(p.B, b, p.flat_ld, JFLAT_CAP);
+  const __amdgpu_buffer_rsrc_t rs = dkv_make_rsrc(p.flat + (long long)b * p.flat_ld, end * 2u);
+  const uint16_t* bsrc = p.bt + (long long)h * p.bt_sh + n * JCH + 8 * g;
+
+  dkv_f32x4 acc[2][8];
+#pragma unroll
+  for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) acc[cb][i] = dkv_f32x4{0.f, 0.f, 0.f, 0.f};
+  auto rank_loop = [&](auto safe_tag) {
+    constexpr bool SAFE = decltype(safe_tag)::value;
+    dkv_u32x4 a[2][8], x[2][2];
+    auto load = [&](int c, int k) {
+      if (c >= c_end) return;
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb) {
+        const int j0 = JCH * c + 8 * g;
+        if constexpr (SAFE)
+          x[k][cb] = dkv_load8_safe(rs, end, toff[cb] + j0, tlen[cb] - j0);
+        else
+          x[k][cb] = dkv_load8_raw(rs, toff[cb] + j0, tlen[cb] - j0);
+      }
+#pragma unroll
+      for (int blk = 0; blk < 8; ++blk)
+        a[k][blk] = *(const dkv_u32x4*)(bsrc + (long long)c * p.bt_sc + 16 * blk * JCH);
+    };
+    auto mul = [&](int c, int k) {
+      if (c >= c_end) return;
+#pragma unroll
+      for (int cb = 0; cb < 2; ++cb) {
+        const dkv_u32x4 xm = dkv_mask8(x[k][cb], tlen[cb] - (JCH * c + 8 * g));
+#pragma unroll
+        for (int blk = 0; blk < 8; ++blk) acc[cb][blk] = dkv_mfma32<DT>(a[k][blk], xm, acc[cb][blk]);
+      }
+    };
+    load(c_begin, 0);
+    for (int c = c_begin; c < c_end; c += 2) {
+      load(c + 1, 1);
+      mul(c, 0);
+      load(c + 2, 0);
+      mul(c + 1, 1);
+    }
+  };
+  if (b == p.B - 1)
+    rank_loop(std::integral_constant<bool, true>{});
+  else
+    rank_loop(std::integral_constant<bool, false>{});
+#pragma unroll
+  for (int cb = 0; cb < 2; ++cb)
+#pragma unroll
+    for (int blk = 0; blk < 8; ++blk) sAcc[wave][8 * cb + blk][lane] = acc[cb][blk];
+  __syncthreads();
+
+  // dims 16pp + 4g + u and 64 + the same of the lane's token: the parts added in rank order
+  dkv_f32x4 k0 = {0.f, 0.f, 0.f, 0.f}, k1 = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int w = 0; w < JWAVES; ++w) {
+    k0 += sAcc[w][8 * tb + pp][lane];
+    k1 += sAcc[w][8 * tb + pp + 4][lane];
+  }
+  const int hn = n & 7;
+  const int qrow = (n & 8) + (hn < p.hpg ? hn : hn % p.hpg);
+  const dkv_u32x4 bq = *(const dkv_u32x4*)&sQ[qrow * 64 + 4 * ((4 * pp + g) ^ qrow)];
+  const float cn[4] = {d0.x, d0.z, d1.x, d1.z}, sn[4] = {d0.y, d0.w, d1.y, d1.w};
+  const float ct[4] = {t0.x, t0.z, t1.x, t1.z}, st[4] = {t0.y, t0.w, t1.y, t1.w};
+  uint32_t kh[4], kl[4];
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    const float c = ct[w] * cn[w] - st[w] * sn[w], s = st[w] * cn[w] + ct[w] * sn[w];
+    dkv_split_bf16x2(k0[w] * c - k1[w] * s, k1[w] * c + k0[w] * s, kh[w], kl[w]);
+  }
+  dkv_f32x4 sc = {0.f, 0.f, 0.f, 0.f};
+  sc = mfma_bf16x32(dkv_u32x4{kh[0], kh[1], kh[2], kh[3]}, bq, sc);
+  sc = mfma_bf16x32(dkv_u32x4{kl[0], kl[1], kl[2], kl[3]}, bq, sc);
+  sSc[wave][lane] = sc;
+  __syncthreads();
+  if (wave >= 2) return;
+  sc = ((sSc[4 * wave][lane] + sSc[4 * wave + 1][lane]) + sSc[4 * wave + 2][lane]) +
+       sSc[4 * wave + 3][lane];
+  // column n += column n + 8 (the lo part of head n) within each row of 16 lanes
+#pragma unroll
+  for (int u = 0; u < 4; ++u)
+    sc[u] += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sc[u]),
+                                                        DKV_DPP_ROW_SHL8, 0xf, 0xf, false));
+  if (n < p.hpg) {
+    const long long ob = (long long)b * p.out_sb + (long long)(h * p.hpg + n) * p.out_sh;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int r = 16 * wave + 4 * g + u, t = s0 + r;
+      if (t < p.S) {
+        const float masked = MODE == 0 ? -1.0e4f * p.scale : -INFINITY;
+        dkv_store_f32<ODT>(p.out, ob + (long long)t * p.out_ss, sLen[r] > 0 ? sc[u] : masked);
       }
     }
   }
@@ -1057,7 +1221,13 @@ extern "C" int dkv_joint_scores(void* stream, int mode, int dtype, int out_dtype
   const long long n_wg = (long long)p.nwin * (p.win / tok) * (n_basis / nhb) * B;
   if (n_wg > 0x7fffffffLL) return DKV_E_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
-  {
+  // up to two rounds of 32-token workgroups, the ranks split over the waves and no sort.
+  // Graph-replayed us of the whole call, that shape / the better of the others: 1 x 100 tokens (32
+  // workgroups) 25.3 / 38.2, 2 x 411 (208) 30.6 / 48.5, 1 x 1000 (256) 32.6 / 52.7, 1 x 2048 (512)
+  // 46.3 / 62.2; 4 x 1000 (1024) 63.2 / 59.1, 2 x 4096 (2048) 101 / 74.8.
+  const bool tiny = B <= 65535 && n_basis <= 65535 &&
+                    (long long)B * ((S + JF_TOK - 1) / JF_TOK) * n_basis <= 512;
+  if (!tiny) {
     JSortParams sp;
     sp.lens = lens;
     sp.lens_sb = lens_sb;
@@ -1077,7 +1247,12 @@ extern "C" int dkv_joint_scores(void* stream, int mode, int dtype, int out_dtype
   const dim3 grid((unsigned)n_wg);
 #define DKV_JS_LAUNCH(DT_, MODE_, ODT_)                                                        \
   do {                                                                                         \
-    if (few)                                                                                   \
+    if (tiny)                                                                                  \
+      hipLaunchKernelGGL((joint_scores_few_kernel<DT_, MODE_, ODT_>),                          \
+                         dim3((unsigned)((S + JF_TOK - 1) / JF_TOK), (unsigned)n_basis,        \
+                              (unsigned)B),                                                    \
+                         dim3(JTHREADS), 0, st, p);                                            \
+    else if (few)                                                                              \
       hipLaunchKernelGGL((joint_scores_sorted_kernel<DT_, MODE_, ODT_, 1, 1, 4>), grid,        \
                          dim3(JTHREADS), 0, st, p);                                            \
     else if (nhb == 2)                                                                         \

@@ -1,6 +1,7 @@
-"""The joint scores' two launch shapes (few workgroups: 128 tokens of one basis head each; else 256
-of two or 512 of one) on both sides of their boundary: against the vector kernel with the bounds of
-the other scores tests, and a batch row's scores the same bits from either shape."""
+"""The joint scores' launch shapes (32 tokens of one basis head with the ranks split over the waves,
+128 of one head, else 256 of two or 512 of one) on both sides of their boundaries: against the
+vector kernel with the bounds of the other scores tests, and a batch row's scores from the shapes
+that sum the ranks in one order the same bits."""
 import pytest
 import torch
 
@@ -11,6 +12,7 @@ from test_gpu_joint import THETA, ULP, _case, _dev, _generic_scores
 # (B, S, R, n_basis, Hq): 128 and 130 workgroups of two heads, 129 of one head, tokens one past a
 # 128-token range, one chunk, five chunks (a remainder of the four-chunk loop)
 CASES = [
+    (8, 1025, 64, 2, 8),
     (64, 129, 64, 2, 8),
     (65, 129, 64, 2, 8),
     (43, 513, 160, 3, 12),
@@ -35,7 +37,47 @@ def test_scores_launch_shapes(dev, i, dtype):
         err = (got.float()[fin] - ref[fin]).abs()
         tol = (2 * ULP[dtype] if mode == 0 else 1e-4) * ref[fin].abs() + 1e-4
         assert (err <= tol).all(), float(err.max())
-        for b in (0, B - 1):  # one row alone: always the small shape
-            one = J.joint_scores(d["q"][b:b + 1], d["kb"], d["fk"][b:b + 1], d["lk"][b:b + 1],
-                                 d["ok"][b:b + 1], **kw)
-            assert torch.equal(one[0], got[b])
+        half = (B + 1) // 2
+        if _wg32(B // 2, S, nb) > 512:  # half the rows: the 128-token shape beside the large one
+            rows = slice(0, half)
+            part = J.joint_scores(d["q"][rows], d["kb"], d["fk"][rows], d["lk"][rows],
+                                  d["ok"][rows], **kw)
+            assert torch.equal(part, got[rows])
+
+
+def _wg32(B, S, nb):
+    return B * ((S + 31) // 32) * nb
+
+
+# (B, S, R, n_basis, Hq): the 32-token shape up to 512 workgroups: fewer chunks than waves, chunks
+# that do not divide among them, a last block of one token, 1 to 8 query heads per basis
+FEW = [
+    (1, 1, 32, 1, 8),
+    (2, 33, 96, 8, 32),
+    (1, 17, 1024, 8, 32),
+    (3, 65, 288, 3, 24),
+    (1, 2048, 512, 8, 8),
+    (16, 512, 128, 2, 4),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("i", range(len(FEW)))
+def test_scores_of_few_tokens(dev, i, dtype):
+    B, S, R, nb, Hq = FEW[i]
+    assert _wg32(B, S, nb) <= 512
+    print(f"[gpu] joint scores few tokens {FEW[i]} {dtype}", flush=True)
+    d = _dev(_case(B, S, R, nb, Hq=Hq, dtype=dtype, seed=600 + i, exact_end=True), dev, dtype)
+    for mode, odt in ((0, dtype), (1, torch.float32)):
+        got = J.joint_scores(d["q"], d["kb"], d["fk"], d["lk"], d["ok"], theta=THETA, mode=mode,
+                             out_dtype=odt).float()
+        ref = _generic_scores(d, d["kb"], mode, odt).float()
+        fin = torch.isfinite(ref)
+        assert torch.equal(torch.isfinite(got), fin)
+        err = (got[fin] - ref[fin]).abs()
+        tol = (2 * ULP[dtype] if mode == 0 else 1e-4) * ref[fin].abs() + 1e-4
+        assert (err <= tol).all(), float(err.max())
+        if mode == 0:
+            masked = (d["lk"] == 0)[:, None, :]
+            assert torch.equal(got.masked_select(masked), ref.masked_select(masked))
