@@ -37,8 +37,8 @@
 // joint_merge_kernel -- workgroup = (rank block of 128, V basis and up to 8 of its query heads,
 //   batch row b): LSE weights of the split records with the route's denominator, the block's
 //   merged coefficients, their projection through the block's basis rows (each basis value
-//   loaded once for the group's heads); joint_project_sum_kernel adds the blocks' partial
-//   projections and rounds the output.
+//   loaded once for the group's heads); the last of a group's blocks to arrive adds the partial
+//   projections in block order and rounds the output.
 #include <type_traits>
 
 #include "dkv_common.h"
@@ -53,7 +53,9 @@ constexpr int JCB = 4;                   // 16-token column blocks per wave (sco
 constexpr int JTOK = JWAVES * JCB * 16;  // tokens per scores workgroup
 constexpr int JCH = 32;                  // ranks per basis chunk
 constexpr int JRMAX = 1024;
-constexpr int JPREC = 4 + JRMAX;         // split record: m (log2 units), l, 2 unused, acc[R]
+// split record: m (log2 units), l, the merge's arrival count (split 0 of a group's first head; an
+// int, zeroed by the V pass), 1 unused, acc[R]
+constexpr int JPREC = 4 + JRMAX;
 constexpr int JRB = 128;                 // ranks per merge workgroup
 constexpr int JROPE_FIXED = 17;          // rows of the RoPE table before the per-tile rows
 constexpr int JFLAT_CAP = DKV_FLAT_RSRC_CAP;  // elements one buffer resource covers
@@ -944,6 +946,7 @@ __global__ __launch_bounds__(JTHREADS, 1) void joint_av_kernel(JAvParams p) {
       float* rec = p.rec + (((long long)b * p.Hq + hq[hs]) * p.n_splits + split) * JPREC;
       rec[0] = m_run[hs];
       rec[1] = l_tot;
+      rec[2] = 0.f;  // the merge's arrival count (the bits of int 0)
     }
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
@@ -961,13 +964,13 @@ __global__ __launch_bounds__(JTHREADS, 1) void joint_av_kernel(JAvParams p) {
 }
 
 struct JMergeParams {
-  const float* rec;
+  float* rec;
   float* part;  // [B][Hq][R/128 rank blocks][Dh] partial projections
   const uint16_t* vb;  // V basis [n_basis][R][Dh] with strides (vb_sh, vb_sr)
   long long vb_sh, vb_sr;
   void* out;
   long long out_sb, out_sh;
-  int Hq, R, n_splits, hpg, n_rb;
+  int Hq, R, n_splits, hpg, n_rb, out_dtype;
 };
 
 // workgroup = (rank block of 128, V basis hv and up to NH of its query heads, batch row b): the
@@ -1106,22 +1109,41 @@ __global__ __launch_bounds__(256) void joint_merge_kernel(JMergeParams p) {
     sOut[rq][j][2 * dp + 1] = o1[j];
   }
   __syncthreads();
+  // The block's partial projections, and the sum over the blocks by the last of the group's
+  // workgroups to arrive: coherent stores, each wave waits for its own, one thread counts the
+  // arrival (relaxed device-scope accesses, as the split kernel exchanges its records).
   for (int i = tid; i < nh * JDH; i += 256) {
     const int j = i / JDH, d = i % JDH;
-    p.part[((head0 + j) * p.n_rb + rb) * JDH + d] =
-        (sOut[0][j][d] + sOut[1][j][d]) + (sOut[2][j][d] + sOut[3][j][d]);
+    __hip_atomic_store(&p.part[((head0 + j) * p.n_rb + rb) * JDH + d],
+                       (sOut[0][j][d] + sOut[1][j][d]) + (sOut[2][j][d] + sOut[3][j][d]),
+                       __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
-}
-
-// workgroup = (query head, batch row b), thread = output dim: the sum of the rank blocks' partial
-// projections, the output rounding
-template <int ODT>
-__global__ __launch_bounds__(JDH) void joint_project_sum_kernel(JMergeParams p) {
-  const int hq = blockIdx.x, b = blockIdx.y, d = threadIdx.x;
-  const float* part = p.part + (((long long)b * p.Hq + hq) * p.n_rb) * JDH + d;
-  float o = 0.f;
-  for (int k = 0; k < p.n_rb; ++k) o += part[(long long)k * JDH];
-  dkv_store_f32<ODT>(p.out, (long long)b * p.out_sb + (long long)hq * p.out_sh + d, o);
+  __shared__ int sLast;
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (tid == 0)
+    sLast = __hip_atomic_fetch_add((int*)(p.rec + head0 * ns * JPREC + 2), 1, __ATOMIC_RELAXED,
+                                   __HIP_MEMORY_SCOPE_AGENT) == p.n_rb - 1;
+  __syncthreads();
+  if (!sLast) return;
+  for (int i = tid; i < nh * JDH; i += 256) {
+    const int j = i / JDH, d = i % JDH;
+    float* part = p.part + (head0 + j) * p.n_rb * JDH + d;
+    float v[JRMAX / JRB], o = 0.f;
+#pragma unroll
+    for (int k = 0; k < JRMAX / JRB; ++k)  // all in flight at once; blocks past the last read it
+      v[k] = __hip_atomic_load(part + (long long)min(k, p.n_rb - 1) * JDH, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+    for (int k = 0; k < JRMAX / JRB; ++k) o += k < p.n_rb ? v[k] : 0.f;
+    const long long oi = (long long)b * p.out_sb + (long long)(hv * p.hpg + j0 + j) * p.out_sh + d;
+    if (p.out_dtype == DKV_BF16)
+      dkv_store_f32<DKV_BF16>(p.out, oi, o);
+    else if (p.out_dtype == DKV_F16)
+      dkv_store_f32<DKV_F16>(p.out, oi, o);
+    else
+      dkv_store_f32<DKV_F32>(p.out, oi, o);
+  }
 }
 
 // sets of 16 query heads per V-pass workgroup: two when the sets pair up
@@ -1390,6 +1412,7 @@ extern "C" int dkv_joint_av(void* stream, int mode, int scores_dtype, int dtype,
   const int hpg = Hq / n_basis;
   m.hpg = hpg;
   m.n_rb = n_rb;
+  m.out_dtype = out_dtype;
   const int nhm = hpg <= 4 ? 4 : 8;  // query heads merged and projected together
   const dim3 mgrid((unsigned)n_rb, (unsigned)(n_basis * ((hpg + nhm - 1) / nhm)), (unsigned)B);
   const size_t wt_bytes = sizeof(float) * nhm * (size_t)ns;
@@ -1424,14 +1447,6 @@ extern "C" int dkv_joint_av(void* stream, int mode, int scores_dtype, int dtype,
           hipLaunchKernelGGL((joint_merge_kernel<DKV_F16, 1, 8>), mgrid, dim3(256), wt_bytes, st, m);
       }
   }
-  DKV_HIP_CHECK_LAUNCH();
-  const dim3 pgrid((unsigned)Hq, (unsigned)B);
-  if (out_dtype == DKV_BF16)
-    hipLaunchKernelGGL((joint_project_sum_kernel<DKV_BF16>), pgrid, dim3(JDH), 0, st, m);
-  else if (out_dtype == DKV_F16)
-    hipLaunchKernelGGL((joint_project_sum_kernel<DKV_F16>), pgrid, dim3(JDH), 0, st, m);
-  else
-    hipLaunchKernelGGL((joint_project_sum_kernel<DKV_F32>), pgrid, dim3(JDH), 0, st, m);
   DKV_HIP_CHECK_LAUNCH();
   return DKV_OK;
 }
