@@ -42,6 +42,9 @@ _SIGNATURES = {
                                    _vp, _ll, _ll, _vp, _ll, _ll, _vp, _ll, _vp, _vp, _ll, _ll, _vp,
                                    _vp, _ll, _ll, _vp, _ll, _ll, _vp, _ll, _vp, _vp, _ll, _ll, _vp]),
     "dkv_decompress": (_i, [_vp, _i, _vp, _ll, _vp, _vp, _ll, _ll, _vp, _i, _i, _i]),
+    "dkv_decompress_kv": (_i, [_vp, _i, _vp, _ll, _vp, _vp, _ll, _ll, _vp, _vp, _ll, _vp, _vp, _ll,
+                               _ll, _vp, _i, _i, _i]),
+    "dkv_row_totals": (_i, [_vp, _vp, _ll, _ll, _vp, _ll, _ll, _i, _i, _i, _vp]),
     "dkv_scores": (_i, [_vp, _i, _i, _i, _i, _vp, _ll, _ll, _vp, _ll, _ll, _i, _vp, _ll,
                         _vp, _ll, _ll, _vp, _ll, _ll, _vp, _ll, _ll, _ll, _i, _i, _i, _i, _i, _f]),
     "dkv_av": (_i, [_vp, _i, _i, _i, _i, _vp, _ll, _ll, _ll, _vp, _ll, _ll, _i, _vp, _ll,

@@ -71,10 +71,27 @@ __global__ __launch_bounds__(256) void append_decode_kv_kernel(AppendSlot k, App
 // Prefill append, workgroup (row, chunk): AP_CHUNK tokens of one row. The row's offsets before
 // the chunk come from a reduction over the earlier tokens' counts (every workgroup reads the
 // row's old pointer, so the pointer itself is advanced by append_prefill_ptr_kernel, launched
-// after); wave 0 scans the chunk, then each wave copies its tokens four at a time (all loads
-// of a group issued before its stores). Offsets follow the unclipped counts, the coefficients
-// are stored at the clipped ones (min(len, max_dim)), as in the one-token append.
+// after); wave 0 scans the chunk, then the copies: 16 lanes per token, 16 bytes per lane and step
+// (the stores fall on element boundaries, which the hardware takes), a piece that a count ends in
+// element by element. Offsets follow the unclipped counts, the coefficients are stored at the
+// clipped ones (min(len, max_dim)), as in the one-token append.
 constexpr int AP_CHUNK = 64;
+
+// 16 bytes of elements on an element boundary
+typedef __attribute__((ext_vector_type(4), aligned(2))) uint32_t piece_t;
+
+// v with the elements from index k on cleared (k <= 0: all)
+template <typename T>
+__device__ __forceinline__ dkv_u32x4 keep_first(dkv_u32x4 v, int k) {
+#pragma unroll
+  for (int d = 0; d < 4; ++d) {
+    if constexpr (sizeof(T) == 4)
+      v[d] = d < k ? v[d] : 0u;
+    else
+      v[d] &= k >= 2 * d + 2 ? 0xffffffffu : (k == 2 * d + 1 ? 0xffffu : 0u);
+  }
+  return v;
+}
 // one slot (K or V cache of a layer) of a prefill append
 struct PrefillSlot {
   const void* states;
@@ -155,36 +172,67 @@ __global__ __launch_bounds__(256) void append_prefill_kernel(PrefillSlot s0, Pre
   T* frow = flat + (long long)row * flat_ld;
   const T* srow = states + (long long)row * states_sb;
   const int nt = min(AP_CHUNK, n_new - c0);
-  for (int t0 = 4 * wave; t0 < nt; t0 += 16) {
-    // tokens t0 .. t0+3 of the chunk: lane j copies element j (and j + 64) of each
-    T v[4][2];
+  constexpr int PE = 16 / sizeof(T);  // elements per piece
+  const int sub = lane >> 4, j = lane & 15;
+  for (int t0 = 4 * wave; t0 < nt; t0 += 32) {
+    // tokens t0 + sub and t0 + 16 + sub of the chunk, both loaded before either is stored
+    dkv_u32x4 v[2];
+    int c[2];
+    const T* src[2];
+    T* dst[2];
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int tt = t0 + u;
-      const int c = tt < nt ? s_clen[tt] : 0;
-      const T* src = srow + (long long)(c0 + tt) * states_ss;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) v[u][h] = lane + 64 * h < c ? src[lane + 64 * h] : T(0);
+    for (int u = 0; u < 2; ++u) {
+      const int tt = t0 + 16 * u + sub;
+      c[u] = tt < nt ? s_clen[tt] : 0;
+      src[u] = srow + (long long)(c0 + min(tt, nt - 1)) * states_ss;
+      dst[u] = frow + s_dst[min(tt, nt - 1)];
+      if (PE * j + PE <= c[u]) v[u] = *(const piece_t*)(src[u] + PE * j);
     }
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int tt = t0 + u;
-      const int c = tt < nt ? s_clen[tt] : 0;
-      T* dst = frow + s_dst[tt < nt ? tt : 0];
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-        if (lane + 64 * h < c) dst[lane + 64 * h] = v[u][h];
-    }
-    // counts above 128 (max_dim past the per-head rank): the rest element by element
-    for (int u = 0; u < 4; ++u) {
-      const int tt = t0 + u;
-      if (tt >= nt) break;
-      const int c = s_clen[tt];
-      const T* src = srow + (long long)(c0 + tt) * states_ss;
-      T* dst = frow + s_dst[tt];
-      for (int j = 128 + lane; j < c; j += 64) dst[j] = src[j];
+    for (int u = 0; u < 2; ++u) {
+      if (PE * j + PE <= c[u])
+        *(piece_t*)(dst[u] + PE * j) = v[u];
+      else
+        for (int e = PE * j; e < min(c[u], PE * j + PE); ++e) dst[u][e] = src[u][e];
+      // counts past 16 pieces
+      for (int q = PE * (j + 16); q < c[u]; q += PE * 16) {
+        if (q + PE <= c[u])
+          *(piece_t*)(dst[u] + q) = *(const piece_t*)(src[u] + q);
+        else
+          for (int e = q; e < c[u]; ++e) dst[u][e] = src[u][e];
+      }
     }
   }
+}
+
+// Per slot (blockIdx.y: K, V) and row: out[0][slot][row] the summed counts of the row's n tokens (they
+// size a new slot's buffer) and out[1][slot][row] the sum of the clipped ones (its pointer after the
+// append).
+__global__ __launch_bounds__(256) void row_totals_kernel(PrefillSlot s0, PrefillSlot s1,
+                                                         int n_new, int max_dim,
+                                                         long long* __restrict__ out) {
+  const PrefillSlot& sl = blockIdx.y ? s1 : s0;
+  __shared__ long long s_red[2][4];
+  const int row = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  long long pu = 0, pc = 0;
+  for (int t = tid; t < n_new; t += 256) {
+    const int len = sl.new_len[(long long)row * sl.len_sb + (long long)t * sl.len_ss];
+    pu += len;
+    pc += max(0, min(len, max_dim));
+  }
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) {
+    pu += __shfl_xor(pu, o, 64);
+    pc += __shfl_xor(pc, o, 64);
+  }
+  if (lane == 0) {
+    s_red[0][wave] = pu;
+    s_red[1][wave] = pc;
+  }
+  __syncthreads();
+  if (tid < 2)
+    out[((long long)tid * gridDim.y + blockIdx.y) * gridDim.x + row] =
+        s_red[tid][0] + s_red[tid][1] + s_red[tid][2] + s_red[tid][3];
 }
 
 // ptr[row] += sum over the appended tokens of min(len, max_dim)
@@ -206,24 +254,48 @@ __global__ __launch_bounds__(256) void append_prefill_ptr_kernel(PrefillSlot s0,
   if (tid == 0) ptr[row] = (int)(ptr[row] + s_red[0] + s_red[1] + s_red[2] + s_red[3]);
 }
 
-// out[b, t, j] = flat[b, offs[b,t] + j] for j < min(lens, max_dim), else 0.
-template <typename T>
-__global__ __launch_bounds__(256) void decompress_kernel(const T* __restrict__ flat,
-                                                         long long flat_ld,
-                                                         const int* __restrict__ lens,
-                                                         const int* __restrict__ offs,
-                                                         long long tab_sb, long long tab_ss,
-                                                         T* __restrict__ out, int seq,
+struct ExpandSlot {
+  const void* flat;
+  long long flat_ld;
+  const int* lens;
+  const int* offs;
+  long long tab_sb, tab_ss;
+  void* out;
+};
+
+// out[b, t, j] = flat[b, offs[b,t] + j] for j < min(lens, max_dim), else 0. Workgroup = (16 tokens,
+// row, slot): 16 lanes per token, 16 bytes per lane and step; a piece that the row's end cuts, or
+// that starts past the count, is not read whole. VEC: the output rows are whole 16-byte pieces on
+// 16-byte boundaries (else element stores).
+template <typename T, bool VEC>
+__global__ __launch_bounds__(256) void decompress_kernel(ExpandSlot s0, ExpandSlot s1, int seq,
                                                          int max_dim) {
-  const int row = blockIdx.y;
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+  constexpr int PE = 16 / sizeof(T);
+  const ExpandSlot& sl = blockIdx.z ? s1 : s0;
+  const int row = blockIdx.y, t = blockIdx.x * 16 + (threadIdx.x >> 4), j = threadIdx.x & 15;
   if (t >= seq) return;
-  const int lane = threadIdx.x & 63;
-  const long long ti = (long long)row * tab_sb + (long long)t * tab_ss;
-  const int n = max(0, min(lens[ti], max_dim));
-  const T* src = flat + (long long)row * flat_ld + offs[ti];
-  T* dst = out + ((long long)row * seq + t) * max_dim;
-  for (int j = lane; j < max_dim; j += 64) dst[j] = j < n ? src[j] : (T)0;
+  const long long ti = (long long)row * sl.tab_sb + (long long)t * sl.tab_ss;
+  const int n = max(0, min(sl.lens[ti], max_dim)), off = sl.offs[ti];
+  const T* src = (const T*)sl.flat + (long long)row * sl.flat_ld + off;
+  T* dst = (T*)sl.out + ((long long)row * seq + t) * max_dim;
+  for (int q = PE * j; q < max_dim; q += PE * 16) {
+    dkv_u32x4 v = {0u, 0u, 0u, 0u};
+    if (q < n && (long long)off + q + PE <= sl.flat_ld) {
+      v = keep_first<T>(*(const piece_t*)(src + q), n - q);
+    } else {
+      // past the count, or the last elements of the row
+#pragma unroll
+      for (int e = 0; e < PE; ++e)
+        if (q + e < n) v[e * sizeof(T) / 4] |= (uint32_t)src[q + e] << (8 * (e * sizeof(T) % 4));
+    }
+    if constexpr (VEC) {
+      *(dkv_u32x4*)(dst + q) = v;
+    } else {
+#pragma unroll
+      for (int e = 0; e < PE; ++e)
+        if (q + e < max_dim) dst[q + e] = (T)(v[e * sizeof(T) / 4] >> (8 * (e * sizeof(T) % 4)));
+    }
+  }
 }
 
 }  // namespace
@@ -361,23 +433,65 @@ extern "C" int dkv_append_prefill_kv(
   return append_prefill_launch(stream, dtype, k, v, 2, seq_pos, rows, n_new, max_dim);
 }
 
-extern "C" int dkv_decompress(void* stream, int dtype, const void* flat, long long flat_ld,
-                              const int* lens, const int* offs, long long tab_sb,
-                              long long tab_ss, void* out, int rows, int seq, int max_dim) {
+extern "C" int dkv_row_totals(void* stream, const int* len_k, long long len_k_sb,
+                              long long len_k_ss, const int* len_v, long long len_v_sb,
+                              long long len_v_ss, int rows, int n_new, int max_dim,
+                              long long* out) {
+  if (rows < 0 || n_new < 0 || max_dim < 0) return DKV_E_ARG;
+  if (rows == 0) return DKV_OK;
+  if (!out || (n_new > 0 && (!len_k || !len_v))) return DKV_E_ARG;
+  PrefillSlot k{}, v{};
+  k.new_len = len_k;
+  k.len_sb = len_k_sb;
+  k.len_ss = len_k_ss;
+  v.new_len = len_v;
+  v.len_sb = len_v_sb;
+  v.len_ss = len_v_ss;
+  hipLaunchKernelGGL(row_totals_kernel, dim3((unsigned)rows, 2), dim3(256), 0, (hipStream_t)stream,
+                     k, v, n_new, max_dim, out);
+  DKV_HIP_CHECK_LAUNCH();
+  return DKV_OK;
+}
+
+static int decompress_launch(void* stream, int dtype, const ExpandSlot& k, const ExpandSlot& v,
+                             int nslots, int rows, int seq, int max_dim) {
   if (rows < 0 || seq < 0 || max_dim < 0) return DKV_E_ARG;
   if (rows == 0 || seq == 0 || max_dim == 0) return DKV_OK;
-  if (!flat || !lens || !offs || !out) return DKV_E_ARG;
+  if (!k.flat || !k.lens || !k.offs || !k.out || !v.flat || !v.lens || !v.offs || !v.out)
+    return DKV_E_ARG;
   const int es = dkv_elt_size(dtype);
   if (es == 0) return DKV_E_ARG;
   if (rows > 65535) return DKV_E_UNSUPPORTED;
-  dim3 grid((seq + 3) / 4, rows), block(256);
+  const dim3 grid((unsigned)((seq + 15) / 16), (unsigned)rows, (unsigned)nslots), block(256);
   hipStream_t s = (hipStream_t)stream;
-  if (es == 4)
-    hipLaunchKernelGGL(decompress_kernel<uint32_t>, grid, block, 0, s, (const uint32_t*)flat,
-                       flat_ld, lens, offs, tab_sb, tab_ss, (uint32_t*)out, seq, max_dim);
+  const bool vec = (long long)max_dim * es % 16 == 0 &&
+                   ((uintptr_t)k.out | (uintptr_t)v.out) % 16 == 0;
+  if (es == 4 && vec)
+    hipLaunchKernelGGL((decompress_kernel<uint32_t, true>), grid, block, 0, s, k, v, seq, max_dim);
+  else if (es == 4)
+    hipLaunchKernelGGL((decompress_kernel<uint32_t, false>), grid, block, 0, s, k, v, seq, max_dim);
+  else if (vec)
+    hipLaunchKernelGGL((decompress_kernel<uint16_t, true>), grid, block, 0, s, k, v, seq, max_dim);
   else
-    hipLaunchKernelGGL(decompress_kernel<uint16_t>, grid, block, 0, s, (const uint16_t*)flat,
-                       flat_ld, lens, offs, tab_sb, tab_ss, (uint16_t*)out, seq, max_dim);
+    hipLaunchKernelGGL((decompress_kernel<uint16_t, false>), grid, block, 0, s, k, v, seq, max_dim);
   DKV_HIP_CHECK_LAUNCH();
   return DKV_OK;
+}
+
+extern "C" int dkv_decompress(void* stream, int dtype, const void* flat, long long flat_ld,
+                              const int* lens, const int* offs, long long tab_sb,
+                              long long tab_ss, void* out, int rows, int seq, int max_dim) {
+  const ExpandSlot k{flat, flat_ld, lens, offs, tab_sb, tab_ss, out};
+  return decompress_launch(stream, dtype, k, k, 1, rows, seq, max_dim);
+}
+
+extern "C" int dkv_decompress_kv(void* stream, int dtype, const void* flat_k, long long flat_k_ld,
+                                 const int* lens_k, const int* offs_k, long long tab_k_sb,
+                                 long long tab_k_ss, void* out_k, const void* flat_v,
+                                 long long flat_v_ld, const int* lens_v, const int* offs_v,
+                                 long long tab_v_sb, long long tab_v_ss, void* out_v, int rows,
+                                 int seq, int max_dim) {
+  const ExpandSlot k{flat_k, flat_k_ld, lens_k, offs_k, tab_k_sb, tab_k_ss, out_k};
+  const ExpandSlot v{flat_v, flat_v_ld, lens_v, offs_v, tab_v_sb, tab_v_ss, out_v};
+  return decompress_launch(stream, dtype, k, v, 2, rows, seq, max_dim);
 }

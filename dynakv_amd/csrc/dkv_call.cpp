@@ -74,6 +74,8 @@ PyMethodDef methods[] = {
     DKV_CALL(dkv_append_prefill),
     DKV_CALL(dkv_append_prefill_kv),
     DKV_CALL(dkv_decompress),
+    DKV_CALL(dkv_decompress_kv),
+    DKV_CALL(dkv_row_totals),
     DKV_CALL(dkv_scores),
     DKV_CALL(dkv_av),
     DKV_CALL(dkv_joint_scores),

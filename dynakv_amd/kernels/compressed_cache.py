@@ -93,7 +93,20 @@ class CustomDynamicCache(_CacheBase):
         """Dense ``(rows, seq, max_dim)`` K and V coefficients (reference :70-81)."""
         c_k = self.key_cache_sp[layer_idx]
         c_v = self.value_cache_sp[layer_idx]
-        return self._decompress(c_k, max_dim), self._decompress(c_v, max_dim)
+        fk, fv, seq = c_k[0], c_v[0], c_k[4]
+        rows = fk.shape[0]
+        if (rows == 0 or seq == 0 or c_v[4] != seq or fv.shape[0] != rows or fv.dtype != fk.dtype
+                or fv.device != fk.device):
+            return self._decompress(c_k, max_dim), self._decompress(c_v, max_dim)
+        ok = fk.new_empty(rows, seq, max_dim)
+        ov = fv.new_empty(rows, seq, max_dim)
+        tk, tv = c_k[1].stride(), c_v[1].stride()
+        _lib.check(_lib.calls().dkv_decompress_kv(
+            _lib.stream_of(fk), _lib.dtype_code(fk.dtype), fk.data_ptr(), fk.stride(0),
+            c_k[1].data_ptr(), c_k[2].data_ptr(), tk[0], tk[1], ok.data_ptr(),
+            fv.data_ptr(), fv.stride(0), c_v[1].data_ptr(), c_v[2].data_ptr(), tv[0], tv[1],
+            ov.data_ptr(), rows, seq, max_dim), "dkv_decompress_kv")
+        return ok, ov
 
     def reset(self):
         self.key_cache_sp = []
@@ -258,7 +271,15 @@ class CustomDynamicCache(_CacheBase):
             raise ValueError("update_sp_prefill_many takes prefill appends (S > 1)")
         # per slot and row: the summed counts (buffer sizing) and the clipped sums (the row's
         # pointer after the append, for a slot that starts empty), in one transfer
-        if len({tuple(l.shape) for l in lens}) == 1:
+        if len(lens) == 2 and self._totals_ok(lens[0], lens[1]):
+            kl, vl = lens
+            tot = torch.empty((2, 2, kl.shape[0]), dtype=torch.int64, device=kl.device)
+            _lib.check(_lib.calls().dkv_row_totals(
+                _lib.stream_of(kl), kl.data_ptr(), kl.stride(0), kl.stride(1), vl.data_ptr(),
+                vl.stride(0), vl.stride(1), kl.shape[0], kl.shape[1], max_dim, tot.data_ptr()),
+                "dkv_row_totals")
+            host = tot.flatten().tolist()
+        elif len({tuple(l.shape) for l in lens}) == 1:
             L = torch.stack(lens)  # one reduction over every slot instead of one per slot
             host = torch.cat([L.sum(dim=2).flatten(),
                               L.clamp(0, max_dim).sum(dim=2).flatten()]).tolist()
@@ -286,6 +307,12 @@ class CustomDynamicCache(_CacheBase):
             self._launch_prefill_pair(ck, kst, kln, kub, cv, vst, vln, vub, max_dim)
             self._finish_slot(ck, kln.shape[1], kadd, False)
             self._finish_slot(cv, vln.shape[1], vadd, False)
+
+    @staticmethod
+    def _totals_ok(kl: torch.Tensor, vl: torch.Tensor) -> bool:
+        """Counts that ``dkv_row_totals`` takes: int32 on one GPU, one shape, some row."""
+        return (kl.is_cuda and vl.device == kl.device and kl.dtype == vl.dtype == torch.int32
+                and kl.shape == vl.shape and kl.dim() == 2 and kl.shape[0] > 0)
 
     def _create_fresh_slots(self, items, lens, host, starts):
         """The slots of ``items`` that do not exist yet, created as ``_prepare_slot`` creates
@@ -365,6 +392,10 @@ class CustomDynamicCache(_CacheBase):
                 _lib.check(rc, "dkv_append_decode_kv")
             self._finish_slot(ck, key_len.shape[1], add_k, True)
             self._finish_slot(cv, value_len.shape[1], add_v, True)
+        elif self._totals_ok(key_len, value_len) and key_states.device == key_len.device:
+            # a prompt: one device read for both slots' sizes, one launch for both appends
+            self.update_sp_prefill_many([(layer_idx, key_states, key_len, value_states, value_len)],
+                                        tensor_d)
         else:
             self._update_layer_cache(self.key_cache_sp, layer_idx, key_states, key_len, tensor_d,
                                      is_decode=False)

@@ -148,6 +148,22 @@ int dkv_decompress(void* stream, int dtype,
                    const void* flat, long long flat_ld,
                    const int* lens, const int* offs, long long tab_sb, long long tab_ss,
                    void* out, int rows, int seq, int max_dim);
+/* The same for a layer's K and V slots in one launch (equal rows, tokens, dtype and max_dim). */
+int dkv_decompress_kv(void* stream, int dtype, const void* flat_k, long long flat_k_ld,
+                      const int* lens_k, const int* offs_k, long long tab_k_sb, long long tab_k_ss,
+                      void* out_k, const void* flat_v, long long flat_v_ld, const int* lens_v,
+                      const int* offs_v, long long tab_v_sb, long long tab_v_ss, void* out_v,
+                      int rows, int seq, int max_dim);
+
+/*
+ * Row totals of a prompt's K and V counts (rows, n_new) int32: out[0][slot][row] = sum of the counts,
+ * out[1][slot][row] = sum of min(max(count, 0), max_dim); slot 0 K, 1 V. What sizes a new slot's flat
+ * buffer and its pointers after the append (compressed_cache.py:138-168), in one launch.
+ */
+int dkv_row_totals(void* stream, const int* len_k, long long len_k_sb, long long len_k_ss,
+                   const int* len_v, long long len_v_sb, long long len_v_ss, int rows, int n_new,
+                   int max_dim, long long* out);
+
 
 /*
  * Reference-semantics QK scores (abx_sparse / _abx_sparse_fwd, reference two_stage.py:48-189).
