@@ -1155,7 +1155,12 @@ int joint_av_split_len(int B, int Hq, int S) {
   // tokens per workgroup (measured on MI355X at B = 16, S = 8192: V pass + merge 72 us with 16
   // splits of 512 tokens, 88 with 32 of 256).
   const long long units = (long long)B * ((Hq + 15) / 16 / joint_av_hsets(Hq));
-  const long long sl = dkv_rounds_split(units, S, 150, 16, 16, JMAX_SPLITS);
+  // Shortest split: 16 tokens up to 800 of them, where the V pass's own tokens are what a call
+  // waits for; above that 32, since the merge walks the splits 16 at a time (32 query heads, 8
+  // bases, whole call with 16 / 32: 1 x 100 23.8 / 26.2 us, 2 x 411 28.8 / 31.8, 2 x 615 21.8 /
+  // 23.2 with 4 bases; 1 x 1000 30.9 / 29.9, 4 x 1000 57.0 / 54.5, 1 x 4096 67.5 / 61.0; 48 and
+  // 64 gain nothing more up to 2048 tokens).
+  const long long sl = dkv_rounds_split(units, S, 150, S <= 800 ? 16 : 32, 16, JMAX_SPLITS);
   return (int)(sl < 16 ? 16 : sl);
 }
 

@@ -1,13 +1,16 @@
 """The joint scores' launch shapes (32 tokens of one basis head with the ranks split over the waves,
 128 of one head, else 256 of two or 512 of one) on both sides of their boundaries: against the
 vector kernel with the bounds of the other scores tests, and a batch row's scores from the shapes
-that sum the ranks in one order the same bits."""
+that sum the ranks in one order the same bits. The V pass on both sides of its shortest split."""
+import numpy as np
 import pytest
 import torch
 
+from dynakv_amd import _lib
 from dynakv_amd.kernels import joint as J
 
-from test_gpu_joint import THETA, ULP, _case, _dev, _generic_scores
+from helpers import assert_close, cast_np
+from test_gpu_joint import THETA, ULP, _case, _dev, _generic_av, _generic_scores
 
 # (B, S, R, n_basis, Hq): 128 and 130 workgroups of two heads, 129 of one head, tokens one past a
 # 128-token range, one chunk, five chunks (a remainder of the four-chunk loop)
@@ -81,3 +84,21 @@ def test_scores_of_few_tokens(dev, i, dtype):
         if mode == 0:
             masked = (d["lk"] == 0)[:, None, :]
             assert torch.equal(got.masked_select(masked), ref.masked_select(masked))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("S", [800, 801, 1025])  # 50 splits of 16; 26 of 32, the last of one token
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_v_pass_shortest_split(dev, S, dtype):
+    B, R, nb, Hq = 2, 160, 4, 16
+    floats = _lib.load().dkv_joint_av_workspace_floats(B, Hq, S, R)
+    assert floats == B * Hq * ({800: 50, 801: 26, 1025: 33}[S] * (4 + 1024) + 256)
+    print(f"[gpu] joint av split line S={S} {dtype}", flush=True)
+    d = _dev(_case(B, S, R, nb, Hq=Hq, dtype=dtype, seed=S, exact_end=True), dev, dtype)
+    z = cast_np(np.random.default_rng(S).standard_normal((B, Hq, S)) * 2, dtype)
+    sc = torch.from_numpy(z).to(dev, dtype)
+    got = J.joint_av(sc, d["vb"], d["fv"], d["lv"], d["ov"], mode=0, out_dtype=torch.float32)
+    ref = _generic_av(sc, d, d["vb"], 0, torch.float32)
+    # the bounds of the other V-pass tests: fp16 caches hold P in fp16, 2^-11 per term
+    assert_close(got, ref.cpu().numpy(), "av", tol_rel=2e-3,
+                 tol_abs=2e-4 if dtype == torch.bfloat16 else 1e-3)
