@@ -23,7 +23,7 @@
 //   blocks; the coefficients go straight into B operand registers (lane = one token x 8 ranks,
 //   elements past the token's count zeroed), two or four chunks ahead, each serving every head of the
 //   workgroup. Then per block: the lane's token rotated by R(p) = R(16T) R(n) (p = 16T + n, its
-//   position; composed from LDS tables) in fp32, K' split into bf16 hi + lo, scores on MFMA
+//   position; composed from the table's rows) in fp32, K' split into bf16 hi + lo, scores on MFMA
 //   against the unrotated query (hi and lo parts in separate operand columns, formed once per
 //   head), the route's masking and rounding, stored at the token's position.
 // joint_scores_few_kernel -- the scores of a short call without the pre-pass: workgroup = (32
@@ -63,8 +63,7 @@ constexpr int JMAX_SPLITS = 1024;  // token splits of the V pass
 constexpr float JLOG2E = 1.4426950408889634f;
 constexpr float JRESCALE = 11.5f;        // log2 units: rescale when the running max grows more
 // the scores kernel's tokens are ordered by chunk count within windows of at most JSWIN
-// positions (a multiple of every scores workgroup's token count); the R(16T) rows of a window's
-// tiles fit in LDS
+// positions (a multiple of every scores workgroup's token count)
 constexpr int JSWIN = 2048;
 constexpr int JSORT_THREADS = 1024;
 
@@ -213,9 +212,11 @@ __global__ __launch_bounds__(JSORT_THREADS) void joint_sort_kernel(JSortParams p
 // Wave w takes sorted blocks w and NBLK-1-w (with one basis head: also 16+w and 31-w), one short
 // and one long, so the waves' products per chunk stay balanced. A token's position is arbitrary
 // within the window, so the key takes the whole rotation R(p) = R(16T) R(n) (p = 16T + n),
-// composed per lane from the R(n) table and the window's R(16T) rows in LDS; the query operand
-// is then the same for every token and formed once per head. Scores are stored at the tokens'
-// positions.
+// composed per lane from the R(n) table in LDS and the token's R(16T) row read from the table in
+// L2 (staging a window's rows, 64 KB per workgroup, cost more than the few a wave uses: whole call,
+// staged / read, 1 x 4096 tokens 61.0 / 59.5 us, 8 x 8000 with 2 bases 54.6 / 53.6, 16 x 8192 the
+// same); the query operand is then the same for every token and formed once per head. Scores are
+// stored at the tokens' positions.
 // NHB basis heads and CB 16-token blocks per wave; a wave's coefficients are loaded PF chunks ahead.
 template <int DT, int MODE, int ODT, int NHB, int CB, int PF>
 __global__ __launch_bounds__(JTHREADS, 1) void joint_scores_sorted_kernel(JScoresParams p) {
@@ -224,11 +225,6 @@ __global__ __launch_bounds__(JTHREADS, 1) void joint_scores_sorted_kernel(JScore
   __shared__ __attribute__((aligned(16))) dkv_u32x4 sB[4][NHB][JDH * JCH / 8];
   // R(n): [2*pp + k][16*g + n] holds (cos, sin) of frequencies 16pp + 4g + 2k and + 1 at delta n
   __shared__ __attribute__((aligned(16))) dkv_f32x4 sRn[8][64];
-  // R(16T) of the window's tiles: [T - T0][(2*pp + k) * 4 + g], the same frequencies; rows of 33
-  // entries (one of padding), so that lanes reading different tiles' entry (k, g) fall in
-  // different banks (with 32-entry rows every tile's entry sits in the same four banks)
-  constexpr int RT_ROW = 33;
-  __shared__ __attribute__((aligned(16))) dkv_f32x4 sRT[JSWIN / 16][RT_ROW];
   // the query operand of each head: row r = head r's hi part (r < 8) or head r-8's lo part,
   // dword i = frequency i, 16-byte chunk c stored at chunk position c ^ r
   __shared__ __attribute__((aligned(16))) uint32_t sQ[NHB][16 * 64];
@@ -291,16 +287,6 @@ __global__ __launch_bounds__(JTHREADS, 1) void joint_scores_sorted_kernel(JScore
     const int i0 = 16 * (k >> 1) + 4 * g + 2 * (k & 1);
     const float* delt = p.rope + n * 128 + 2 * i0;
     sRn[k][lane] = dkv_f32x4{delt[0], delt[1], delt[2], delt[3]};
-  }
-  {
-    const int T0 = wbase / 16, ntl = (wlen + 15) / 16;
-    for (int e = tid; e < ntl * 32; e += JTHREADS) {
-      const int tl = e >> 5, k = (e >> 2) & 7, gg = e & 3;
-      const int i0 = 16 * (k >> 1) + 4 * gg + 2 * (k & 1);
-      const int T = min(T0 + tl, p.rope_tiles - 1);
-      // 16-byte aligned (2 * i0 is a multiple of 4; the host checks the table's alignment)
-      sRT[tl][4 * k + gg] = *(const dkv_f32x4*)(p.rope + (long long)(JROPE_FIXED + T) * 128 + 2 * i0);
-    }
   }
   // the tokens arrive sorted by chunk count (joint_sort_kernel): a token's products and
   // rotation do not depend on its place in the block, and chunks past its count add zeros
@@ -459,12 +445,14 @@ __global__ __launch_bounds__(JTHREADS, 1) void joint_scores_sorted_kernel(JScore
     // R(p) = R(16T) R(n) for the lane's token: (cos, sin) of its 16 frequencies
     float rc[16], rsn[16];
     {
-      const int pl = pos_n < 0 ? 0 : pos_n - wbase;
-      const int tl = pl >> 4, nn = pl & 15;
+      const int pl = max(pos_n, 0), nn = pl & 15;
+      // the table's row of the token's tile (16-byte pieces; the host checks the table)
+      const float* rt = p.rope +
+                        (long long)(JROPE_FIXED + min(pl >> 4, p.rope_tiles - 1)) * 128 + 8 * g;
 #pragma unroll
       for (int k = 0; k < 8; ++k) {
         const dkv_f32x4 d = sRn[k][16 * g + nn];
-        const dkv_f32x4 t = sRT[tl][4 * k + g];
+        const dkv_f32x4 t = *(const dkv_f32x4*)(rt + 32 * (k >> 1) + 4 * (k & 1));
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           const float ct = t[2 * e], st = t[2 * e + 1], cn = d[2 * e], sn = d[2 * e + 1];
