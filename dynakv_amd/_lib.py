@@ -41,6 +41,9 @@ _SIGNATURES = {
     "dkv_append_prefill_kv": (_i, [_vp, _i, _i, _i, _i, _i,
                                    _vp, _ll, _ll, _vp, _ll, _ll, _vp, _ll, _vp, _vp, _ll, _ll, _vp,
                                    _vp, _ll, _ll, _vp, _ll, _ll, _vp, _ll, _vp, _vp, _ll, _ll, _vp]),
+    "dkv_append_prefill_new_kv": (_i, [_vp, _i, _i, _i, _i,
+                                   _vp, _ll, _ll, _vp, _ll, _ll, _vp, _ll, _vp, _vp, _ll, _ll, _vp,
+                                   _vp, _ll, _ll, _vp, _ll, _ll, _vp, _ll, _vp, _vp, _ll, _ll, _vp, _vp]),
     "dkv_decompress": (_i, [_vp, _i, _vp, _ll, _vp, _vp, _ll, _ll, _vp, _i, _i, _i]),
     "dkv_decompress_kv": (_i, [_vp, _i, _vp, _ll, _vp, _vp, _ll, _ll, _vp, _vp, _ll, _vp, _vp, _ll,
                                _ll, _vp, _i, _i, _i]),

@@ -73,6 +73,7 @@ PyMethodDef methods[] = {
     DKV_CALL(dkv_append_decode_kv),
     DKV_CALL(dkv_append_prefill),
     DKV_CALL(dkv_append_prefill_kv),
+    DKV_CALL(dkv_append_prefill_new_kv),
     DKV_CALL(dkv_decompress),
     DKV_CALL(dkv_decompress_kv),
     DKV_CALL(dkv_row_totals),

@@ -271,6 +271,7 @@ class CustomDynamicCache(_CacheBase):
             raise ValueError("update_sp_prefill_many takes prefill appends (S > 1)")
         # per slot and row: the summed counts (buffer sizing) and the clipped sums (the row's
         # pointer after the append, for a slot that starts empty), in one transfer
+        tot = None
         if len(lens) == 2 and self._totals_ok(lens[0], lens[1]):
             kl, vl = lens
             tot = torch.empty((2, 2, kl.shape[0]), dtype=torch.int64, device=kl.device)
@@ -290,6 +291,8 @@ class CustomDynamicCache(_CacheBase):
         rows = [l.shape[0] for l in lens]
         starts = [sum(rows[:k]) for k in range(len(lens))]
         half = sum(rows)
+        if tot is not None and self._append_new_pair(items[0], host, tot, max_dim):
+            return
         created = self._create_fresh_slots(items, lens, host, starts)
         for n, (layer_idx, ks, kl, vs, vl) in enumerate(items):
             prepared = []
@@ -314,13 +317,52 @@ class CustomDynamicCache(_CacheBase):
         return (kl.is_cuda and vl.device == kl.device and kl.dtype == vl.dtype == torch.int32
                 and kl.shape == vl.shape and kl.dim() == 2 and kl.shape[0] > 0)
 
-    def _create_fresh_slots(self, items, lens, host, starts):
+    def _append_new_pair(self, item, host, tot, max_dim) -> bool:
+        """A prompt onto K and V slots that do not exist yet, of one shape and dtype: the slots of
+        ``_create_fresh_slots`` with nothing filled, and one ``dkv_append_prefill_new_kv`` launch
+        that writes all of them. ``tot``: ``dkv_row_totals``' output, ``host`` its values. False,
+        with nothing changed, for any other call."""
+        layer_idx, ks, kl, vs, vl = item
+        B, S = kl.shape
+        lists = (self.key_cache_sp, self.value_cache_sp)
+        if (any(len(c) > layer_idx and c[layer_idx] is not None for c in lists) or S == 0
+                or ks.shape != vs.shape or ks.dtype != vs.dtype
+                or not ks.device == vs.device == kl.device
+                or max(host[:B]) <= 0 or max(host[B:2 * B]) <= 0
+                or seq_capacity_after(S, 0, S) != S):
+            return False
+        code = _lib.dtype_code(ks.dtype)  # raises before a slot is made
+        sk = ks if ks.stride(-1) == 1 else ks.contiguous()
+        sv = vs if vs.stride(-1) == 1 else vs.contiguous()
+        self._create_fresh_slots([item], [kl, vl], host, [0, B], fill=False)
+        slots = [c[layer_idx] for c in lists]
+        (fk, lk, okk, pk, _, _), (fv, lv, ov, pv, _, _) = slots
+        rc = _lib.calls().dkv_append_prefill_new_kv(
+            _lib.stream_of(fk), code, B, S, max_dim,
+            sk.data_ptr(), sk.stride(0), sk.stride(1), kl.data_ptr(), kl.stride(0), kl.stride(1),
+            fk.data_ptr(), fk.stride(0), lk.data_ptr(), okk.data_ptr(), lk.stride(0),
+            lk.stride(1), pk.data_ptr(),
+            sv.data_ptr(), sv.stride(0), sv.stride(1), vl.data_ptr(), vl.stride(0), vl.stride(1),
+            fv.data_ptr(), fv.stride(0), lv.data_ptr(), ov.data_ptr(), lv.stride(0),
+            lv.stride(1), pv.data_ptr(), tot.data_ptr() + tot.stride(0) * tot.element_size())
+        if rc != _lib.DKV_OK:
+            for c in lists:
+                c[layer_idx] = None  # nothing wrote them
+        _lib.check(rc, "dkv_append_prefill_new_kv")
+        for n, slot in enumerate(slots):
+            slot[4] = S
+            slot[5] = host[(2 + n) * B:(3 + n) * B]
+        return True
+
+    def _create_fresh_slots(self, items, lens, host, starts, fill=True):
         """The slots of ``items`` that do not exist yet, created as ``_prepare_slot`` creates
         them (flat sized to the largest row total, tables to the prompt, pointers zero) but
         from one zeroed buffer for every flat and pointer array and one unfilled buffer for the
         tables (the prefill append writes every table entry of a fresh slot): two fills in all
         instead of four per slot. Returns the created slots as ``(0 (K) | 1 (V), layer)``;
-        a slot whose rows hold no coefficient at all is left to ``_prepare_slot``."""
+        a slot whose rows hold no coefficient at all is left to ``_prepare_slot``. ``fill=False``
+        leaves the flats and pointers unfilled too (the caller's append writes all of them)."""
+        new = torch.zeros if fill else torch.empty
         fresh = []
         for n, it in enumerate(items):
             layer_idx = it[0]
@@ -341,10 +383,10 @@ class CustomDynamicCache(_CacheBase):
             by_dtype.setdefault(f[2].dtype, []).append(f)
         tab_elems = sum(f[3].numel() for f in fresh)
         tabs = torch.empty(2 * tab_elems, dtype=torch.int32, device=dev)
-        ptrs = torch.zeros(sum(f[3].shape[0] for f in fresh), dtype=torch.int32, device=dev)
+        ptrs = new(sum(f[3].shape[0] for f in fresh), dtype=torch.int32, device=dev)
         t_at = p_at = 0
         for dt, group in by_dtype.items():
-            flats = torch.zeros(sum(f[3].shape[0] * f[4] for f in group), dtype=dt, device=dev)
+            flats = new(sum(f[3].shape[0] * f[4] for f in group), dtype=dt, device=dev)
             f_at = 0
             for cache_list, layer_idx, st, ln, cap, _ in group:
                 B, S = ln.shape

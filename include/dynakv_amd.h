@@ -138,6 +138,21 @@ int dkv_append_prefill_kv(void* stream, int dtype, int seq_pos, int rows, int n_
                           long long tab_v_sb, long long tab_v_ss, int* ptr_v);
 
 /*
+ * The same for two slots that start empty (seq_pos 0, every row's pointer 0), in one launch, with
+ * flat and ptr unfilled on entry: every element of the rows' flat_ld and every pointer is written.
+ * totals: (2, rows) on the device, the clipped sums of dkv_row_totals (its out[1]) for these counts.
+ */
+int dkv_append_prefill_new_kv(void* stream, int dtype, int rows, int n_new, int max_dim,
+                          const void* states_k, long long states_k_sb, long long states_k_ss,
+                          const int* new_len_k, long long len_k_sb, long long len_k_ss,
+                          void* flat_k, long long flat_k_ld, int* lens_k, int* offs_k,
+                          long long tab_k_sb, long long tab_k_ss, int* ptr_k,
+                          const void* states_v, long long states_v_sb, long long states_v_ss,
+                          const int* new_len_v, long long len_v_sb, long long len_v_ss,
+                          void* flat_v, long long flat_v_ld, int* lens_v, int* offs_v,
+                          long long tab_v_sb, long long tab_v_ss, int* ptr_v, const long long* totals);
+
+/*
  * Dense re-expansion of a packed slot: out[b, t, j] = flat[b, offs[b,t] + j] for
  * j < min(lens[b,t], max_dim), else 0. out is (rows, seq, max_dim) contiguous, cache dtype.
  * Replaces simple_decompress (reference src/dynakv/kernels/compressed_cache.py:36-56),

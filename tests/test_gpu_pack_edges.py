@@ -45,6 +45,49 @@ def test_pack_and_expand(dev, i):
                                           ref.decompress(W).astype(np.float32))
 
 
+# (rows, tokens, width, dtype, state order): new slots of rows with very different totals
+NEW = [
+    (1, 2, 8, torch.bfloat16, "rows"),
+    (3, 65, 7, torch.float16, "rows"),
+    (4, 300, 128, torch.bfloat16, "tokens"),
+    (2, 33, 60, torch.float32, "dims"),
+    (9, 1030, 33, torch.bfloat16, "rows"),
+]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("i", range(len(NEW)))
+def test_new_slots_written_whole(dev, i):
+    """A prompt onto slots that do not exist, in memory that held other values: the zeros past
+    each row's last coefficient (rows without any among them) and the pointers are written."""
+    B, S, W, dtype, order = NEW[i]
+    print(f"[gpu] new slots {NEW[i]}", flush=True)
+    rng = np.random.default_rng(1300 + i)
+    perm = {"rows": (0, 1, 2), "tokens": (1, 0, 2), "dims": (0, 2, 1)}[order]  # memory order
+    x = [_rounded(rng.standard_normal((B, S, W)).astype(np.float32), dtype) for _ in range(2)]
+    n = [rng.integers(0, W + 1, (B, S)).astype(np.int32) for _ in range(2)]
+    for k, t in enumerate(n):
+        t[:, S // (2 + k):] //= np.arange(1, B + 1)[:, None] ** 2
+        if B > 2:
+            t[B - 2 + k] = 0
+    n[0][0, 0], n[1][0, 1] = W, W
+    inv = np.argsort(perm).tolist()
+    g = [t.permute(perm).contiguous().to(dev).permute(inv) for t in x]
+    dirty = [torch.full((m,), -1, dtype=torch.int16, device=dev)
+             for m in (64, 256, 512, 2 * B * S * W, 4 * B * S * W)]
+    del dirty
+    cache, rk, rv = CustomDynamicCache(), PackedSlot(), PackedSlot()
+    cache.update_sp(g[0], torch.from_numpy(n[0]).to(dev), g[1], torch.from_numpy(n[1]).to(dev),
+                    W, 0, W)
+    rk.append_prefill(x[0].float().numpy(), n[0], W)
+    rv.append_prefill(x[1].float().numpy(), n[1], W)
+    for slot, ref, what in ((cache.key_cache_sp[0], rk, "K"), (cache.value_cache_sp[0], rv, "V")):
+        _cmp_slot(slot, ref, what)
+        for b, end in enumerate(slot[3].tolist()):
+            assert end == slot[5][b]
+            assert not slot[0][b, end:].any()
+
+
 @pytest.mark.gpu
 def test_row_totals(dev):
     """Sums of raw and clipped counts, negative and oversized ones among them, strided tables."""
