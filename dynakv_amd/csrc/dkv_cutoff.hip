@@ -171,7 +171,7 @@ constexpr int CG_TN = 128;  // logits per tiled workgroup
 constexpr int CG_KS = 64;   // inputs per staged step
 
 // Logits of wide heads for many rows (a prompt), D = 128 * STEPS: workgroup = TM rows x 128
-// logits, four waves of TM/2 x 64, the inputs staged in LDS 64 at a time (three buffers,
+// logits, four waves of TM/2 x 64, the inputs staged in LDS 64 at a time (two to four buffers,
 // direct-to-LDS loads, 16-byte chunk c of a row at position c ^ (row % 8)). A = W rows, staged in
 // the order that gives lane (row n, g) the 16 consecutive logits 16g .. of its wave's 64 (LDS row
 // 16 * blk + i is logit 16 * (i / 4) + 4 * blk + i % 4), B = x rows. The products of each quarter
@@ -300,19 +300,8 @@ __global__ __launch_bounds__(256, 2) void cutoff_logits_tile_kernel(CutoffParams
   }
 }
 
-// e^d of d <= 0: exp2 of the product's leading part times its remainder (log2(e) as a hi + lo
-// pair), so the relative error stays that of v_exp_f32. d = -inf gives 0, NaN stays NaN.
-__device__ __forceinline__ float cf_exp(float d) {
-  constexpr float L_HI = 1.44269502162933349609375f, L_LO = 1.92596299112661746887e-8f;
-  constexpr float LN2 = 0.693147180559945286f;
-  d = d < -200.f ? -200.f : d;  // 2^-288 is 0 in fp32; a NaN fails the compare and stays
-  const float y = d * L_HI;
-  const float r = __builtin_fmaf(d, L_LO, __builtin_fmaf(d, L_HI, -y));
-  const float e = __builtin_amdgcn_exp2f(y);
-  return __builtin_fmaf(e, r * LN2, e);
-}
-
-// a / s from r = 1 / s: the product and one correction step (within an ulp of the division).
+// a / s from r = 1 / s (correctly rounded): the product and one correction step by the exact
+// remainder, which rounds as the division does (Markstein's theorem) short of underflow.
 __device__ __forceinline__ float cf_div(float a, float s, float r) {
   const float q = a * r;
   return __builtin_fmaf(__builtin_fmaf(-q, s, a), r, q);
@@ -348,7 +337,7 @@ __device__ __forceinline__ int cutoff_row_len(const CutoffParams& p, const uint1
   float s = 0.f;
 #pragma unroll
   for (int e = 0; e < E; ++e) {
-    x[e] = cf_exp(x[e] - mx);
+    x[e] = expf(x[e] - mx);
     s += x[e];
   }
   s = dkv_wave_sum_fast(s);
@@ -500,9 +489,9 @@ __device__ __forceinline__ float cf_max4(float v) {
   return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
 }
 __device__ __forceinline__ float cf_sum4(float v) {
-  auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   v = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-  r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+  r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
   return __uint_as_float(r[0]) + __uint_as_float(r[1]);
 }
 
@@ -516,8 +505,9 @@ constexpr int CF_WAVES = 4;
 // row: A row i of block blk is logit D / 4 * (i / 4) + 4 * blk + i % 4. A row's maximum, sum
 // and prefix sums then need two exchanges between four lanes instead of six steps across the
 // wave for each, for 16 rows at once, and the masked copy is the B operand itself.
-// Bound: VALU (softmax and counts, ~25 instructions per logit) and HBM about alike. 8192 rows x
-// 8 groups x 128, bf16: 31.7 us for 102 MB (3.2 TB/s; two kernels, one a wave per row, 108.3).
+// Bound: VALU (softmax and counts, ~35 instructions per logit) and HBM. 8192 rows x 8 groups x
+// 128, bf16: 31.2 us a call for 102 MB (two kernels, one a wave per row, 104.6; with the sums in
+// the lanes' own order, whose counts fall otherwise on rounding ties, 29.0).
 template <int DT, int NB>
 __global__ __launch_bounds__(64 * CF_WAVES, 3) void cutoff_fused_kernel(CutoffParams p) {
   constexpr int D = 16 * NB, KS = D / 32, PL = D / 4;  // PL: logits per lane
@@ -594,31 +584,54 @@ __global__ __launch_bounds__(64 * CF_WAVES, 3) void cutoff_fused_kernel(CutoffPa
 #pragma unroll
     for (int e = 1; e < PL; ++e) mx = fmaxf(mx, logit(e));
     mx = cf_max4(mx);
-    float pr[PL];
-    float part[4] = {0.f, 0.f, 0.f, 0.f};
+    // The sums below are taken in the order of cutoff_row_len (64 lanes of E consecutive positions:
+    // a lane here holds 16 of those lanes' positions), so that a count on a rounding tie falls
+    // the same way on every path.
+    constexpr int E = PL / 16;
+    float pr[PL], part[16];
 #pragma unroll
-    for (int e = 0; e < PL; ++e) {
-      pr[e] = cf_exp(logit(e) - mx);
-      part[e & 3] += pr[e];
+    for (int l = 0; l < 16; ++l) {
+      part[l] = 0.f;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        pr[E * l + e] = expf(logit(E * l + e) - mx);
+        part[l] += pr[E * l + e];
+      }
     }
-    const float sum = cf_sum4((part[0] + part[1]) + (part[2] + part[3]));
+#pragma unroll
+    for (int d = 1; d < 16; d <<= 1)  // the butterfly's tree
+#pragma unroll
+      for (int l = 0; l < 16; l += 2 * d) part[l] += part[l + d];
+    const float sum = cf_sum4(part[0]);
     // probabilities in the compute dtype, their prefix sums in fp32
     const float rcp = 1.0f / sum;
-    float run = 0.f;
 #pragma unroll
-    for (int e = 0; e < PL; ++e) {
-      run += dkv_round_to<DT>(cf_div(pr[e], sum, rcp));
-      pr[e] = run;
+    for (int l = 0; l < 16; ++l) {
+      float run = 0.f;
+#pragma unroll
+      for (int e = 0; e < E; ++e) {
+        run += dkv_round_to<DT>(cf_div(pr[E * l + e], sum, rcp));
+        pr[E * l + e] = run;
+      }
+      part[l] = run;
     }
+#pragma unroll
+    for (int d = 1; d < 16; d <<= 1)  // inclusive scan of the 16 totals
+#pragma unroll
+      for (int l = 15; l >= d; --l) part[l] += part[l - d];
     // the totals of the row's lanes before this one
-    const float t16 = __shfl_xor(run, 16, 64);
-    const float t32 = __shfl_xor(run + t16, 32, 64);
-    const float excl = ((g & 1) ? t16 : 0.f) + ((g & 2) ? t32 : 0.f);
+    const float t16 = __shfl_xor(part[15], 16, 64);
+    const float t32 = __shfl_xor(part[15] + t16, 32, 64);
+    const float b1 = (g & 1) ? t16 : 0.f, b2 = (g & 2) ? t32 : 0.f;
     // a prefix sum counts when its rounding reaches the threshold, i.e. when it reaches the
     // smallest fp32 value that rounds to it
     int cnt = 0;
 #pragma unroll
-    for (int e = 0; e < PL; ++e) cnt += excl + pr[e] >= p.count_min ? 1 : 0;
+    for (int l = 0; l < 16; ++l) {
+      const float excl = ((part[l] + b1) + b2) - pr[E * l + E - 1];
+#pragma unroll
+      for (int e = 0; e < E; ++e) cnt += excl + pr[E * l + e] >= p.count_min ? 1 : 0;
+    }
     cnt += __shfl_xor(cnt, 16, 64);
     cnt += __shfl_xor(cnt, 32, 64);
     const int len = min(cnt, max(p.low_rank, 0));
@@ -933,7 +946,8 @@ extern "C" int dkv_cutoff_kv(void* stream, int dtype, const void* xk, const void
   // 256 CUs once, the wave-per-tile kernel past that. Graph-replayed us per call, 8-wave / wave
   // per tile: G = 8, D = 128: 33 rows 5.2 / 6.7, 301 rows 7.0 / 7.2, 1024 rows 13.4 / 8.5, 8192
   // rows 72.3 / 31.7 (two kernels, a wave per row, before: 5.9, 8.7, 19.6, 108.3); G = 4: 301
-  // rows 5.3 / 7.1, 1024 rows 8.4 / 7.7.
+  // rows 5.3 / 7.1, 1024 rows 8.4 / 7.7 (the wave-per-tile figures from before its sums took the
+  // row kernel's order, about 2 us more at 8192 rows).
   const long long row_tiles = (M + CT_ROWS - 1) / CT_ROWS;
   if (D <= 128 && (row_tiles == 1 || 2 * G * row_tiles <= 320)) {
     const dim3 sgrid((unsigned)(2 * G), (unsigned)row_tiles);

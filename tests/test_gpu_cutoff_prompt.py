@@ -75,3 +75,22 @@ def test_special_values_and_unaligned_outputs(dev):
     torch.cuda.synchronize()
     assert torch.equal(ln[0], lk)
     assert torch.equal(out[0, 1:].view(M, H).view(torch.int16), k.view(torch.int16))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,dtype", [(128, torch.bfloat16), (128, torch.float16),
+                                     (64, torch.bfloat16)])
+def test_prompt_counts_equal_decode_counts(dev, D, dtype):
+    """A prompt in one call gives every row the count and the masked copy that the decode-size
+    kernel gives it, bit for bit: sums in one order, so rounding ties fall alike."""
+    G, M = 8, 8192
+    print(f"[gpu] cutoff prompt against decode sizes D={D} {dtype}", flush=True)
+    x, W, b = _inputs(G, D, M, dtype, 3.0, seed=8400 + D)
+    t = lambda a: torch.from_numpy(a).to(device=dev, dtype=dtype)  # noqa: E731
+    xd, wd, bd = t(x), t(W), t(b)
+    head = CK.CutoffHead(wd, bd, wd, bd, groups=G)
+    k, _, lk, _, _, _ = head.kv_process_fused(xd, xd)
+    for r in range(0, M, 128):
+        few, _, lf, _, _, _ = head.kv_process_fused(xd[r:r + 128], xd[r:r + 128])
+        assert torch.equal(lk[r:r + 128], lf), r
+        assert torch.equal(k[r:r + 128].view(torch.int16), few.view(torch.int16)), r
