@@ -300,11 +300,17 @@ __global__ __launch_bounds__(256, 2) void cutoff_logits_tile_kernel(CutoffParams
   }
 }
 
-// a / s from r = 1 / s (correctly rounded): the product and one correction step by the exact
-// remainder, which rounds as the division does (Markstein's theorem) short of underflow.
+// a / s rounded to fp32, from r = 1 / s (correctly rounded): the product and one correction step by
+// the exact remainder, which rounds as the division does (Markstein's theorem) while the remainder
+// does not underflow (quotients above about 2^-100; smaller ones only a threshold as small could
+// see). The empty asm keeps the fp32 quotient a value of its own: the compiler otherwise folds the
+// last fma and the conversion to fp16 that follows into one v_fma_mixlo_f16, which rounds once, and
+// probabilities beside an fp16 tie come out as the other neighbour.
 __device__ __forceinline__ float cf_div(float a, float s, float r) {
   const float q = a * r;
-  return __builtin_fmaf(__builtin_fmaf(-q, s, a), r, q);
+  float v = __builtin_fmaf(__builtin_fmaf(-q, s, a), r, q);
+  asm("" : "+v"(v));
+  return v;
 }
 
 // The retained count of one (row m, group g) of a matrix, computed by one wave from the
