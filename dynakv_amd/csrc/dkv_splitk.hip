@@ -68,13 +68,12 @@ constexpr int DPP_ROW_SHL8 = 0x108;      // DPP row_shl:8: lane i of a 16-lane r
 struct SplitParams {
   const uint16_t* q;
   long long q_sb, q_sh;
-  // bases: element (unit u, rank r, dim d) at u * unit + r * sr + d (bt = 0, sr the rank
-  // stride), or at u * unit + d * sr + r (bt = 1: a transposed basis, sr the dim stride)
+  // bases: element (unit u, rank r, dim d) at u * unit + r * sr + d (sr the rank stride), or in
+  // the BT instances of the kernels at u * unit + d * sr + r (transposed bases, sr the dim stride)
   const uint16_t* k_basis;
   long long k_unit, k_sr;
   const uint16_t* v_basis;
   long long v_unit, v_sr;
-  int bt;
   const uint16_t* k_flat;
   const uint16_t* v_flat;
   int k_ld, v_ld;
@@ -395,9 +394,10 @@ __device__ __forceinline__ void merge_records_w(const SplitParams& p, const floa
 // 8 * (ch % 16); of a transposed basis dim ch / 16, ranks 8 * (ch % 16)); unconditional loads
 // (pieces of ranks past R read real ones and are zeroed when staged), so that none waits for
 // another.
+template <bool BT>
 __device__ __forceinline__ void load_vbasis(const SplitParams& p, int kvh, dkv_u32x4 (&vbr)[VB_CHUNKS]) {
   const uint16_t* vb = p.v_basis + (long long)kvh * p.v_unit;
-  if (p.bt) {
+  if constexpr (BT) {
 #pragma unroll
     for (int k = 0; k < VB_CHUNKS; ++k) {
       const int ch = (int)threadIdx.x + k * NTHREADS;
@@ -412,11 +412,11 @@ __device__ __forceinline__ void load_vbasis(const SplitParams& p, int kvh, dkv_u
   }
 }
 
-template <int DT, int ODT>
+template <int DT, int ODT, bool BT>
 __device__ __forceinline__ void project_store(const SplitParams& p, int unit, uint8_t* scratch,
                                               const dkv_u32x4 (&vbr)[VB_CHUNKS]);
 
-template <int DT, int ROUTE, int ODT>
+template <int DT, int ROUTE, int ODT, bool BT>
 __device__ __forceinline__ void merge_unit_t(const SplitParams& p, int unit, uint8_t* scratch) {
   const int kvh = unit % p.Hkv;
   const long long stride = (long long)p.hpg * PREC;  // between splits of one head
@@ -424,7 +424,7 @@ __device__ __forceinline__ void merge_unit_t(const SplitParams& p, int unit, uin
   float* sA = reinterpret_cast<float*>(scratch + DH * DH * 2);    // [16][DH] merged, normalised
   // the V basis in flight while the records are read and merged
   dkv_u32x4 vbr[VB_CHUNKS];
-  load_vbasis(p, kvh, vbr);
+  load_vbasis<BT>(p, kvh, vbr);
   // merged coefficient of (head slot hs, rank r); slots past hpg are zero. A batch of MB
   // splits' record loads is issued before any is used, so a call pays one load latency per
   // MB splits (MB the smallest of 8, 16, 32 that covers the splits). Up to 8 splits merge
@@ -441,13 +441,13 @@ __device__ __forceinline__ void merge_unit_t(const SplitParams& p, int unit, uin
     merge_records_w<32, ROUTE>(p, base, stride, sA, sM, sL, sW);
   else
     merge_records<32, ROUTE>(p, base, stride, sA);
-  project_store<DT, ODT>(p, unit, scratch, vbr);
+  project_store<DT, ODT, BT>(p, unit, scratch, vbr);
 }
 
 // out = the merged, normalised coefficients sA (scratch + DH * DH * 2, [16][DH], written by
 // every thread before the call) through the V basis (vbr, staged here at scratch), stored in
 // the output dtype (all threads of the block).
-template <int DT, int ODT>
+template <int DT, int ODT, bool BT>
 __device__ __forceinline__ void project_store(const SplitParams& p, int unit, uint8_t* scratch,
                                               const dkv_u32x4 (&vbr)[VB_CHUNKS]) {
   const int b = unit / p.Hkv, kvh = unit % p.Hkv;
@@ -460,8 +460,8 @@ __device__ __forceinline__ void project_store(const SplitParams& p, int unit, ui
 #pragma unroll
   for (int k = 0; k < VB_CHUNKS; ++k) {
     const int ch = tid + k * NTHREADS;
-    const int at = p.bt ? (ch & ~15) | ((ch & 15) ^ ((ch >> 4) & 15)) : ch;
-    const bool live = p.bt ? 8 * (ch & 15) < p.R : ch < p.R * (DH / 8);
+    const int at = BT ? (ch & ~15) | ((ch & 15) ^ ((ch >> 4) & 15)) : ch;
+    const bool live = BT ? 8 * (ch & 15) < p.R : ch < p.R * (DH / 8);
     *(dkv_u32x4*)(sVB + at * 8) = live ? vbr[k] : dkv_u32x4{0u, 0u, 0u, 0u};
   }
   __syncthreads();
@@ -493,7 +493,7 @@ __device__ __forceinline__ void project_store(const SplitParams& p, int unit, ui
       }
     }
     dkv_u32x4 bop;
-    if (p.bt) {  // ranks k0 .. k0 + 7 of dim d0 + n
+    if constexpr (BT) {  // ranks k0 .. k0 + 7 of dim d0 + n
       bop = *(const dkv_u32x4*)(sVB + (d0 + n) * DH + 8 * ((4 * c + g) ^ n));
     } else {
       const uint16_t* src = sVB + (k0 + (n >> 2)) * DH + d0 + 4 * (n & 3);
@@ -519,12 +519,12 @@ __device__ __forceinline__ void project_store(const SplitParams& p, int unit, ui
     }
   }
 }
-template <int DT, int ROUTE>
+template <int DT, int ROUTE, bool BT>
 __device__ __forceinline__ void merge_unit(const SplitParams& p, int unit, uint8_t* scratch) {
   if (p.out_f32)
-    merge_unit_t<DT, ROUTE, DKV_F32>(p, unit, scratch);
+    merge_unit_t<DT, ROUTE, DKV_F32, BT>(p, unit, scratch);
   else
-    merge_unit_t<DT, ROUTE, DT>(p, unit, scratch);
+    merge_unit_t<DT, ROUTE, DT, BT>(p, unit, scratch);
 }
 
 // HMAX: the most query heads per unit the instance handles (4, 8 or 16); each lane keeps HMAX
@@ -532,7 +532,7 @@ __device__ __forceinline__ void merge_unit(const SplitParams& p, int unit, uint8
 // heads (WIDE) the query operand carries the heads' hi parts in its 16 columns and a second
 // product takes the lo parts; with up to 8 heads the hi parts sit in columns 0..7 and the lo
 // parts in columns 8..15 of one product.
-template <int DT, int ROUTE, int HMAX, bool PAIR>
+template <int DT, int ROUTE, int HMAX, bool PAIR, bool BT>
 __global__ __launch_bounds__(NTHREADS, 1) void splitk_kernel(SplitParams p) {
   constexpr bool WIDE = HMAX > 8;
   // LDS: per-wave rings (NSLOT gather slots: K then V, 4 chunks x 64 lanes x 16 bytes each;
@@ -639,7 +639,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void splitk_kernel(SplitParams p) {
     const uint16_t* kb = p.k_basis + (long long)kvh * p.k_unit;
     const int j = tid & 127, dq = tid >> 7;  // 4 groups of 8-dim slices
     static_assert(NREG_PP == 4, "a transposed basis is staged whole");
-    if (p.bt) {
+    if constexpr (BT) {
       // already [dim][rank]: 16-byte pieces (dim ch / 16, ranks 8 * (ch % 16); R is a multiple
       // of 8)
 #pragma unroll
@@ -649,22 +649,23 @@ __global__ __launch_bounds__(NTHREADS, 1) void splitk_kernel(SplitParams p) {
         if (r8 >= R) v = dkv_u32x4{0u, 0u, 0u, 0u};
         *(dkv_u32x4*)(sBK + d * BK_LD + r8) = v;
       }
-    } else
+    } else {
 #pragma unroll
-    for (int it = 0; it < 4; ++it) {
-      const int d8 = (dq + 4 * it) * 8;
-      dkv_u32x4 v = dkv_u32x4{0u, 0u, 0u, 0u};
-      if (j < R) v = *(const dkv_u32x4*)(kb + (long long)j * p.k_sr + d8);
-      const uint32_t e[4] = {v.x, v.y, v.z, v.w};
+      for (int it = 0; it < 4; ++it) {
+        const int d8 = (dq + 4 * it) * 8;
+        dkv_u32x4 v = dkv_u32x4{0u, 0u, 0u, 0u};
+        if (j < R) v = *(const dkv_u32x4*)(kb + (long long)j * p.k_sr + d8);
+        const uint32_t e[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
-      for (int t = 0; t < 8; ++t) {
-        const int d = d8 + t;
-        const uint16_t x = (uint16_t)((e[t >> 1] >> (16 * (t & 1))) & 0xffffu);
-        const int pp = (d & 63) >> 4;
-        if (pp >= NREG_PP)
-          sBH[(((d >> 6) * (4 - NREG_PP) + pp - NREG_PP) * 16 + (d & 15)) * BK_LD + j] = x;
-        else
-          sBK[d * BK_LD + j] = x;
+        for (int t = 0; t < 8; ++t) {
+          const int d = d8 + t;
+          const uint16_t x = (uint16_t)((e[t >> 1] >> (16 * (t & 1))) & 0xffffu);
+          const int pp = (d & 63) >> 4;
+          if (pp >= NREG_PP)
+            sBH[(((d >> 6) * (4 - NREG_PP) + pp - NREG_PP) * 16 + (d & 15)) * BK_LD + j] = x;
+          else
+            sBK[d * BK_LD + j] = x;
+        }
       }
     }
     // row MASK_BIAS + dk: keep-mask of the lane's last piece when its token has dk elements from
@@ -1167,7 +1168,7 @@ __global__ __launch_bounds__(NTHREADS, 1) void splitk_kernel(SplitParams p) {
     // its record and the record merge (a single record's weight is 1), without writing the
     // record, counting the arrival and reading the record back
     dkv_u32x4 vbr[VB_CHUNKS];
-    load_vbasis(p, kvh, vbr);
+    load_vbasis<BT>(p, kvh, vbr);
     constexpr int NA = 16 * DH / NTHREADS;
     float av[NA];
 #pragma unroll
@@ -1198,9 +1199,9 @@ __global__ __launch_bounds__(NTHREADS, 1) void splitk_kernel(SplitParams p) {
 #pragma unroll
     for (int k = 0; k < NA; ++k) sA[tid + k * NTHREADS] = av[k];
     if (p.out_f32)
-      project_store<DT, DKV_F32>(p, unit, sRing, vbr);
+      project_store<DT, DKV_F32, BT>(p, unit, sRing, vbr);
     else
-      project_store<DT, DT>(p, unit, sRing, vbr);
+      project_store<DT, DT, BT>(p, unit, sRing, vbr);
     return;
   }
   float* prec = p.partials + ((long long)unit * p.n_splits + split) * p.hpg * PREC;
@@ -1238,13 +1239,13 @@ __global__ __launch_bounds__(NTHREADS, 1) void splitk_kernel(SplitParams p) {
   }
   __syncthreads();
   if (!sLast) return;
-  merge_unit<DT, ROUTE>(p, unit, sRing);
+  merge_unit<DT, ROUTE, BT>(p, unit, sRing);
   if (tid == 0) p.counters[unit] = 0;  // ready for the next call (calls are stream-ordered)
 }
 
 // One workgroup per (unit, head slot): LSE-merge the split records of that head, normalise with
 // the route's denominator, project once through the unit's V basis, store in the output dtype.
-template <int DT, int ROUTE, int ODT>
+template <int DT, int ROUTE, int ODT, bool BT>
 __global__ __launch_bounds__(256) void merge_kernel(SplitParams p) {
   __shared__ float sW[1024];  // split weights (n_splits <= 1024 handled in chunks)
   __shared__ float sA[DH];
@@ -1297,7 +1298,7 @@ __global__ __launch_bounds__(256) void merge_kernel(SplitParams p) {
     float o = 0.f;
 #pragma unroll 8
     for (int j = half; j < R; j += 2)
-      o = fmaf(sA[j], elt_to_f32<DT>(vb[p.bt ? (long long)d * p.v_sr + j : (long long)j * p.v_sr + d]), o);
+      o = fmaf(sA[j], elt_to_f32<DT>(vb[BT ? (long long)d * p.v_sr + j : (long long)j * p.v_sr + d]), o);
     __syncthreads();
     sO[half][d] = o;
     __syncthreads();
@@ -1474,7 +1475,7 @@ struct ProfileState {
 };
 static ProfileState g_prof;
 
-template <int DT, int RT>
+template <int DT, int RT, bool BT>
 static void launch_splitk_t(const SplitParams& p, int out_dtype, dim3 grid, dim3 mgrid,
                             hipStream_t st) {
   const int slot = (g_prof.on && g_prof.n < g_prof.cap) ? g_prof.n++ : -1;
@@ -1484,24 +1485,43 @@ static void launch_splitk_t(const SplitParams& p, int out_dtype, dim3 grid, dim3
   // pair's query operand of hi and lo rows would add spills)
   const bool pair = p.split_len >= 2 * WAVES * TILE;
   if (p.hpg > 8)
-    hipLaunchKernelGGL((splitk_kernel<DT, RT, 16, false>), grid, dim3(NTHREADS), 0, st, p);
+    hipLaunchKernelGGL((splitk_kernel<DT, RT, 16, false, BT>), grid, dim3(NTHREADS), 0, st, p);
   else if (p.hpg > 4 && pair)
-    hipLaunchKernelGGL((splitk_kernel<DT, RT, 8, true>), grid, dim3(NTHREADS), 0, st, p);
+    hipLaunchKernelGGL((splitk_kernel<DT, RT, 8, true, BT>), grid, dim3(NTHREADS), 0, st, p);
   else if (p.hpg > 4)
-    hipLaunchKernelGGL((splitk_kernel<DT, RT, 8, false>), grid, dim3(NTHREADS), 0, st, p);
+    hipLaunchKernelGGL((splitk_kernel<DT, RT, 8, false, BT>), grid, dim3(NTHREADS), 0, st, p);
   else if (pair)
-    hipLaunchKernelGGL((splitk_kernel<DT, RT, 4, true>), grid, dim3(NTHREADS), 0, st, p);
+    hipLaunchKernelGGL((splitk_kernel<DT, RT, 4, true, BT>), grid, dim3(NTHREADS), 0, st, p);
   else
-    hipLaunchKernelGGL((splitk_kernel<DT, RT, 4, false>), grid, dim3(NTHREADS), 0, st, p);
+    hipLaunchKernelGGL((splitk_kernel<DT, RT, 4, false, BT>), grid, dim3(NTHREADS), 0, st, p);
   if (ev) (void)hipEventRecord(ev[1], st);
   if (!p.fused_merge) {
     if (out_dtype == DKV_F32)
-      hipLaunchKernelGGL((merge_kernel<DT, RT, DKV_F32>), mgrid, dim3(256), 0, st, p);
+      hipLaunchKernelGGL((merge_kernel<DT, RT, DKV_F32, BT>), mgrid, dim3(256), 0, st, p);
     else
-      hipLaunchKernelGGL((merge_kernel<DT, RT, DT>), mgrid, dim3(256), 0, st, p);
+      hipLaunchKernelGGL((merge_kernel<DT, RT, DT, BT>), mgrid, dim3(256), 0, st, p);
     if (ev) (void)hipEventRecord(ev[2], st);
   }
   if (slot >= 0) g_prof.merged[slot] = !p.fused_merge;
+}
+
+// BT: transposed bases. Instances of their own: the branch taken at run time in one kernel cost
+// rank-major calls 1-2% (graph-replayed us, 32 query / 8 KV heads, bf16, with it / without: 1 x 96
+// tokens 13.03 / 12.91, 1 x 2048 19.42 / 19.05, 4 x 8192 31.4 / 30.9).
+template <bool BT>
+static void launch_splitk(const SplitParams& p, int route, int dtype, int out_dtype, dim3 grid,
+                          dim3 mgrid, hipStream_t st) {
+  if (dtype == DKV_BF16) {
+    if (route == DKV_ROUTE_FUSED)
+      launch_splitk_t<DKV_BF16, DKV_ROUTE_FUSED, BT>(p, out_dtype, grid, mgrid, st);
+    else
+      launch_splitk_t<DKV_BF16, DKV_ROUTE_TWO_STAGE, BT>(p, out_dtype, grid, mgrid, st);
+  } else {
+    if (route == DKV_ROUTE_FUSED)
+      launch_splitk_t<DKV_F16, DKV_ROUTE_FUSED, BT>(p, out_dtype, grid, mgrid, st);
+    else
+      launch_splitk_t<DKV_F16, DKV_ROUTE_TWO_STAGE, BT>(p, out_dtype, grid, mgrid, st);
+  }
 }
 
 static void profile_release() {
@@ -1623,7 +1643,6 @@ static int splitk_launch(void* stream, int route, int dtype, int bt, const void*
   p.v_basis = (const uint16_t*)v_basis;
   p.v_unit = v_unit_stride;
   p.v_sr = v_basis_sr;
-  p.bt = bt;
   p.k_flat = (const uint16_t*)k_flat;
   p.v_flat = (const uint16_t*)v_flat;
   p.k_ld = (int)k_ld;
@@ -1661,17 +1680,10 @@ static int splitk_launch(void* stream, int route, int dtype, int bt, const void*
   p.minus_one = -1.0f;
   const dim3 grid((unsigned)(units * n_splits)), mgrid((unsigned)(units * (Hq / Hkv)));
   hipStream_t st = (hipStream_t)stream;
-  if (dtype == DKV_BF16) {
-    if (route == DKV_ROUTE_FUSED)
-      launch_splitk_t<DKV_BF16, DKV_ROUTE_FUSED>(p, out_dtype, grid, mgrid, st);
-    else
-      launch_splitk_t<DKV_BF16, DKV_ROUTE_TWO_STAGE>(p, out_dtype, grid, mgrid, st);
-  } else {
-    if (route == DKV_ROUTE_FUSED)
-      launch_splitk_t<DKV_F16, DKV_ROUTE_FUSED>(p, out_dtype, grid, mgrid, st);
-    else
-      launch_splitk_t<DKV_F16, DKV_ROUTE_TWO_STAGE>(p, out_dtype, grid, mgrid, st);
-  }
+  if (bt)
+    launch_splitk<true>(p, route, dtype, out_dtype, grid, mgrid, st);
+  else
+    launch_splitk<false>(p, route, dtype, out_dtype, grid, mgrid, st);
   DKV_HIP_CHECK_LAUNCH();
   return DKV_OK;
 }
