@@ -318,24 +318,28 @@ class CustomDynamicCache(_CacheBase):
                 and kl.shape == vl.shape and kl.dim() == 2 and kl.shape[0] > 0)
 
     def _append_new_pair(self, item, host, tot, max_dim) -> bool:
-        """A prompt onto K and V slots that do not exist yet, of one shape and dtype: the slots of
-        ``_create_fresh_slots`` with nothing filled, and one ``dkv_append_prefill_new_kv`` launch
-        that writes all of them. ``tot``: ``dkv_row_totals``' output, ``host`` its values. False,
-        with nothing changed, for any other call."""
+        """A prompt onto K and V slots that do not exist yet, of one shape and dtype: the slots as
+        ``_prepare_slot`` sizes them, unfilled, and one ``dkv_append_prefill_new_kv`` launch that
+        writes all of them. Each slot has buffers of its own (one slot's growth frees its old ones).
+        ``tot``: ``dkv_row_totals``' output, ``host`` its values. False, with nothing changed, for
+        any other call."""
         layer_idx, ks, kl, vs, vl = item
         B, S = kl.shape
         lists = (self.key_cache_sp, self.value_cache_sp)
+        caps = max(host[:B]), max(host[B:2 * B])
         if (any(len(c) > layer_idx and c[layer_idx] is not None for c in lists) or S == 0
                 or ks.shape != vs.shape or ks.dtype != vs.dtype
-                or not ks.device == vs.device == kl.device
-                or max(host[:B]) <= 0 or max(host[B:2 * B]) <= 0
+                or not ks.device == vs.device == kl.device or min(caps) <= 0
                 or seq_capacity_after(S, 0, S) != S):
             return False
         code = _lib.dtype_code(ks.dtype)  # raises before a slot is made
         sk = ks if ks.stride(-1) == 1 else ks.contiguous()
         sv = vs if vs.stride(-1) == 1 else vs.contiguous()
-        self._create_fresh_slots([item], [kl, vl], host, [0, B], fill=False)
-        slots = [c[layer_idx] for c in lists]
+        slots = []
+        for cap in caps:
+            lens, offs = torch.empty((2, B, S), dtype=torch.int32, device=ks.device).unbind(0)
+            slots.append([torch.empty((B, cap), dtype=ks.dtype, device=ks.device), lens, offs,
+                          torch.empty(B, dtype=torch.int32, device=ks.device), S, None])
         (fk, lk, okk, pk, _, _), (fv, lv, ov, pv, _, _) = slots
         rc = _lib.calls().dkv_append_prefill_new_kv(
             _lib.stream_of(fk), code, B, S, max_dim,
@@ -345,24 +349,21 @@ class CustomDynamicCache(_CacheBase):
             sv.data_ptr(), sv.stride(0), sv.stride(1), vl.data_ptr(), vl.stride(0), vl.stride(1),
             fv.data_ptr(), fv.stride(0), lv.data_ptr(), ov.data_ptr(), lv.stride(0),
             lv.stride(1), pv.data_ptr(), tot.data_ptr() + tot.stride(0) * tot.element_size())
-        if rc != _lib.DKV_OK:
-            for c in lists:
-                c[layer_idx] = None  # nothing wrote them
         _lib.check(rc, "dkv_append_prefill_new_kv")
-        for n, slot in enumerate(slots):
-            slot[4] = S
+        for n, (c, slot) in enumerate(zip(lists, slots)):
             slot[5] = host[(2 + n) * B:(3 + n) * B]
+            while len(c) <= layer_idx:
+                c.append(None)
+            c[layer_idx] = slot
         return True
 
-    def _create_fresh_slots(self, items, lens, host, starts, fill=True):
+    def _create_fresh_slots(self, items, lens, host, starts):
         """The slots of ``items`` that do not exist yet, created as ``_prepare_slot`` creates
         them (flat sized to the largest row total, tables to the prompt, pointers zero) but
         from one zeroed buffer for every flat and pointer array and one unfilled buffer for the
         tables (the prefill append writes every table entry of a fresh slot): two fills in all
         instead of four per slot. Returns the created slots as ``(0 (K) | 1 (V), layer)``;
-        a slot whose rows hold no coefficient at all is left to ``_prepare_slot``. ``fill=False``
-        leaves the flats and pointers unfilled too (the caller's append writes all of them)."""
-        new = torch.zeros if fill else torch.empty
+        a slot whose rows hold no coefficient at all is left to ``_prepare_slot``."""
         fresh = []
         for n, it in enumerate(items):
             layer_idx = it[0]
@@ -383,10 +384,10 @@ class CustomDynamicCache(_CacheBase):
             by_dtype.setdefault(f[2].dtype, []).append(f)
         tab_elems = sum(f[3].numel() for f in fresh)
         tabs = torch.empty(2 * tab_elems, dtype=torch.int32, device=dev)
-        ptrs = new(sum(f[3].shape[0] for f in fresh), dtype=torch.int32, device=dev)
+        ptrs = torch.zeros(sum(f[3].shape[0] for f in fresh), dtype=torch.int32, device=dev)
         t_at = p_at = 0
         for dt, group in by_dtype.items():
-            flats = new(sum(f[3].shape[0] * f[4] for f in group), dtype=dt, device=dev)
+            flats = torch.zeros(sum(f[3].shape[0] * f[4] for f in group), dtype=dt, device=dev)
             f_at = 0
             for cache_list, layer_idx, st, ln, cap, _ in group:
                 B, S = ln.shape
