@@ -9,11 +9,14 @@ from __future__ import annotations
 
 import ctypes as C
 import importlib.util
+import sysconfig
 import threading
 from pathlib import Path
 
 import torch
 
+# the CPython binding's file beside the library, named for the interpreter it was built for
+CALL_NAME = "_dkv_call" + sysconfig.get_config_var("EXT_SUFFIX")
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "libdynakv_amd.so"
 
 DKV_F32, DKV_F16, DKV_BF16 = 0, 1, 2
@@ -160,22 +163,22 @@ def load() -> C.CDLL:
 
 def calls():
     """The per-call entry points as the ``_dkv_call`` module's functions: the same C functions as
-    ``load()``'s, without ctypes' argument conversion (~5 us of a 40-argument call). Raises if the
-    module has not been built."""
+    ``load()``'s, without ctypes' argument conversion (~5 us of a 40-argument call). ``load()``'s
+    own where there is no module for this interpreter beside the library."""
     global _calls
     if _calls is not None:
         return _calls
-    load()  # the library (and torch's HIP runtime) first: the module binds to it
+    lib = load()  # the library (and torch's HIP runtime) first: the module binds to it
     with _lock:
         if _calls is None:
-            path = LIB_PATH.with_name("_dkv_call.so")
-            if not path.exists():
-                raise RuntimeError(f"dynakv_amd call module not found at {path}; "
-                                   "build it with `python -m dynakv_amd.build`")
-            spec = importlib.util.spec_from_file_location("_dkv_call", path)
-            mod = importlib.util.module_from_spec(spec)
-            spec.loader.exec_module(mod)
-            _calls = mod
+            path = LIB_PATH.with_name(CALL_NAME)
+            if path.exists():
+                spec = importlib.util.spec_from_file_location("_dkv_call", path)
+                mod = importlib.util.module_from_spec(spec)
+                spec.loader.exec_module(mod)
+                _calls = mod
+            else:
+                _calls = lib
     return _calls
 
 

@@ -1,8 +1,10 @@
 """Build the C-ABI shared library ``dynakv_amd/lib/libdynakv_amd.so`` for gfx950.
 
 Plain ``hipcc`` per source file (in parallel), then one link step, then the CPython binding of its
-per-call entry points (``dkv_call.cpp``, ``dynakv_amd/lib/_dkv_call.so``) linked against it. Both
-are built in-tree so they travel with the repository snapshot to the GPU host.
+per-call entry points (``dkv_call.cpp``, ``dynakv_amd/lib/_dkv_call.<interpreter tag>.so``) linked
+against it. Both are built in-tree so they travel with the repository snapshot to the GPU host. The
+binding needs the interpreter's C headers; without them it is left out and the ctypes binding serves
+(the same functions, about 5 us more per call).
 
 Usage: ``python -m dynakv_amd.build`` (or ``dynakv_amd.build.build()``).
 """
@@ -21,7 +23,7 @@ PKG_DIR = Path(__file__).resolve().parent
 CSRC = PKG_DIR / "csrc"
 LIB_DIR = PKG_DIR / "lib"
 LIB_PATH = LIB_DIR / "libdynakv_amd.so"
-CALL_PATH = LIB_DIR / "_dkv_call.so"
+CALL_PATH = LIB_DIR / ("_dkv_call" + sysconfig.get_config_var("EXT_SUFFIX"))
 OBJ_DIR = PKG_DIR / "_build"
 SOURCES = ("dkv_append.hip", "dkv_generic.hip", "dkv_splitk.hip", "dkv_cutoff.hip",
            "dkv_prefill.hip", "dkv_layer.hip", "dkv_model.hip", "dkv_joint.hip", "dkv_dense.hip",
@@ -62,11 +64,18 @@ def _compile(src: Path, obj: Path) -> None:
         raise RuntimeError(f"hipcc failed for {src.name}:\n{' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
 
 
-def _build_binding() -> None:
+def _build_binding(verbose: bool) -> None:
     """The CPython module over the library's entry points, found beside it at run time."""
+    headers = Path(sysconfig.get_paths()["include"])
+    CALL_PATH.unlink(missing_ok=True)  # never one built against an earlier library
+    if not (headers / "Python.h").exists():
+        if verbose:
+            print(f"[dynakv_amd] no Python.h under {headers}: call module left out, ctypes serves",
+                  file=sys.stderr)
+        return
     tmp = CALL_PATH.with_suffix(".so.tmp")
     cmd = [_hipcc(), "-x", "c++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wno-cast-function-type",
-           "-I", sysconfig.get_paths()["include"], str(CSRC / "dkv_call.cpp"), "-o", str(tmp),
+           "-I", str(headers), str(CSRC / "dkv_call.cpp"), "-o", str(tmp),
            f"-L{LIB_DIR}", "-l:libdynakv_amd.so", "-Wl,-rpath,$ORIGIN"]
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
@@ -89,7 +98,7 @@ def build(verbose: bool = True) -> Path:
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{' '.join(cmd)}\n{res.stdout}\n{res.stderr}")
     os.replace(tmp, LIB_PATH)
-    _build_binding()
+    _build_binding(verbose)
     if verbose:
         print(f"[dynakv_amd] built {LIB_PATH}", file=sys.stderr)
     return LIB_PATH
