@@ -140,7 +140,7 @@ def cutoff_kv(key_states: torch.Tensor, value_states: torch.Tensor, wt_k: torch.
         st = _lib.stream_of(key_states)
         nb = int(lib.dkv_cutoff_workspace_bytes(M, G, D))
         ws = _workspace(dev, st, nb)
-        lr = -1 if low_rank is None else int(low_rank)
+        lr = -1 if low_rank is None else max(-1, min(int(low_rank), D))  # any int: a C int holds it
         rc = lib.dkv_cutoff_kv(st, _lib.dtype_code(dt), xk.data_ptr(), xv.data_ptr(), ld,
                                wt_k.data_ptr(), wt_v.data_ptr(), b_k.data_ptr(), b_v.data_ptr(),
                                float(threshold), lr, out_k.data_ptr(), out_v.data_ptr(), hidden,

@@ -69,7 +69,7 @@ class DecodeLayerPlan:
         h = self.head
         a = _lib.DecodeLayerArgs()
         a.dtype, a.B, a.G, a.Hq, a.R, a.Dh = _lib.dtype_code(dt), B, G, Hq, R, Dh
-        a.low_rank = -1 if h.low_rank is None else int(h.low_rank)
+        a.low_rank = -1 if h.low_rank is None else max(-1, min(int(h.low_rank), R))
         a.switch_tokens = int(self.policy.switch_tokens)
         a.threshold, a.log_theta = float(h.threshold), math.log(self.theta)
         a.wt_k, a.wt_v = h.wt_k.data_ptr(), h.wt_v.data_ptr()
