@@ -9,16 +9,19 @@
 // is R(16T) R(n) composed in fp32 from the rows of the RoPE table (dkv_rope_table: cos and sin
 // of the fp32 angles n * inv_freq and 16T * inv_freq), not a sine and cosine per element.
 //
-// Workgroup = (RW * 16 * tiles tokens, cache row, K | V), four waves of 16 tokens at a time. The
-// row's basis ([rank][dim], ranks past R zero) is staged in LDS, read transposed
-// (ds_read_b64_tr_b16) once and kept in registers as the A operand (dims x ranks) of every tile;
-// each lane loads its token's 8 coefficients of a 32-rank chunk as the B operand, a tile ahead. The
-// dims are dealt to the A rows so that lane (token n, g) ends up with dims 16g .. 16g + 15 and
-// 64 + 16g .. of its token: the rotate-half pairs (d, d + 64) in one lane, stored 16 bytes at a
-// time. A lane's positions all have one offset in their 16-position tile, so R(n) stays in
-// registers too.
+// recon_kv_kernel: workgroup = (RW * 16 * tiles tokens, cache row, K | V), four waves of 16 tokens
+// at a time (recon_one_kernel, below: a single tile). The row's basis ([rank][dim], ranks past R
+// zero) is staged in LDS, read transposed (ds_read_b64_tr_b16) once and kept in registers as the A
+// operand (dims x ranks) of every tile; each lane loads its token's 8 coefficients of a 32-rank
+// chunk as the B operand, a tile ahead; a transposed basis (BT) comes straight into the operand
+// registers. The dims are dealt to the A rows so that lane (token n, g) ends up with dims 16g ..
+// 16g + 15 and 64 + 16g .. of its token: the rotate-half pairs (d, d + 64) in one lane, stored 16
+// bytes at a time. A lane's positions all have one offset in their 16-position tile, so R(n) stays
+// in registers too.
 // Bound: HBM. B = 4, 8 groups, S = 2048, rank 128 (67 MB): 21 us, 3.2 TB/s; with one 64-token tile
-// per workgroup, the basis staged for each and 8-byte stores 32 us.
+// per workgroup, the basis staged for each and 8-byte stores 32 us. Ranks of 96 and fewer skip the
+// chunks past them (16 rows x 2048 tokens, us with all four chunks / skipping: rank 64 12.0 / 10.2,
+// rank 8 11.7 / 9.0).
 #include "dkv_common.h"
 #include "dkv_mfma_ops.h"
 
@@ -28,11 +31,110 @@ constexpr int DH = 128;
 constexpr int RW = 4;  // waves per workgroup (16 tokens each)
 constexpr int RT_FIXED = 17;  // RoPE table rows before the tile rows R(16T)
 
+// One 64-token tile per workgroup (grids of up to 512 workgroups, where the latency of a single tile
+// is what a call takes): the A operands read from LDS as each product needs them, chunks past the
+// rank skipped, nothing kept for a further tile. Result lane (n, g): dims 16 blk + 4g + u. Graph-
+// replayed us, this kernel / recon_kv_kernel with one tile (rows x tokens, rank): 8 x 17, 128
+// 5.6 / 6.8; 64 x 128, 128 7.4 / 7.9; 32 x 333, 64 7.4 / 8.9; 16 x 100, 8 4.9 / 6.5; at 512
+// workgroups (8 x 2048, 128) 9.9 / 10.1. Above, several tiles per workgroup are ahead (16 x 2048,
+// 128 15.0 / 12.9).
 template <int DT>
+__global__ __launch_bounds__(RW * 64) void recon_one_kernel(
+    const uint16_t* __restrict__ ck, const uint16_t* __restrict__ cv, long long c_sr,
+    long long c_st, const uint16_t* __restrict__ kb, const uint16_t* __restrict__ vb,
+    long long b_sg, long long b_sr, uint16_t* __restrict__ ko, uint16_t* __restrict__ vo,
+    long long o_sr, long long o_st, int G, int S, int R, int pos0, const float* __restrict__ rope) {
+  __shared__ __attribute__((aligned(16))) uint16_t sB[DH * DH];  // [rank][dim]
+  const bool is_k = blockIdx.z == 0;
+  const int row = blockIdx.y, grp = row % G;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int n = lane & 15, g = lane >> 4;
+  const uint16_t* c = is_k ? ck : cv;
+  const uint16_t* bg = (is_k ? kb : vb) + (long long)grp * b_sg;
+  uint16_t* o = is_k ? ko : vo;
+
+  // this lane's token and its coefficient pieces (ranks 32 cc + 8g .. +8; R is a multiple of 8)
+  const int t = (blockIdx.x * RW + wave) * 16 + n;
+  const uint16_t* cr = c + (long long)row * c_sr + (long long)min(t, S - 1) * c_st;
+  dkv_u32x4 xc[4];
+#pragma unroll
+  for (int cc = 0; cc < 4; ++cc) {
+    const int r0 = 32 * cc + 8 * g;
+    xc[cc] = (t < S && r0 < R) ? *(const dkv_u32x4*)(cr + r0) : dkv_u32x4{0u, 0u, 0u, 0u};
+  }
+  // the basis, 16-byte pieces (rank r, dims d8 .. d8 + 7), ranks past R as zeros
+  for (int pc = tid; pc < DH * DH / 8; pc += RW * 64) {
+    const int r = pc >> 4, d8 = (pc & 15) * 8;
+    *(dkv_u32x4*)(sB + r * DH + d8) =
+        r < R ? *(const dkv_u32x4*)(bg + (long long)r * b_sr + d8) : dkv_u32x4{0u, 0u, 0u, 0u};
+  }
+  __syncthreads();
+
+  dkv_f32x4 acc[8];
+#pragma unroll
+  for (int blk = 0; blk < 8; ++blk) acc[blk] = dkv_f32x4{0.f, 0.f, 0.f, 0.f};
+  typedef __attribute__((address_space(3))) dkv_i16x4 lds_i16x4;
+#pragma unroll
+  for (int cc = 0; cc < 4; ++cc) {
+    if (32 * cc >= R) break;  // uniform: chunks wholly past the rank are zero
+#pragma unroll
+    for (int blk = 0; blk < 8; ++blk) {
+      // lane (n, g) receives ranks 32 cc + 8g .. +3 and +4 .. +7 of dim 16 blk + n
+      const uint16_t* src = sB + (32 * cc + 8 * g + (n >> 2)) * DH + 16 * blk + 4 * (n & 3);
+      const dkv_u32x2 b0 = __builtin_bit_cast(
+          dkv_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                         (lds_i16x4*)(__attribute__((address_space(3))) uint16_t*)src));
+      const dkv_u32x2 b1 = __builtin_bit_cast(
+          dkv_u32x2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                         (lds_i16x4*)(__attribute__((address_space(3))) uint16_t*)(src + 4 * DH)));
+      acc[blk] = dkv_mfma32<DT>(dkv_u32x4{b0.x, b0.y, b1.x, b1.y}, xc[cc], acc[blk]);
+    }
+  }
+  if (t >= S) return;
+  // lane (n, g): dims 16 blk + 4g + u of token t in acc[blk][u]
+  if (is_k) {
+    const int pos = pos0 + t;
+    // (cos, sin) of frequencies 16 blk + 4g .. +3: 32 contiguous bytes of a table row
+    const float* rn = rope + (pos & 15) * 128 + 8 * g;
+    const float* rt = rope + (RT_FIXED + (pos >> 4)) * 128 + 8 * g;
+#pragma unroll
+    for (int blk = 0; blk < 4; ++blk) {
+      const dkv_f32x4 n0 = *(const dkv_f32x4*)(rn + 32 * blk), n1 = *(const dkv_f32x4*)(rn + 32 * blk + 4);
+      const dkv_f32x4 t0 = *(const dkv_f32x4*)(rt + 32 * blk), t1 = *(const dkv_f32x4*)(rt + 32 * blk + 4);
+      const float nc[4] = {n0.x, n0.z, n1.x, n1.z}, ns[4] = {n0.y, n0.w, n1.y, n1.w};
+      const float tc[4] = {t0.x, t0.z, t1.x, t1.z}, ts[4] = {t0.y, t0.w, t1.y, t1.w};
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const float cs = tc[u] * nc[u] - ts[u] * ns[u], sn = ts[u] * nc[u] + tc[u] * ns[u];
+        // the projection rounded to the dtype first, then rotated: the reference's two steps
+        // (the up-projection's product in the dtype, then apply_rotary_pos_emb_)
+        const float a = dkv_round_to<DT>(acc[blk][u]), bb = dkv_round_to<DT>(acc[blk + 4][u]);
+        acc[blk][u] = a * cs - bb * sn;
+        acc[blk + 4][u] = bb * cs + a * sn;
+      }
+    }
+  }
+  uint16_t* orow = o + (long long)row * o_sr + (long long)t * o_st;
+#pragma unroll
+  for (int blk = 0; blk < 8; ++blk) {
+    uint32_t w[2];
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const float lo = acc[blk][2 * e], hi = acc[blk][2 * e + 1];
+      if constexpr (DT == DKV_BF16)
+        w[e] = dkv_f32_to_bf16_bits(lo) | (dkv_f32_to_bf16_bits(hi) << 16);
+      else
+        w[e] = dkv_f32_to_f16_bits(lo) | (dkv_f32_to_f16_bits(hi) << 16);
+    }
+    *(dkv_u32x2*)(orow + 16 * blk + 4 * g) = dkv_u32x2{w[0], w[1]};
+  }
+}
+
+template <int DT, bool BT>
 __global__ __launch_bounds__(RW * 64, 2) void recon_kv_kernel(
     const uint16_t* __restrict__ ck, const uint16_t* __restrict__ cv, long long c_sr,
     long long c_st, const uint16_t* __restrict__ kb, const uint16_t* __restrict__ vb,
-    long long b_sg, long long b_sr, int bt, uint16_t* __restrict__ ko, uint16_t* __restrict__ vo,
+    long long b_sg, long long b_sr, uint16_t* __restrict__ ko, uint16_t* __restrict__ vo,
     long long o_sr, long long o_st, int G, int S, int R, int pos0, const float* __restrict__ rope,
     int tiles) {
   __shared__ __attribute__((aligned(16))) uint16_t sB[DH * DH];  // [rank][dim]
@@ -69,7 +171,7 @@ __global__ __launch_bounds__(RW * 64, 2) void recon_kv_kernel(
   // receives ranks 32 cc + 8g .. +3 and +4 .. +7 of its row's dim
   typedef __attribute__((address_space(3))) dkv_i16x4 lds_i16x4;
   dkv_u32x4 a[4][8];
-  if (bt) {
+  if constexpr (BT) {
     // a transposed basis ([dim][rank]) holds them as they are taken
 #pragma unroll
     for (int cc = 0; cc < 4; ++cc)
@@ -80,15 +182,17 @@ __global__ __launch_bounds__(RW * 64, 2) void recon_kv_kernel(
                             : dkv_u32x4{0u, 0u, 0u, 0u};
       }
   } else {
-    // the basis, 16-byte pieces (rank r, dims d8 .. d8 + 7), ranks past R as zeros
-    for (int pc = tid; pc < DH * DH / 8; pc += RW * 64) {
+    // the basis up to its last 32-rank chunk, 16-byte pieces (rank r, dims d8 .. d8 + 7), ranks past
+    // R as zeros
+    for (int pc = tid; pc < (R + 31) / 32 * 32 * (DH / 8); pc += RW * 64) {
       const int r = pc >> 4, d8 = (pc & 15) * 8;
       *(dkv_u32x4*)(sB + r * DH + d8) =
           r < R ? *(const dkv_u32x4*)(bg + (long long)r * b_sr + d8) : dkv_u32x4{0u, 0u, 0u, 0u};
     }
     __syncthreads();
 #pragma unroll
-    for (int cc = 0; cc < 4; ++cc)
+    for (int cc = 0; cc < 4; ++cc) {
+      if (32 * cc >= R) break;  // uniform: chunks wholly past the rank take no part
 #pragma unroll
       for (int blk = 0; blk < 8; ++blk) {
         const uint16_t* src = sB + (32 * cc + 8 * g + (n >> 2)) * DH + 64 * (blk >> 2) +
@@ -101,6 +205,7 @@ __global__ __launch_bounds__(RW * 64, 2) void recon_kv_kernel(
                            (lds_i16x4*)(__attribute__((address_space(3))) uint16_t*)(src + 4 * DH)));
         a[cc][blk] = dkv_u32x4{b0.x, b0.y, b1.x, b1.y};
       }
+    }
   }
 
   for (int i = 0; i < tiles; ++i) {
@@ -110,9 +215,12 @@ __global__ __launch_bounds__(RW * 64, 2) void recon_kv_kernel(
 #pragma unroll
     for (int blk = 0; blk < 8; ++blk) acc[blk] = dkv_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-    for (int cc = 0; cc < 4; ++cc)
+    for (int cc = 0; cc < 4; ++cc) {
+      // (a transposed basis' operands are all loaded: the branches cost 1% at R = 128)
+      if (!BT && 32 * cc >= R) break;
 #pragma unroll
       for (int blk = 0; blk < 8; ++blk) acc[blk] = dkv_mfma32<DT>(a[cc][blk], xn[cc], acc[blk]);
+    }
     if (i + 1 < tiles) load_x(t + RW * 16);
     if (t >= S) continue;
     // lane (n, g): dims 64h + 16g + 4b + u of token t in acc[4h + b][u]
@@ -187,16 +295,28 @@ static int recon_kv(int bt, void* stream, int dtype, const void* ck, const void*
   const int tiles = (int)(per < t64 ? per : t64);
   const dim3 grid((unsigned)((t64 + tiles - 1) / tiles), (unsigned)rows, 2);
   hipStream_t st = (hipStream_t)stream;
-  if (dtype == DKV_BF16)
-    hipLaunchKernelGGL(recon_kv_kernel<DKV_BF16>, grid, dim3(RW * 64), 0, st,
-                       (const uint16_t*)ck, (const uint16_t*)cv, c_sr, c_st,
-                       (const uint16_t*)k_basis, (const uint16_t*)v_basis, b_sg, b_sr, bt,
-                       (uint16_t*)k_out, (uint16_t*)v_out, o_sr, o_st, G, S, R, pos0, rope, tiles);
-  else
-    hipLaunchKernelGGL(recon_kv_kernel<DKV_F16>, grid, dim3(RW * 64), 0, st,
-                       (const uint16_t*)ck, (const uint16_t*)cv, c_sr, c_st,
-                       (const uint16_t*)k_basis, (const uint16_t*)v_basis, b_sg, b_sr, bt,
-                       (uint16_t*)k_out, (uint16_t*)v_out, o_sr, o_st, G, S, R, pos0, rope, tiles);
+#define DKV_RECON(KERNEL, ...)                                                                  \
+  hipLaunchKernelGGL((KERNEL), grid, dim3(RW * 64), 0, st, (const uint16_t*)ck,                 \
+                     (const uint16_t*)cv, c_sr, c_st, (const uint16_t*)k_basis,                 \
+                     (const uint16_t*)v_basis, b_sg, b_sr, (uint16_t*)k_out, (uint16_t*)v_out,  \
+                     o_sr, o_st, G, S, R, pos0, rope __VA_OPT__(, ) __VA_ARGS__)
+  if (tiles == 1 && !bt) {
+    if (dtype == DKV_BF16)
+      DKV_RECON(recon_one_kernel<DKV_BF16>);
+    else
+      DKV_RECON(recon_one_kernel<DKV_F16>);
+  } else if (bt) {
+    if (dtype == DKV_BF16)
+      DKV_RECON((recon_kv_kernel<DKV_BF16, true>), tiles);
+    else
+      DKV_RECON((recon_kv_kernel<DKV_F16, true>), tiles);
+  } else {
+    if (dtype == DKV_BF16)
+      DKV_RECON((recon_kv_kernel<DKV_BF16, false>), tiles);
+    else
+      DKV_RECON((recon_kv_kernel<DKV_F16, false>), tiles);
+  }
+#undef DKV_RECON
   DKV_HIP_CHECK_LAUNCH();
   return DKV_OK;
 }

@@ -45,3 +45,25 @@ def test_unaligned_outputs(dev):
         rows = got[4:].view(G, S, ld)
         assert torch.equal(rows[..., :128], want.view(G, S, 128))
         assert not rows[..., 128:].any()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("R", [8, 40, 64, 128])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_one_tile_equals_several(dev, R, dtype, transposed):
+    """A call of several tiles per workgroup, and the same tokens in calls of up to 512 workgroups
+    (one tile each, another kernel for rank-major bases): the same bits."""
+    B, G, S = 16, 8, 257  # 16 x 8 rows x 5 tiles x K, V: 1280 workgroups of one tile
+    print(f"[gpu] recon one tile against several R={R} {dtype} transposed={transposed}", flush=True)
+    ck, cv, kb, vb = (torch.from_numpy(a).to(device=dev, dtype=dtype)
+                      for a in base._inputs(B, G, S, R, dtype, seed=40 + R))
+    if transposed:
+        kb, vb = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (kb, vb))
+    k, v = base.recon_kv(ck, cv, kb, vb, batch=B, theta=base.THETA)
+    for b in range(0, B, 3):
+        rows = slice(b * G, (b + 1) * G)
+        for t0, t1 in ((0, 64), (64, 200), (192, 257)):
+            kk, vv = base.recon_kv(ck[rows, t0:t1], cv[rows, t0:t1], kb, vb, batch=1,
+                                   theta=base.THETA, pos0=t0)
+            assert torch.equal(kk[0], k[b, :, t0:t1]) and torch.equal(vv[0], v[b, :, t0:t1])
