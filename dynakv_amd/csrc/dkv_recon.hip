@@ -13,11 +13,13 @@
 // at a time (recon_one_kernel, below: a single tile). The row's basis ([rank][dim], ranks past R
 // zero) is staged in LDS, read transposed (ds_read_b64_tr_b16) once and kept in registers as the A
 // operand (dims x ranks) of every tile; each lane loads its token's 8 coefficients of a 32-rank
-// chunk as the B operand, a tile ahead; a transposed basis (BT) comes straight into the operand
-// registers. The dims are dealt to the A rows so that lane (token n, g) ends up with dims 16g ..
-// 16g + 15 and 64 + 16g .. of its token: the rotate-half pairs (d, d + 64) in one lane, stored 16
-// bytes at a time. A lane's positions all have one offset in their 16-position tile, so R(n) stays
-// in registers too.
+// chunk as the B operand, a tile ahead. The dims are dealt to the A rows so that lane (token n, g)
+// ends up with dims 16g .. 16g + 15 and 64 + 16g .. of its token: the rotate-half pairs (d, d + 64)
+// in one lane, stored 16 bytes at a time. A lane's positions all have one offset in their
+// 16-position tile, so R(n) stays in registers too. A transposed basis (BT) is staged and read as
+// it lies (us with every wave loading its operands from the basis / staged, rank 128: 64 rows x 128
+// tokens 8.1 / 6.6, 16 x 2048 15.7 / 11.5, 4096 x 64 158 / 88, where copying the bases first took
+// 99).
 // Bound: HBM. B = 4, 8 groups, S = 2048, rank 128 (67 MB): 21 us, 3.2 TB/s; with one 64-token tile
 // per workgroup, the basis staged for each and 8-byte stores 32 us. Ranks of 96 and fewer skip the
 // chunks past them (16 rows x 2048 tokens, us with all four chunks / skipping: rank 64 12.0 / 10.2,
@@ -172,15 +174,16 @@ __global__ __launch_bounds__(RW * 64, 2) void recon_kv_kernel(
   typedef __attribute__((address_space(3))) dkv_i16x4 lds_i16x4;
   dkv_u32x4 a[4][8];
   if constexpr (BT) {
-    // a transposed basis ([dim][rank]) holds them as they are taken
-#pragma unroll
-    for (int cc = 0; cc < 4; ++cc)
-#pragma unroll
-      for (int blk = 0; blk < 8; ++blk) {
-        const int r0 = 32 * cc + 8 * g, d = 64 * (blk >> 2) + 16 * (n >> 2) + 4 * (blk & 3) + (n & 3);
-        a[cc][blk] = r0 < R ? *(const dkv_u32x4*)(bg + (long long)d * b_sr + r0)
-                            : dkv_u32x4{0u, 0u, 0u, 0u};
-      }
+    // [dim][rank] as it comes, 16-byte pieces (dim d, ranks 8c .. 8c + 7; those past R as zeros; of
+    // 32, 64 or 128 ranks) at position c ^ (d % 4 + 4 (d / 16 % 4)), so that the 16 rows of an
+    // operand read lie apart
+    const int sh = R > 64 ? 4 : (R > 32 ? 3 : 2);
+    for (int pc = tid; pc < DH << sh; pc += RW * 64) {
+      const int d = pc >> sh, c8 = pc & ((1 << sh) - 1);
+      *(dkv_u32x4*)(sB + d * DH + 8 * (c8 ^ ((d & 3) | ((d >> 2) & 12)))) =
+          8 * c8 < R ? *(const dkv_u32x4*)(bg + (long long)d * b_sr + 8 * c8)
+                     : dkv_u32x4{0u, 0u, 0u, 0u};
+    }
   } else {
     // the basis up to its last 32-rank chunk, 16-byte pieces (rank r, dims d8 .. d8 + 7), ranks past
     // R as zeros
@@ -189,12 +192,17 @@ __global__ __launch_bounds__(RW * 64, 2) void recon_kv_kernel(
       *(dkv_u32x4*)(sB + r * DH + d8) =
           r < R ? *(const dkv_u32x4*)(bg + (long long)r * b_sr + d8) : dkv_u32x4{0u, 0u, 0u, 0u};
     }
-    __syncthreads();
+  }
+  __syncthreads();
 #pragma unroll
-    for (int cc = 0; cc < 4; ++cc) {
-      if (32 * cc >= R) break;  // uniform: chunks wholly past the rank take no part
+  for (int cc = 0; cc < 4; ++cc) {
+    if (32 * cc >= R) break;  // uniform: chunks wholly past the rank take no part
 #pragma unroll
-      for (int blk = 0; blk < 8; ++blk) {
+    for (int blk = 0; blk < 8; ++blk) {
+      if constexpr (BT) {
+        const int d = 64 * (blk >> 2) + 16 * (n >> 2) + 4 * (blk & 3) + (n & 3);
+        a[cc][blk] = *(const dkv_u32x4*)(sB + d * DH + 8 * ((4 * cc + g) ^ n));
+      } else {
         const uint16_t* src = sB + (32 * cc + 8 * g + (n >> 2)) * DH + 64 * (blk >> 2) +
                               16 * (n & 3) + 4 * (blk & 3);
         const dkv_u32x2 b0 = __builtin_bit_cast(
@@ -216,8 +224,7 @@ __global__ __launch_bounds__(RW * 64, 2) void recon_kv_kernel(
     for (int blk = 0; blk < 8; ++blk) acc[blk] = dkv_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int cc = 0; cc < 4; ++cc) {
-      // (a transposed basis' operands are all loaded: the branches cost 1% at R = 128)
-      if (!BT && 32 * cc >= R) break;
+      if (32 * cc >= R) break;
 #pragma unroll
       for (int blk = 0; blk < 8; ++blk) acc[blk] = dkv_mfma32<DT>(a[cc][blk], xn[cc], acc[blk]);
     }
