@@ -220,16 +220,18 @@ def joint_attention(q3, k_flat, k_up, v_flat, v_up, l_k, o_k, l_v, o_v, *, theta
 
 def joint_flops(lens_k: torch.Tensor, R: int, n_basis: int, B: int) -> float:
     """MFMA flops of the scores kernel as launched: 2 * 128 dims * 32 ranks per processed chunk,
-    per token slot and basis head. A workgroup takes 512 tokens (256 when the basis heads pair
-    up), sorts them by chunk count and runs each block of 16 sorted tokens up to its own
-    longest token's chunk count."""
+    per token slot and basis head. Calls of up to 512 workgroups of 32 tokens run all of a
+    workgroup's tokens to the longest one's chunk count; the others sort the tokens of a window (up
+    to 2048) by chunk count, pads first, and run each block of 16 to its own longest token's."""
     S = lens_k.shape[1]
-    tok = 256 if n_basis % 2 == 0 else 512
+    if B * ((S + 31) // 32) * n_basis <= 512:
+        tok, run = 32, 32
+    else:
+        tok, run = min(2048, (S + 511) // 512 * 512), 16
     groups = (S + tok - 1) // tok
-    pad = groups * tok - S
-    L = torch.nn.functional.pad(lens_k.clamp(0, R), (0, pad)).view(B, groups, tok)
-    chunks = ((L + 31) // 32).sort(dim=2).values.view(B, groups, tok // 16, 16)[..., -1]
-    return float(chunks.sum().item()) * 16 * 2 * 128 * 32 * n_basis
+    L = torch.nn.functional.pad(lens_k.clamp(0, R), (0, groups * tok - S)).view(B, groups, tok)
+    chunks = ((L + 31) // 32).sort(dim=2).values.view(B, groups, tok // run, run)[..., -1]
+    return float(chunks.sum().item()) * run * 2 * 128 * 32 * n_basis
 
 
 __all__ = ["joint_attention", "joint_scores", "joint_av", "scores_eligible", "av_eligible",

@@ -12,8 +12,9 @@ from dynakv_amd.kernels import joint as J
 from helpers import assert_close, cast_np
 from test_gpu_joint import THETA, ULP, _case, _dev, _generic_av, _generic_scores
 
-# (B, S, R, n_basis, Hq): 128 and 130 workgroups of two heads, 129 of one head, tokens one past a
-# 128-token range, one chunk, five chunks (a remainder of the four-chunk loop)
+# (B, S, R, n_basis, Hq): with two heads per workgroup 48, 128 and 130 workgroups, with one head
+# 128, 129 (half the rows: 66) and 258, tokens one past a 128-token range, one chunk, five chunks (a
+# remainder of the four-chunk loop)
 CASES = [
     (8, 1025, 64, 2, 8),
     (64, 129, 64, 2, 8),
@@ -21,7 +22,28 @@ CASES = [
     (43, 513, 160, 3, 12),
     (9, 2049, 32, 2, 2),
     (17, 1025, 224, 4, 16),
+    (43, 290, 160, 3, 12),
+    (128, 129, 96, 1, 4),
 ]
+
+
+def _shape(B, S, nb):
+    """The scores' launch shape: "32" (tokens of one head), "128" (of one head), or the large one."""
+    if _wg32(B, S, nb) <= 512:
+        return "32"
+    win = 2048 if S >= 2048 else -(-S // 512) * 512
+    tok, heads = (512, 1) if nb % 2 else (256, 2)
+    return "128" if -(-S // win) * (win // tok) * (nb // heads) * B <= 128 else f"{tok}x{heads}"
+
+
+def test_cases_cross_the_boundaries():
+    """The listed cases take every shape, and their halves other ones than the whole."""
+    whole = [_shape(*c[:2], c[3]) for c in CASES]
+    half = [_shape((c[0] + 1) // 2, c[1], c[3]) for c in CASES]
+    assert set(whole) == {"128", "256x2", "512x1"}
+    crossed = {(w, h) for w, h, c in zip(whole, half, CASES)
+               if w != h and _wg32(c[0] // 2, c[1], c[3]) > 512}
+    assert crossed >= {("256x2", "128"), ("512x1", "128")}
 
 
 @pytest.mark.gpu
