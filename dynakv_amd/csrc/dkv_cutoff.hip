@@ -948,14 +948,15 @@ extern "C" int dkv_cutoff_kv(void* stream, int dtype, const void* xk, const void
   const int E = D / 64;
   if (E != 1 && E != 2 && E != 4 && E != 8 && E != 16) return DKV_E_UNSUPPORTED;
   hipStream_t st = (hipStream_t)stream;
-  // D <= 128: the 8-wave kernel (a 16-row tile per workgroup) while the tiles about fill the
-  // 256 CUs once, the wave-per-tile kernel past that. Graph-replayed us per call, 8-wave / wave
-  // per tile: G = 8, D = 128: 33 rows 5.2 / 6.7, 301 rows 7.0 / 7.2, 1024 rows 13.4 / 8.5, 8192
-  // rows 72.3 / 31.7 (two kernels, a wave per row, before: 5.9, 8.7, 19.6, 108.3); G = 4: 301
-  // rows 5.3 / 7.1, 1024 rows 8.4 / 7.7 (the wave-per-tile figures from before its sums took the
-  // row kernel's order, about 2 us more at 8192 rows).
+  // D <= 128: the 8-wave kernel (a 16-row tile per workgroup) up to one workgroup per CU, the
+  // wave-per-tile kernel past that. Graph-replayed us per call, 8-wave / wave per tile (bf16, fp16
+  // within 2%): G = 8, D = 128: 33 rows (48 workgroups) 5.3 / 6.7, 250 (256) 5.6 / 7.1, 301 (304)
+  // 7.5 / 7.3, 1024 rows 12.4 / 8.2, 8192 rows 66 / 31.6 (two kernels, a wave per row, before: 5.9
+  // at 33 rows, 19.6 at 1024, 105 at 8192); G = 4: 500 rows (256) 5.6 / 7.1, 640 (320) 7.5 / 7.3;
+  // G = 2: 1024 (256) 5.7 / 7.1, 1300 (328) 7.7 / 7.2; G = 32: 33 (192) 5.4 / 6.8, 100 (448) 7.8 /
+  // 7.4; G = 8, D = 64: 250 4.4 / 4.5, 301 5.7 / 4.7.
   const long long row_tiles = (M + CT_ROWS - 1) / CT_ROWS;
-  if (D <= 128 && (row_tiles == 1 || 2 * G * row_tiles <= 320)) {
+  if (D <= 128 && (row_tiles == 1 || 2 * G * row_tiles <= 256)) {
     const dim3 sgrid((unsigned)(2 * G), (unsigned)row_tiles);
     if (dtype == DKV_BF16) {
       if (E == 1)

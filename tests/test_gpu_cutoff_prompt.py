@@ -22,6 +22,9 @@ CASES = [
     (2, 256, 385, torch.bfloat16, None, 8),
     (1, 512, 1345, torch.float16, None, 0),
     (2, 512, 161, torch.bfloat16, None, 0),
+    (8, 128, 256, torch.float16, None, 0),     # 256 workgroups of the 8-wave kernel, then one
+    (8, 128, 257, torch.float16, None, 0),     # row more
+    (2, 64, 1025, torch.bfloat16, None, 8),
 ]
 
 
