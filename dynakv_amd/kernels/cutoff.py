@@ -15,7 +15,7 @@ CUDA graph before appending to the cache (:321-334):
 ``D = hidden / G`` dims with per-group weights ``(G, D, D)`` / ``(G, D)`` (the per-head layout,
 row = b*G + g in the cache); ``len`` then has shape ``(B, S, G)``.
 
-Both matrices run in one ``dkv_cutoff_kv`` call (two kernels on the current stream). The
+Both matrices run in one ``dkv_cutoff_kv`` call (one or two kernels on the current stream). The
 weights are copied once, transposed (input dimension contiguous), when the head is built;
 ``refresh()`` re-reads them after an in-place update.
 """
