@@ -296,8 +296,9 @@ static int recon_kv(int bt, void* stream, int dtype, const void* ck, const void*
     return DKV_E_UNSUPPORTED;
   if (S > 65535 * 64 || rows > 65535) return DKV_E_UNSUPPORTED;
   // 64-token tiles per workgroup: the grid within the 512 workgroups that run at once (two per
-  // CU). us at 1 / 2 / 4 tiles: 512 tiles in all (B = 1, S = 2048, G = 8) 10.1 / 9.9 / 12.3; 1024
-  // (B = 2) 20.1 / 14.1 / 15.9; 2048 (B = 4) 36.6 / 27.6 / 21.0.
+  // CU). Graph-replayed us, rank 128, one tile each in recon_one_kernel / the chosen count: 512 tiles
+  // in all (8 rows x 2048 tokens) 9.9; 768 12.8 / 11.9 (two); 1024 14.9 / 12.7 (two); 2048 28.6 / 20.1
+  // (four; 1 / 2 / 4 tiles of recon_kv_kernel when it was written: 36.6 / 27.6 / 21.0).
   const long long t64 = (S + 63) / 64, per = (t64 * rows * 2 + 511) / 512;
   const int tiles = (int)(per < t64 ? per : t64);
   const dim3 grid((unsigned)((t64 + tiles - 1) / tiles), (unsigned)rows, 2);
